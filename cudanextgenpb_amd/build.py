@@ -29,6 +29,7 @@ HIP_SOURCES = [
     "ngpb_krylov.hip",
     "ngpb_lis.hip",
     "ngpb_mixed.hip",
+    "ngpb_mg.hip",
     "ngpb_energy.hip",
     "ngpb_batch.hip",
     "ngpb_rays.hip",

@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "ngpb.h"
+#include "ngpb_mg.h"
 
 namespace ngpb {
 
@@ -310,6 +311,11 @@ struct ngpb_ctx {
   ngpb::DBuf<int32_t> row_perm;
   ngpb::DBuf<int64_t> sell_pk_hdr_list;
   ngpb::DBuf<double> dscale;         // 1/sqrt(diag)
+  // multigrid preconditioner of the mixed solve, built with the compact operator
+  int mg_state = 0;  // 0 not built, 1 in use, -1 does not apply to this operator
+  ngpb::MgHierarchy mg;
+  ngpb::DBuf<float> mg_pool, mg_dense, mg_sd, mg_r, mg_z;  // mg_r, mg_z: with SpMV guard entries
+  ngpb::DBuf<uint32_t> mg_pos;
   int spmv_sched = 6;                // SpMV work schedule (0 .. 6)
   int sell_resident = 0;             // resident blocks of the compact SpMV (0: not yet queried)
   int csr_resident = 0;              // resident blocks of the FP64 CSR SpMV (0: not yet queried)
@@ -445,6 +451,19 @@ void spmv_compact(ngpb_ctx* c, const double* x, double* y);
 void solve_mixed(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st);
 double spmv_compact_bytes(const ngpb_ctx* c);
 double time_spmv_compact(ngpb_ctx* c, int reps);
+
+// multigrid preconditioner (ngpb_mg.hip): one CG iteration runs an SpMV on r,
+// mg_precondition, an SpMV on z, mg_direction, an SpMV on p and mg_update. par is the
+// parity of the iteration; every kernel returns at once after the stop flag.
+bool mg_setup(ngpb_ctx* c);
+// z0 from r and ar = Ahat r; stops first if (r, r) from the partials met the target
+void mg_precondition(ngpb_ctx* c, const float* r, const float* ar, float* z, const double* rr_part, int npr, int par,
+                     bool first);
+// z = z0 + omega (r - az), az = Ahat z0; p = z + beta p
+void mg_direction(ngpb_ctx* c, const float* r, const float* az, float* z, float* p, double* part, int par);
+// x += alpha p, r -= alpha ap, ap = Ahat p; per block (r, r)
+void mg_update(ngpb_ctx* c, float* x, float* r, const float* p, const float* ap, const double* pq_part, int npq,
+               double* part, int par);
 
 // energy
 void run_energy(ngpb_ctx* c, ngpb_energy_out* out);

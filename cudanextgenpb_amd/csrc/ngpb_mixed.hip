@@ -882,6 +882,56 @@ __global__ void __launch_bounds__(kFin) k_mx_fin_resid(KrylovScalars* ks, const 
   }
 }
 
+// Start of a multigrid solve: rows without off-diagonals (the Dirichlet nodes, sd = 0)
+// take their solution b / d at once, so the iteration runs on the coupled rows only;
+// x = 0 and r = b elsewhere. Per block (b, b), and over the coupled rows (b, b) and
+// (rhat, rhat).
+__global__ void __launch_bounds__(kBS) k_mx_start(int64_t n, const double* __restrict__ b,
+                                                  const double* __restrict__ dscale, const float* __restrict__ sd,
+                                                  float* __restrict__ rs, double* __restrict__ x, float* __restrict__ xs,
+                                                  float* __restrict__ ps, double* __restrict__ partials,
+                                                  const int32_t* __restrict__ perm) {
+  __shared__ double s_red[kBS / 64];
+  double bb = 0.0, rr = 0.0, ss = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * kBS + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBS) {
+    const int64_t o = perm ? (int64_t)perm[i] : i;
+    const double bi = b[o], s = dscale[i];
+    const bool alone = sd[i] == 0.f;
+    const float si = alone ? 0.f : (float)(s * bi);
+    x[o] = alone ? s * s * bi : 0.0;
+    xs[i] = 0.f;
+    ps[i] = 0.f;
+    rs[i] = si;
+    bb += bi * bi;
+    if (!alone) rr += bi * bi;
+    ss += (double)si * (double)si;
+  }
+  bb = dev::block_sum<kBS>(bb, s_red);
+  rr = dev::block_sum<kBS>(rr, s_red);
+  ss = dev::block_sum<kBS>(ss, s_red);
+  if (threadIdx.x == 0) {
+    partials[3 * blockIdx.x] = bb;
+    partials[3 * blockIdx.x + 1] = rr;
+    partials[3 * blockIdx.x + 2] = ss;
+  }
+}
+
+__global__ void __launch_bounds__(kFin) k_mx_fin_start(KrylovScalars* ks, const double* __restrict__ partials, int np) {
+  __shared__ double s_red[kFin / 64];
+  const double BB = dev::sum_partials<kFin>(partials, np, 3, s_red);
+  const double RR = dev::sum_partials<kFin>(partials + 1, np, 3, s_red);
+  const double SS = dev::sum_partials<kFin>(partials + 2, np, 3, s_red);
+  if (threadIdx.x == 0) {
+    ks->bb = BB;
+    ks->beta = 0.0;
+    ks->iter = 0;
+    ks->aux[0] = RR;
+    ks->aux[1] = SS;
+    ks->rho = SS;
+    ks->rr = SS;
+  }
+}
+
 __global__ void k_to_scaled(int64_t n, const double* __restrict__ x, const double* __restrict__ dscale,
                             float* __restrict__ xs, const int32_t* __restrict__ perm) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1306,17 +1356,20 @@ void build_compact_from(ngpb_ctx* c, const int32_t* rowptr, const int32_t* colid
   }
   NGPB_HIP(hipStreamSynchronize(c->stream));
   c->have_compact = true;
+  c->mg_state = 0;
 }
 
 // The FP32 SpMV input vector of the context (the scaled direction p of the mixed
 // solve): x_0 .. x_n-1 with kGuard zero entries on either side, which the lean SpMV
 // gathers from in place of clamped indices. Every kernel writes only x_0 .. x_n-1.
-float* spmv_input(ngpb_ctx* c) {
-  c->ps.reserve((size_t)(c->n + 2 * kGuard));
-  hipLaunchKernelGGL(k_zero_guard, dim3(1), dim3(2 * kGuard), 0, c->stream, c->ps.p, c->n);
+float* guarded_vector(ngpb_ctx* c, DBuf<float>& v) {
+  v.reserve((size_t)(c->n + 2 * kGuard));
+  hipLaunchKernelGGL(k_zero_guard, dim3(1), dim3(2 * kGuard), 0, c->stream, v.p, c->n);
   NGPB_HIP(hipGetLastError());
-  return c->ps.p + kGuard;
+  return v.p + kGuard;
 }
+
+float* spmv_input(ngpb_ctx* c) { return guarded_vector(c, c->ps); }
 
 double spmv_compact_bytes(const ngpb_ctx* c) {
   // delta-slice entries (4: value), offset-slice entries (4 value + 2 offset), slot
@@ -1367,90 +1420,144 @@ double time_spmv_compact(ngpb_ctx* c, int reps) {
   return (double)ms / std::max(reps, 1);
 }
 
+// Solves with the multigrid preconditioner where it applies (mg_setup): an inner cycle
+// is then CG preconditioned by one V-cycle, 20-30 iterations in all against 300-900 with
+// Jacobi scaling alone. Should the cycle not converge (kMgCycleIters iterations, or a
+// non-finite residual), the solve goes on with the Jacobi-scaled CG.
 void solve_mixed(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
+  constexpr int kMgCycleIters = 100;
   const int64_t n = c->n;
   check_operator(c);
   if (!c->have_compact) build_compact(c);
+  bool mg = mg_setup(c);
   c->x.resize((size_t)n);
   c->q.reserve((size_t)n);
   c->xs.reserve((size_t)n);
-  c->rs.reserve((size_t)n);
   float* const pv = spmv_input(c);
+  float* rv;  // residual of the inner iteration
+  float* zv = nullptr;
+  if (mg) {
+    rv = guarded_vector(c, c->mg_r);
+    zv = guarded_vector(c, c->mg_z);
+  } else {
+    c->rs.reserve((size_t)n);
+    rv = c->rs.p;
+  }
   const int32_t* const perm = c->sell_banded ? c->row_perm.p : nullptr;  // FP32 row -> node
   c->qs.reserve((size_t)n);
   const unsigned gv = vec_grid(n);
   const unsigned gs = (unsigned)sell_partials(c);
-  ensure_reduce(c, std::max<int64_t>(gs, 2048) + 2 * (int64_t)gv);
+  const int64_t region = std::max<int64_t>(gs, 2048);
+  ensure_reduce(c, 2 * region + 3 * (int64_t)gv);
   double* part = c->red.partials.p;
-  double* ppq = part;                                  // SpMV (p, q) partials
-  double* pup = part + std::max<int64_t>(gs, 2048);    // update (rhat, rhat) partials
-  int64_t launch = 0;                                  // iteration launches (parity)
+  double* ppq = part;            // SpMV (p, q) partials
+  double* pun = part + region;   // SpMV partials that are not used
+  double* pup = pun + region;    // update (rhat, rhat) partials
+  double* prz = pup + gv;        // (rhat, z) partials
+  int64_t launch = 0;            // iteration launches (parity)
   KrylovScalars* ks = c->ks.p;
   KrylovScalars* h = c->ks_host;
   const double drop = (o.drop > 0.0 && o.drop < 1.0) ? o.drop : 1e-3;
-  const int chunk = std::max(1, o.check_every);
 
   hipEvent_t e0, e1;
   NGPB_HIP(hipEventCreate(&e0));
   NGPB_HIP(hipEventCreate(&e1));
   NGPB_HIP(hipEventRecord(e0, c->stream));
-  hipLaunchKernelGGL(k_mx_resid, dim3(gv), dim3(kBS), 0, c->stream, n, c->rhs.p, (const double*)nullptr, c->dscale.p,
-                     c->rs.p, c->x.p, c->xs.p, pv, 1, part, perm);
-  hipLaunchKernelGGL(k_mx_fin_resid, dim3(1), dim3(kFin), 0, c->stream, ks, part, (int)gv, 1);
-  NGPB_HIP(hipGetLastError());
-  NGPB_HIP(hipMemcpyAsync(h, ks, sizeof(KrylovScalars), hipMemcpyDeviceToHost, c->stream));
-  NGPB_HIP(hipStreamSynchronize(c->stream));
+  auto start_jacobi = [&] {
+    hipLaunchKernelGGL(k_mx_resid, dim3(gv), dim3(kBS), 0, c->stream, n, c->rhs.p, (const double*)nullptr, c->dscale.p,
+                       rv, c->x.p, c->xs.p, pv, 1, part, perm);
+    hipLaunchKernelGGL(k_mx_fin_resid, dim3(1), dim3(kFin), 0, c->stream, ks, part, (int)gv, 1);
+  };
+  if (mg) {
+    hipLaunchKernelGGL(k_mx_start, dim3(gv), dim3(kBS), 0, c->stream, n, c->rhs.p, c->dscale.p, c->mg_sd.p, rv, c->x.p,
+                       c->xs.p, pv, part, perm);
+    hipLaunchKernelGGL(k_mx_fin_start, dim3(1), dim3(kFin), 0, c->stream, ks, part, (int)gv);
+  } else {
+    start_jacobi();
+  }
+  auto read_scalars = [&] {
+    NGPB_HIP(hipGetLastError());
+    NGPB_HIP(hipMemcpyAsync(h, ks, sizeof(KrylovScalars), hipMemcpyDeviceToHost, c->stream));
+    NGPB_HIP(hipStreamSynchronize(c->stream));
+  };
+  read_scalars();
   const double bb = h->bb;
   const double target = o.tol * o.tol * bb;
   int status = 0, iters = 0, repl = 0;
-  double true_rr = bb;
-  if (bb > 0.0) {
+  double true_rr = h->aux[0];
+  if (bb > 0.0 && !(true_rr <= target)) {
     status = NGPB_E_NOCONV;
     double prev_true = bb;
     int stagnant = 0;
+    int ahead = 6;         // multigrid iterations launched before the first poll of a cycle
+    double mg_rho = 0.0;   // (r, z) of the last multigrid iteration
     while (iters < o.maxiter) {
       // cycle: stop at drop^2 of the current scaled residual or at the scaled image
       // of the FP64 target (ratio of the two norms taken at the last replacement)
       const double ss = h->aux[1], tt = h->aux[0];
       const double ratio = tt > 0.0 ? ss / tt : 1.0;
       h->stop_rr = std::max(drop * drop * ss, 0.25 * target * ratio);
-      h->maxiter = o.maxiter;
+      h->maxiter = mg ? std::min(o.maxiter, iters + kMgCycleIters) : o.maxiter;
       h->iter = iters;
       h->done = 0;
-      h->rho2[launch & 1] = h->rho;
+      h->rho2[launch & 1] = mg ? mg_rho : h->rho;
       h->iter2[launch & 1] = iters;
+      if (mg) {  // xhat is complete when the flag is raised: k_mx_accum adds nothing to it
+        h->alpha2[0] = h->alpha2[1] = 0.0;
+        h->stop_par = 0;
+      }
       NGPB_HIP(hipMemcpyAsync(ks, h, sizeof(KrylovScalars), hipMemcpyHostToDevice, c->stream));
       const int64_t cycle_start = launch;
-      hipLaunchKernelGGL(k_mx_dir, dim3(gv), dim3(kBS), 0, c->stream, n, c->rs.p, pv, ks);
+      if (!mg) hipLaunchKernelGGL(k_mx_dir, dim3(gv), dim3(kBS), 0, c->stream, n, rv, pv, ks);
+      int chunk = std::max(1, mg ? std::min(ahead, o.check_every) : o.check_every);
       while (true) {
         for (int k = 0; k < chunk; ++k, ++launch) {
           const int par = (int)(launch & 1);
+          if (mg) {
+            launch_sell(c, true, rv, c->qs.p, pun);
+            mg_precondition(c, rv, c->qs.p, zv, pup, (int)gv, par, launch == cycle_start);
+            launch_sell(c, true, zv, c->qs.p, pun);
+            mg_direction(c, rv, c->qs.p, zv, pv, prz, par);
+          }
           prof_begin(c, 1, launch);
           launch_sell(c, true, pv, c->qs.p, ppq);
           prof_end(c, 1);
-          hipLaunchKernelGGL(k_mx_update, dim3(gv), dim3(kBS), 0, c->stream, n, c->rs.p, c->qs.p, ks, ppq, (int)gs, pup,
-                             par);
-          hipLaunchKernelGGL(k_mx_dir_x, dim3(gv), dim3(kBS), 0, c->stream, n, c->rs.p, pv, c->xs.p, ks, pup,
-                             (int)gv, par);
+          if (mg) {
+            mg_update(c, c->xs.p, rv, pv, c->qs.p, ppq, (int)gs, pup, par);
+            continue;
+          }
+          hipLaunchKernelGGL(k_mx_update, dim3(gv), dim3(kBS), 0, c->stream, n, rv, c->qs.p, ks, ppq, (int)gs, pup, par);
+          hipLaunchKernelGGL(k_mx_dir_x, dim3(gv), dim3(kBS), 0, c->stream, n, rv, pv, c->xs.p, ks, pup, (int)gv, par);
         }
-        NGPB_HIP(hipGetLastError());
-        NGPB_HIP(hipMemcpyAsync(h, ks, sizeof(KrylovScalars), hipMemcpyDeviceToHost, c->stream));
-        NGPB_HIP(hipStreamSynchronize(c->stream));
+        read_scalars();
         prof_collect(c, 1, cycle_start + (h->iter - iters));
         if (h->done) break;
+        if (mg) chunk = std::max(1, std::min(2, o.check_every));
       }
+      const int cycle_iters = h->iter - iters;
       iters = h->iter;
+      bool mg_failed = false;
+      if (mg) {
+        mg_rho = h->rho2[(cycle_start + cycle_iters) & 1];
+        mg_failed = !std::isfinite(h->rr) || (h->rr > h->stop_rr && iters < o.maxiter);
+        ahead = std::max(2, cycle_iters + 1);
+      }
+      if (mg && !std::isfinite(h->rr)) {  // start over without the preconditioner
+        mg = false;
+        start_jacobi();
+        read_scalars();
+        true_rr = h->aux[0];
+        continue;
+      }
       // FP64 residual replacement
       hipLaunchKernelGGL(k_mx_accum, dim3(gv), dim3(kBS), 0, c->stream, n, c->dscale.p, c->x.p, c->xs.p, pv, ks, perm);
       prof_begin(c, 0, -1);
       spmv_fp64(c, c->x.p, c->q.p);
       prof_end(c, 0);
-      hipLaunchKernelGGL(k_mx_resid, dim3(gv), dim3(kBS), 0, c->stream, n, c->rhs.p, c->q.p, c->dscale.p, c->rs.p, c->x.p,
+      hipLaunchKernelGGL(k_mx_resid, dim3(gv), dim3(kBS), 0, c->stream, n, c->rhs.p, c->q.p, c->dscale.p, rv, c->x.p,
                          c->xs.p, pv, 0, part, perm);
       hipLaunchKernelGGL(k_mx_fin_resid, dim3(1), dim3(kFin), 0, c->stream, ks, part, (int)gv, 0);
-      NGPB_HIP(hipGetLastError());
-      NGPB_HIP(hipMemcpyAsync(h, ks, sizeof(KrylovScalars), hipMemcpyDeviceToHost, c->stream));
-      NGPB_HIP(hipStreamSynchronize(c->stream));
+      read_scalars();
       prof_collect(c, 0, -1);
       ++repl;
       true_rr = h->aux[0];
@@ -1459,12 +1566,20 @@ void solve_mixed(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
         break;
       }
       // the FP32 inner solve no longer reduces the FP64 residual
-      if (true_rr > 0.81 * prev_true) {
-        if (++stagnant >= 3) break;
+      bool stalled = false;
+      if (!(true_rr <= 0.81 * prev_true)) {
+        stalled = ++stagnant >= 3;
       } else {
         stagnant = 0;
       }
       prev_true = std::min(prev_true, true_rr);
+      if (mg && (mg_failed || stalled)) {
+        mg = false;
+        stagnant = 0;
+        h->beta = 0.0;
+      } else if (stalled) {
+        break;
+      }
     }
   }
   NGPB_HIP(hipEventRecord(e1, c->stream));
@@ -1478,8 +1593,13 @@ void solve_mixed(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
   st.replacements = repl;
   st.relres = bb > 0 ? std::sqrt(true_rr / bb) : 0.0;
   st.ms_solve = ms;
-  // SpMV + update (rhat, q read; rhat written) + direction (rhat, p, xhat read; p, xhat written)
-  st.bytes_per_iter = spmv_compact_bytes(c) + (double)n * 4.0 * (3.0 + 5.0);
+  // SpMV + update (rhat, q read; rhat written) + direction (rhat, p, xhat read; p, xhat
+  // written); with the preconditioner three SpMVs, the vector streams of its five row
+  // kernels (25 x 4 bytes) and the uniform levels (the dense array twice, then some 100
+  // bytes per node of the first level and an eighth of that for each further one)
+  st.bytes_per_iter = mg ? 3.0 * spmv_compact_bytes(c) + (double)n * 100.0 + 4.0 * (double)c->mg_dense.n +
+                               115.0 * (double)c->mg.lev[0].nodes()
+                         : spmv_compact_bytes(c) + (double)n * 4.0 * (3.0 + 5.0);
   c->have_phi = true;
   c->phi_len = c->n;
 }

@@ -60,7 +60,9 @@ enum ngpb_status_code {
 
 enum ngpb_precision {
   NGPB_PREC_FP64 = 0,  /* plain method: FP64 CSR, FP64 vectors, Jacobi PCG (LIS -i cg -p jacobi) */
-  NGPB_PREC_MIXED = 1  /* FP32 compact operator + FP32 inner CG, FP64 residual/reductions/update */
+  NGPB_PREC_MIXED = 1  /* FP32 compact operator + FP32 inner CG, FP64 residual/reductions/update;
+                          on octree meshes with Dirichlet data on the box faces the inner CG is
+                          preconditioned by a multigrid cycle on top of the Jacobi scaling */
 };
 
 /* Model parameters (relative permittivities, temperature in K, ionic strength in M). */

@@ -1,0 +1,106 @@
+"""The multigrid preconditioner of the mixed solve (csrc/ngpb_mg.hip).
+
+Each system's mixed potential against its FP64 solve to 1e-12: both stop on the true
+residual (1e-10 of ||b||), so the difference is bounded by the condition of the scaled
+operator times 1e-10; 1e-8 leaves a factor of 100 over the largest measured (3e-11 on
+meshes of this size). Sizes where a level can go wrong: 3 cells an axis (one coarse
+interior node), odd counts (the last coarse cell reaches past the box), boxes of uneven
+sides (a last level of several nodes), four refinement levels (nodes that live on levels
+2 to 4), rows in bands. Where the preconditioner does not apply (a lattice too sparse, a
+Dirichlet set other than the box faces, an operator loaded as CSR) the Jacobi-scaled
+iteration gives the same potential.
+"""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from cudanextgenpb_amd import native, workload as W
+from cudanextgenpb_amd.batch import prepare
+
+pytestmark = pytest.mark.gpu
+
+
+def box_spec(n, h=0.5, levels=0, bands=(), atoms=3):
+    n = np.asarray(n, np.int64)
+    half = 0.5 * n * h
+    rng = np.random.default_rng(int(n.sum()))
+    xyz = rng.uniform(-0.4, 0.4, (atoms, 3)) * half
+    a = W.Atoms(xyz, rng.uniform(0.3, 0.45, atoms) * half.min(), rng.normal(0.0, 0.5, atoms))
+    return W.Spec("box", W.Physics(), a, -half, h, n, levels, tuple(bands), 2, W.P4EST_TOL * n[0] * h)
+
+
+def solve_both(ctx):
+    phi64, st64 = ctx.solve(native.PREC_FP64, tol=1e-12)
+    phi, st = ctx.solve(native.PREC_MIXED, tol=1e-10)
+    rel = np.linalg.norm(phi - phi64) / np.linalg.norm(phi64)
+    print(f"   n={ctx.n}: FP64 {st64['iterations']} it, mixed {st['iterations']} it, phi rel {rel:.1e}", flush=True)
+    assert st["status"] == 0 and st["relres"] <= 1e-10 and rel <= 1e-8
+    return phi, st
+
+
+@pytest.mark.parametrize("n", [(3, 3, 3), (4, 4, 4), (5, 4, 7), (9, 8, 11), (17, 33, 16), (12, 40, 96), (64, 64, 64),
+                               (61, 61, 61)])
+def test_uniform_boxes(n):
+    print(f"[mg] uniform box {n}", flush=True)
+    p = prepare(box_spec(n))
+    phi, st = solve_both(p.ctx)
+    assert st["iterations"] <= 60
+    again, _ = p.ctx.solve(native.PREC_MIXED, tol=1e-10)
+    assert np.array_equal(phi, again)
+    p.ctx.close()
+
+
+@pytest.mark.parametrize("levels,bands,n", [(1, (1.0,), 40), (2, (1.0, 2.5), 48), (3, (1.0, 2.5, 5.0), 64),
+                                            (4, (1.0, 2.0, 4.0, 8.0), 64)])
+def test_octree_levels(levels, bands, n):
+    print(f"[mg] {levels} refinement levels", flush=True)
+    p = prepare(box_spec((n, n, n), levels=levels, bands=bands, atoms=4))
+    phi, st = solve_both(p.ctx)
+    assert st["iterations"] <= 60
+    p.ctx.set_row_order(4)
+    banded, _ = p.ctx.solve(native.PREC_MIXED, tol=1e-10)
+    assert np.linalg.norm(banded - phi) <= 1e-8 * np.linalg.norm(phi)
+    p.ctx.close()
+
+
+def test_sparse_lattice_uses_jacobi():
+    """More than 32 finest-lattice vertices per node: the dense transfer array is not built."""
+    p = prepare(box_spec((192, 192, 192), h=0.25, levels=4, bands=(0.1, 0.1, 0.1, 0.1), atoms=1))
+    assert 193 ** 3 > 32 * p.n
+    _, st = solve_both(p.ctx)
+    p.ctx.close()
+
+
+def test_other_dirichlet_sets_and_csr_use_jacobi():
+    P = W.three_spheres()
+    ctx = native.Context(0)
+    ctx.set_physics(P.physics)
+    ctx.set_mesh(P.mesh)
+    ctx.set_rays(P.rays)
+    ctx.create_markers()
+    ctx.set_charges(P.atoms.xyz, P.atoms.q, P.owner)
+    inner = int(np.argmin(np.abs(P.mesh.node_xyz).sum(axis=1)))
+    nodes = np.append(P.mesh.bnd_nodes, inner).astype(np.int32)  # one fixed node inside
+    ctx.set_dirichlet(nodes, np.linspace(0.0, 0.1, len(nodes)))
+    ctx.assemble()
+    solve_both(ctx)
+    csr = ctx.export_csr()
+    ctx.close()
+    other = native.Context(0)
+    other.set_csr(*csr)
+    solve_both(other)
+    other.close()
+
+
+def test_host_mesh_equals_device_mesh():
+    """The hierarchy is found from the mesh arrays alone: a mesh handed over by the caller
+    and the same mesh built on the device give the same potential bit for bit."""
+    P = W.three_spheres()
+    out = []
+    for device_mesh in (False, True):
+        p = prepare(P, device_mesh=device_mesh)
+        out.append(p.ctx.solve(native.PREC_MIXED, tol=1e-10))
+        p.ctx.close()
+    assert out[0][1]["iterations"] == out[1][1]["iterations"] <= 60
+    assert np.array_equal(out[0][0], out[1][0])
