@@ -86,7 +86,7 @@ int64_t ngpb_ctx::device_bytes() const {
        sell_list_packed.bytes() + sell_list_offset.bytes() + sell_dpair.bytes() + sell_pk_hdr_list.bytes();
   b += x.bytes() + r.bytes() + z.bytes() + p.bytes() + q.bytes() + dinv.bytes();
   b += lis_rt.bytes() + lis_u.bytes() + lis_v.bytes() + lis_ph.bytes() + lis_uh.bytes() + lis_t.bytes() +
-       diag_pos.bytes() + lev_rows_f.bytes() + lev_rows_b.bytes();
+       diag_pos.bytes() + ssor_f.bytes() + ssor_b.bytes();
   b += xs.bytes() + rs.bytes() + ps.bytes() + qs.bytes() + ks.bytes();
   b += mg_pool.bytes() + mg_dense.bytes() + mg_sd.bytes() + mg_r.bytes() + mg_z.bytes() + mg_pos.bytes();
   b += red.partials.bytes() + scan_tmp.bytes();

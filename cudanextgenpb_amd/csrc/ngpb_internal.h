@@ -327,8 +327,21 @@ struct ngpb_ctx {
   ngpb::DBuf<double> lis_rt, lis_u, lis_v, lis_ph, lis_uh, lis_t;
   bool have_levels = false;
   ngpb::DBuf<int32_t> diag_pos;              // position of each row's diagonal entry
-  ngpb::DBuf<int32_t> lev_rows_f, lev_rows_b;  // rows by forward / backward level
-  std::vector<int64_t> lev_ptr_f, lev_ptr_b;   // level offsets (host)
+  // one triangle in level order (the values are packed at each solve)
+  struct SsorTriangle {
+    struct Run {
+      int32_t first, last;  // pieces of narrow levels, or the positions of one wide level
+      bool pieces;
+    };
+    std::vector<Run> runs;
+    ngpb::DBuf<int32_t> rows, pos, from, ptr, col;
+    ngpb::DBuf<int2> pieces;
+    ngpb::DBuf<double> val, dinv, own, z;
+    int64_t bytes() const {
+      return rows.bytes() + pos.bytes() + from.bytes() + ptr.bytes() + pieces.bytes() + col.bytes() + val.bytes() +
+             dinv.bytes() + own.bytes() + z.bytes();
+    }
+  } ssor_f, ssor_b;
   ngpb::DBuf<float> xs, rs, ps, qs;
   ngpb::DBuf<ngpb::KrylovScalars> ks;
   ngpb::KrylovScalars* ks_host = nullptr;  // pinned mirror

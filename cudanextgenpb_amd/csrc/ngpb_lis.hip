@@ -16,9 +16,17 @@
 //
 // The sweeps are level-scheduled: a row's forward level is one more than the largest
 // level among its lower neighbours (backward: upper neighbours), so the rows of one
-// level are independent and one launch per level processes them, one thread per row.
-// The levels depend only on the sparsity pattern and are built once per pattern on
-// the host from the CSR (rows sorted by level, ascending row within a level).
+// level are independent. The levels depend only on the sparsity pattern and are built
+// once per pattern on the host from the CSR. Rows take positions in level order; a
+// sweep's vectors and entries are packed in that order and name neighbours by position.
+//
+// A sweep is a serial chain of levels (427 on a 255,000-row protein mesh, 600 rows each
+// on average), so its time is the chain's latency. Runs of levels of up to kNarrow rows
+// go to one block (k_ssor_run), piece by piece (a piece: rows of one level that fit the
+// staging buffers): the next pieces' entries stream into LDS while one is solved, the
+// solution of the last kWindow positions stays in LDS, and pieces are separated by a
+// block barrier. Wider levels, which fill more than one compute unit, are launched one by
+// one (k_ssor_level).
 //
 // Reductions follow the FP64 CG: per-block partials, summed in a fixed order by a
 // one-block finalize kernel that also updates the scalars and the stop flag; every
@@ -27,6 +35,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "ngpb_internal.h"
@@ -302,45 +311,299 @@ __global__ void __launch_bounds__(kBS) k_jacobi_apply(int64_t n, const double* _
     out[i] = dinv[i] * in[i];
 }
 
-// One level of the SSOR forward sweep: z_i = (r_i - w sum_{j<i} a_ij z_j) d_i^-1.
-__global__ void __launch_bounds__(kBS) k_ssor_fwd(const int32_t* __restrict__ rows, int cnt,
-                                                  const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
-                                                  const double* __restrict__ val, const int32_t* __restrict__ diag,
-                                                  const double* __restrict__ dinv, double w,
-                                                  const double* __restrict__ r, double* z, const KrylovScalars* ks) {
-  if (ks->done) return;
-  const int k = blockIdx.x * kBS + threadIdx.x;
-  if (k >= cnt) return;
-  const int32_t i = rows[k];
-  double t = r[i];
-  for (int32_t e = rowptr[i], de = diag[i]; e < de; ++e) t = t - (w * val[e]) * z[col[e]];
-  z[i] = t * dinv[i];
+// ---- SSOR sweeps
+constexpr int kRunBS = 1024;
+constexpr int kPieceRows = 512;
+constexpr int kPieceEntries = 4 * (kRunBS - kPieceRows);
+constexpr int kWindow = 8192;  // positions kept in LDS (64 KB)
+// Widest level of a one-block run: four pieces, about 4 us, the time of a launch (5-6 us
+// per dependent level measured).
+constexpr int kNarrow = 2048;
+
+// One triangle in level order: position k has the entries ptr[k] .. ptr[k + 1).
+struct Sweep {
+  const int32_t* ptr;
+  const int32_t* col;   // neighbour's position
+  const double* val;    // forward: omega a_ij; backward: a_ij
+  const double* dinv;
+  const double* own;    // forward: r_i; backward: y_i
+  double* z;
+};
+
+template <bool FWD>
+__device__ __forceinline__ double ssor_add(double t, double p) {
+  return FWD ? t - p : t + p;
+}
+template <bool FWD>
+__device__ __forceinline__ double ssor_finish(double t, double own, double dinv, double w) {
+  return FWD ? t * dinv : own - (w * t) * dinv;
 }
 
-// One level of the backward sweep: z_i = z_i - (w sum_{j>i} a_ij z_j) d_i^-1.
-__global__ void __launch_bounds__(kBS) k_ssor_bwd(const int32_t* __restrict__ rows, int cnt,
-                                                  const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
-                                                  const double* __restrict__ val, const int32_t* __restrict__ diag,
-                                                  const double* __restrict__ dinv, double w, double* z,
-                                                  const KrylovScalars* ks) {
+// A level as one launch: forward z_i = (r_i - sum_{j<i} (w a_ij) z_j) d_i^-1, backward
+// z_i = y_i - (w sum_{j>i} a_ij z_j) d_i^-1.
+template <bool FWD>
+__global__ void __launch_bounds__(kBS) k_ssor_level(Sweep S, int first, int end, double w, const KrylovScalars* ks) {
   if (ks->done) return;
-  const int k = blockIdx.x * kBS + threadIdx.x;
-  if (k >= cnt) return;
-  const int32_t i = rows[k];
-  double t = 0.0;
-  for (int32_t e = diag[i] + 1, ee = rowptr[i + 1]; e < ee; ++e) t = t + val[e] * z[col[e]];
-  z[i] = z[i] - (w * t) * dinv[i];
+  const int k = first + (int)(blockIdx.x * kBS + threadIdx.x);
+  if (k >= end) return;
+  const double own = S.own[k];
+  double t = FWD ? own : 0.0;
+  for (int32_t e = S.ptr[k], ee = S.ptr[k + 1]; e < ee; ++e) t = ssor_add<FWD>(t, S.val[e] * S.z[S.col[e]]);
+  S.z[k] = ssor_finish<FWD>(t, own, S.dinv[k], w);
 }
 
-// rows sorted by level (counting sort, ascending row within a level)
-void sort_by_level(const std::vector<int32_t>& lev, int32_t nlev, std::vector<int32_t>& rows,
-                   std::vector<int64_t>& ptr) {
-  ptr.assign((size_t)nlev + 1, 0);
-  for (int32_t l : lev) ++ptr[(size_t)l + 1];
-  for (int32_t l = 0; l < nlev; ++l) ptr[(size_t)l + 1] += ptr[(size_t)l];
-  std::vector<int64_t> fill(ptr.begin(), ptr.end() - 1);
-  rows.resize(lev.size());
-  for (size_t i = 0; i < lev.size(); ++i) rows[(size_t)fill[(size_t)lev[i]]++] = (int32_t)i;
+struct RunLds {
+  double z[kWindow];
+  struct {
+    double val[kPieceEntries];
+    int32_t col[kPieceEntries];
+  } piece[2];
+};
+static_assert(sizeof(RunLds) <= 160 * 1024, "one block's LDS");
+
+// The pieces [i0, i1) of a run in one block, a barrier between pieces. Threads
+// 0 .. kPieceRows - 1 solve piece i, a row each, from one LDS buffer, while the others
+// write the entries of piece i + 1 to the other buffer; all loads are issued two to six
+// pieces ahead. Neighbours within the last kWindow positions come from LDS; for an older
+// one (or one of an earlier launch) the entry's value is replaced by its product when
+// the entry is written (column -1), with a value loaded past the L1 two pieces before.
+// It is in memory by then: at least 16 - 3 pieces old, and every solving wave completes
+// all its stores every 8 pieces.
+//
+// Every load is unconditional (addresses clamped): the compiler can then count the
+// loads in flight and wait for just those it needs. A sweep over the 255,000-row mesh
+// took 2.3 ms with one launch per level; in one block 1.46 ms with guarded loads (each
+// piece waited for all of them), 0.92 ms with clamped loads and every thread doing both
+// jobs, 0.87 ms with loads one piece ahead of their use and 0.69 ms now, about 1 us a
+// piece. What bounds it is the latency of a piece, not bandwidth (22 GB/s).
+template <bool FWD>
+__global__ void __launch_bounds__(kRunBS) k_ssor_run(Sweep S, const int2* __restrict__ pieces, int i0, int i1,
+                                                     double w, const KrylovScalars* ks) {
+  extern __shared__ char s_mem[];
+  RunLds& L = *reinterpret_cast<RunLds*>(s_mem);
+  static_assert(kWindow >= 16 * kPieceRows, "older values must have left the store queue");
+  constexpr int kStagers = kRunBS - kPieceRows, kPer = kPieceEntries / kStagers;
+  static_assert(kPer * kStagers == kPieceEntries && kStagers % 64 == 0 && kPieceRows % 64 == 0, "");
+  if (ks->done) return;
+  struct Bounds {
+    int r0, r1, e0, e1;
+  };
+  auto bounds = [&](int i) {  // pieces past i1 are empty
+    const int2 p = pieces[min(i, i1)], q = pieces[min(i + 1, i1)];  // first position and entry
+    return Bounds{p.x, q.x, p.y, q.y};
+  };
+  // LDS writes are done at the barrier; loads in flight stay in flight
+  auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+  Bounds b[7];  // pieces i .. i + 6
+#pragma unroll
+  for (int u = 0; u < 7; ++u) b[u] = bounds(i0 + u);
+  auto next = [&](int i) {
+#pragma unroll
+    for (int u = 0; u < 6; ++u) b[u] = b[u + 1];
+    b[6] = bounds(i);
+  };
+
+  if (threadIdx.x < kPieceRows) {
+    const int t = threadIdx.x;
+    struct Row {
+      double own, dinv;
+      int32_t off, end;
+    } r[4];
+    auto load = [&](const Bounds& o, Row& q) {
+      const int k = max(min(o.r0 + t, o.r1 - 1), 0);
+      q.own = S.own[k];
+      q.dinv = S.dinv[k];
+      q.off = S.ptr[k];
+      q.end = S.ptr[k + 1];
+    };
+    // entries e .. e + N - 1 of a row that ends at ee, all LDS reads in flight together
+    auto add = [&](auto n, double acc, int e, int ee, const auto& p) {
+      constexpr int N = decltype(n)::value;
+      int32_t c[N];
+      double v[N], z[N];
+#pragma unroll
+      for (int u = 0; u < N; ++u) {
+        const int at = max(min(e + u, ee - 1), 0);
+        c[u] = p.col[at];
+        v[u] = p.val[at];
+      }
+#pragma unroll
+      for (int u = 0; u < N; ++u) z[u] = L.z[c[u] & (kWindow - 1)];
+#pragma unroll
+      for (int u = 0; u < N; ++u)
+        if (e + u < ee) acc = ssor_add<FWD>(acc, c[u] < 0 ? v[u] : v[u] * z[u]);
+      return acc;
+    };
+    auto solve = [&](const Bounds& o, const Row& q, const auto& p) {
+      if (t >= o.r1 - o.r0) return;
+      double acc = FWD ? q.own : 0.0;
+      const int e = q.off - o.e0, ee = q.end - o.e0;
+      // rows of a level are in the order of their counts: a wave's rows are mostly alike
+      if (!__any(ee - e > 4)) acc = add(std::integral_constant<int, 4>(), acc, e, ee, p);
+      else if (!__any(ee - e > 8)) acc = add(std::integral_constant<int, 8>(), acc, e, ee, p);
+      else
+        for (int x = e; __any(x < ee); x += 16) acc = add(std::integral_constant<int, 16>(), acc, x, ee, p);
+      const double z = ssor_finish<FWD>(acc, q.own, q.dinv, w);
+      const int k = o.r0 + t;
+      L.z[k & (kWindow - 1)] = z;
+      S.z[k] = z;
+    };
+#pragma unroll
+    for (int u = 0; u < 4; ++u) load(b[u], r[u]);
+    barrier();
+    for (int i = i0; i < i1; i += 8) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        solve(b[0], r[u & 3], L.piece[u & 1]);
+        load(b[4], r[u & 3]);
+        if (u == 7) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        barrier();
+        next(i + u + 7);
+      }
+    }
+  } else {
+    const int t = threadIdx.x - kPieceRows;
+    const int run0 = pieces[i0].x;
+    int32_t col[8][kPer];  // loaded six pieces ahead,
+    double val[4][kPer];   // four,
+    double far[4][kPer];   // and three
+    auto oldest = [&](const Bounds& q) { return max(run0, q.r1 - kWindow); };
+    auto entry = [&](const Bounds& q, int u) { return max(min(q.e0 + u * kStagers + t, q.e1 - 1), 0); };
+    auto load_col = [&](const Bounds& q, int32_t* c) {
+#pragma unroll
+      for (int u = 0; u < kPer; ++u) c[u] = S.col[entry(q, u)];
+    };
+    auto load_val = [&](const Bounds& q, double* v) {
+#pragma unroll
+      for (int u = 0; u < kPer; ++u) v[u] = S.val[entry(q, u)];
+    };
+    // lanes without an old neighbour read position 0: one request for all of them
+    auto load_far = [&](const Bounds& q, const int32_t* c, double* f) {
+      const int lo = oldest(q);
+#pragma unroll
+      for (int u = 0; u < kPer; ++u)
+        f[u] = __hip_atomic_load(S.z + (c[u] < lo ? c[u] : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    auto store = [&](const Bounds& q, const int32_t* c, const double* v, const double* f, auto& p) {
+      const int lo = oldest(q);
+#pragma unroll
+      for (int u = 0; u < kPer; ++u) {
+        const int e = u * kStagers + t;
+        if (e < q.e1 - q.e0) {
+          const bool old = c[u] < lo;
+          p.val[e] = old ? v[u] * f[u] : v[u];
+          p.col[e] = old ? -1 : c[u];
+        }
+      }
+    };
+#pragma unroll
+    for (int u = 0; u < 6; ++u) load_col(b[u], col[u]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) load_val(b[u], val[u]);
+#pragma unroll
+    for (int u = 0; u < 3; ++u) load_far(b[u], col[u], far[u]);
+    store(b[0], col[0], val[0], far[0], L.piece[0]);
+    barrier();
+    for (int i = i0; i < i1; i += 8) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        load_far(b[3], col[(u + 3) & 7], far[(u + 3) & 3]);
+        load_val(b[4], val[u & 3]);
+        load_col(b[6], col[(u + 6) & 7]);
+        store(b[1], col[(u + 1) & 7], val[(u + 1) & 3], far[(u + 1) & 3], L.piece[(u + 1) & 1]);
+        barrier();
+        next(i + u + 7);
+      }
+    }
+  }
+}
+
+// entries of a triangle in level order
+template <bool FWD>
+__global__ void __launch_bounds__(kBS) k_ssor_pack(int64_t n, const int32_t* __restrict__ row,
+                                                   const int32_t* __restrict__ rowptr,
+                                                   const int32_t* __restrict__ diag, const int32_t* __restrict__ ccol,
+                                                   const double* __restrict__ cval, const double* __restrict__ dinv,
+                                                   const int32_t* __restrict__ pos, const int32_t* __restrict__ ptr,
+                                                   double w, int32_t* __restrict__ col, double* __restrict__ val,
+                                                   double* __restrict__ pdinv) {
+  const int64_t k = (int64_t)blockIdx.x * kBS + threadIdx.x;
+  if (k >= n) return;
+  const int32_t i = row[k];
+  pdinv[k] = dinv[i];
+  const int32_t b = FWD ? rowptr[i] : diag[i] + 1, e = FWD ? diag[i] : rowptr[i + 1];
+  const int32_t o = ptr[k];
+  for (int32_t t = b; t < e; ++t) {
+    col[o + t - b] = pos[ccol[t]];
+    val[o + t - b] = FWD ? w * cval[t] : cval[t];
+  }
+}
+
+// out[k] = in[idx[k]]: a vector into level order, from one sweep's order to the other's,
+// or back to row order
+__global__ void __launch_bounds__(kBS) k_ssor_gather(int64_t n, const int32_t* __restrict__ idx,
+                                                     const double* __restrict__ in, double* __restrict__ out,
+                                                     const KrylovScalars* ks) {
+  if (ks->done) return;
+  const int64_t k = (int64_t)blockIdx.x * kBS + threadIdx.x;
+  if (k < n) out[k] = in[idx[k]];
+}
+
+// A triangle in level order: rows (by falling entry count within a level, so that a
+// wave's rows are alike, then ascending), their positions, entry
+// offsets, and the launches of a sweep: pieces of narrow levels and single wide levels.
+// cnt(i): entries of row i.
+template <class Cnt>
+void order_triangle(ngpb_ctx* c, ngpb_ctx::SsorTriangle& t, const std::vector<int32_t>& lev, int32_t nlev, Cnt&& cnt) {
+  const size_t n = lev.size();
+  std::vector<int32_t> first((size_t)nlev + 1, 0), rows(n), pos(n), ptr(n + 1, 0);
+  for (int32_t l : lev) ++first[(size_t)l + 1];
+  for (int32_t l = 0; l < nlev; ++l) first[(size_t)l + 1] += first[(size_t)l];
+  std::vector<int32_t> fill(first.begin(), first.end() - 1);
+  int32_t longest = 0;
+  for (size_t i = 0; i < n; ++i) longest = std::max(longest, cnt(i));
+  std::vector<int32_t> by_count(n), start((size_t)longest + 2, 0);
+  for (size_t i = 0; i < n; ++i) ++start[(size_t)(longest - cnt(i)) + 1];
+  for (int32_t q = 0; q <= longest; ++q) start[(size_t)q + 1] += start[(size_t)q];
+  for (size_t i = 0; i < n; ++i) by_count[(size_t)start[(size_t)(longest - cnt(i))]++] = (int32_t)i;
+  for (int32_t i : by_count) {
+    const int32_t k = fill[(size_t)lev[(size_t)i]]++;
+    rows[(size_t)k] = i;
+    pos[(size_t)i] = k;
+  }
+  for (size_t k = 0; k < n; ++k) ptr[k + 1] = ptr[k] + cnt((size_t)rows[k]);
+  t.runs.clear();
+  std::vector<int32_t> pieces;
+  for (int32_t l = 0; l < nlev; ++l) {
+    const int32_t a = first[(size_t)l], b = first[(size_t)l + 1];
+    if (b - a > kNarrow || longest > kPieceEntries) {
+      t.runs.push_back({a, b, false});
+      continue;
+    }
+    if (t.runs.empty() || !t.runs.back().pieces) {
+      t.runs.push_back({(int32_t)pieces.size(), (int32_t)pieces.size(), true});
+      pieces.push_back(a);
+    }
+    for (int32_t k = a; k < b;) {
+      int32_t e = k;
+      while (e < b && e - k < kPieceRows && ptr[(size_t)e + 1] - ptr[(size_t)k] <= kPieceEntries) ++e;
+      pieces.push_back(e);  // the end of this piece, the start of the next
+      k = e;
+    }
+    t.runs.back().last = (int32_t)pieces.size() - 1;
+  }
+  t.rows.upload(rows.data(), n, c->stream);
+  t.pos.upload(pos.data(), n, c->stream);
+  t.ptr.upload(ptr.data(), n + 1, c->stream);
+  std::vector<int2> starts;
+  for (int32_t k : pieces) starts.push_back(make_int2(k, ptr[(size_t)k]));
+  t.pieces.upload(starts.data(), starts.size(), c->stream);
+  t.col.resize((size_t)std::max(ptr[n], 1));
+  t.val.resize((size_t)std::max(ptr[n], 1));
+  t.dinv.resize(n);
+  t.own.resize(n);
+  t.z.resize(n);
+  NGPB_HIP(hipStreamSynchronize(c->stream));  // the host arrays end here
 }
 
 }  // namespace
@@ -371,17 +634,47 @@ void build_ssor_levels(ngpb_ctx* c) {
     lb[(size_t)i] = l;
     nb = std::max(nb, l + 1);
   }
-  std::vector<int32_t> rows;
-  sort_by_level(lf, nf, rows, c->lev_ptr_f);
-  c->lev_rows_f.upload(rows.data(), rows.size(), c->stream);
-  sort_by_level(lb, nb, rows, c->lev_ptr_b);
-  c->lev_rows_b.upload(rows.data(), rows.size(), c->stream);
-  c->diag_pos.upload(diag.data(), diag.size(), c->stream);
-  NGPB_HIP(hipStreamSynchronize(c->stream));
+  order_triangle(c, c->ssor_f, lf, nf, [&](size_t i) { return diag[i] - rp[i]; });
+  order_triangle(c, c->ssor_b, lb, nb, [&](size_t i) { return rp[i + 1] - diag[i] - 1; });
+  {  // the backward sweep takes the forward sweep's result from the forward positions
+    std::vector<int32_t> rows((size_t)n), pos((size_t)n), from((size_t)n);
+    c->ssor_b.rows.download(rows.data(), rows.size(), c->stream);
+    c->ssor_f.pos.download(pos.data(), pos.size(), c->stream);
+    NGPB_HIP(hipStreamSynchronize(c->stream));
+    for (size_t k = 0; k < from.size(); ++k) from[k] = pos[(size_t)rows[k]];
+    c->ssor_b.from.upload(from.data(), from.size(), c->stream);
+    c->diag_pos.upload(diag.data(), diag.size(), c->stream);
+    NGPB_HIP(hipStreamSynchronize(c->stream));
+  }
   c->have_levels = true;
 }
 
 namespace {
+
+// One sweep over the runs of a triangle; t.own holds its input, t.z takes its result.
+template <bool FWD>
+void sweep(ngpb_ctx* c, const ngpb_ctx::SsorTriangle& t, double w) {
+  const Sweep S{t.ptr.p, t.col.p, t.val.p, t.dinv.p, t.own.p, t.z.p};
+  for (const auto& r : t.runs) {
+    if (r.pieces)
+      hipLaunchKernelGGL(k_ssor_run<FWD>, dim3(1), dim3(kRunBS), sizeof(RunLds), c->stream, S, t.pieces.p, r.first,
+                         r.last, w, c->ks.p);
+    else
+      hipLaunchKernelGGL(k_ssor_level<FWD>, dim3(blocks_for(r.last - r.first, kBS)), dim3(kBS), 0, c->stream, S,
+                         r.first, r.last, w, c->ks.p);
+  }
+}
+
+// The packed entries of one triangle for the current values and relaxation.
+template <bool FWD>
+void pack_triangle(ngpb_ctx* c, ngpb_ctx::SsorTriangle& t, double w) {
+  hipLaunchKernelGGL(k_ssor_pack<FWD>, dim3(blocks_for(c->n, kBS)), dim3(kBS), 0, c->stream, c->n, t.rows.p,
+                     c->rowptr.p, c->diag_pos.p, c->col.p, c->val.p, c->dinv.p, t.pos.p, t.ptr.p, w, t.col.p, t.val.p,
+                     t.dinv.p);
+  NGPB_HIP(hipGetLastError());
+  NGPB_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_ssor_run<FWD>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(RunLds)));
+}
 
 // z = M^-1 in; returns the vector that holds the result (`in` itself without a
 // preconditioner). c->dinv must hold the inverse diagonal.
@@ -393,25 +686,21 @@ const double* psolve(ngpb_ctx* c, int precon, double w, const double* in, double
     hipLaunchKernelGGL(k_jacobi_apply, dim3(vec_grid(n)), dim3(kBS), 0, c->stream, n, c->dinv.p, in, out, ks);
     return out;
   }
-  const size_t nf = c->lev_ptr_f.size() - 1, nb = c->lev_ptr_b.size() - 1;
-  for (size_t l = 0; l < nf; ++l) {
-    const int64_t o = c->lev_ptr_f[l], cnt = c->lev_ptr_f[l + 1] - o;
-    hipLaunchKernelGGL(k_ssor_fwd, dim3((unsigned)((cnt + kBS - 1) / kBS)), dim3(kBS), 0, c->stream,
-                       c->lev_rows_f.p + o, (int)cnt, c->rowptr.p, c->col.p, c->val.p, c->diag_pos.p, c->dinv.p, w,
-                       in, out, ks);
-  }
-  for (size_t l = 0; l < nb; ++l) {
-    const int64_t o = c->lev_ptr_b[l], cnt = c->lev_ptr_b[l + 1] - o;
-    hipLaunchKernelGGL(k_ssor_bwd, dim3((unsigned)((cnt + kBS - 1) / kBS)), dim3(kBS), 0, c->stream,
-                       c->lev_rows_b.p + o, (int)cnt, c->rowptr.p, c->col.p, c->val.p, c->diag_pos.p, c->dinv.p, w,
-                       out, ks);
-  }
+  const dim3 G(blocks_for(n, kBS)), B(kBS);
+  hipLaunchKernelGGL(k_ssor_gather, G, B, 0, c->stream, n, c->ssor_f.rows.p, in, c->ssor_f.own.p, ks);
+  sweep<true>(c, c->ssor_f, w);
+  hipLaunchKernelGGL(k_ssor_gather, G, B, 0, c->stream, n, c->ssor_b.from.p, c->ssor_f.z.p, c->ssor_b.own.p, ks);
+  sweep<false>(c, c->ssor_b, w);
+  hipLaunchKernelGGL(k_ssor_gather, G, B, 0, c->stream, n, c->ssor_b.pos.p, c->ssor_b.z.p, out, ks);
   return out;
 }
 
-void prepare_precon(ngpb_ctx* c, int precon) {
+void prepare_precon(ngpb_ctx* c, int precon, double w) {
   check_operator(c);  // inverse diagonal, NaN/Inf and diagonal checks
-  if (precon == NGPB_PRECON_SSOR && !c->have_levels) build_ssor_levels(c);
+  if (precon != NGPB_PRECON_SSOR) return;
+  if (!c->have_levels) build_ssor_levels(c);
+  pack_triangle<true>(c, c->ssor_f, w);
+  pack_triangle<false>(c, c->ssor_b, w);
 }
 
 }  // namespace
@@ -428,7 +717,7 @@ void check_lis_options(const ngpb_solve_opts& o) {
 }
 
 void precond_apply(ngpb_ctx* c, int precon, double omega, const double* r, double* z) {
-  prepare_precon(c, precon);
+  prepare_precon(c, precon, omega);
   ensure_reduce(c, 2048);
   KrylovScalars zero;
   std::memset(&zero, 0, sizeof(zero));
@@ -443,7 +732,7 @@ void solve_lis(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
   check_lis_options(o);
   const int64_t n = c->n;
   const double w = ssor_omega(o);
-  prepare_precon(c, o.precon);
+  prepare_precon(c, o.precon, w);
   c->x.resize((size_t)n);
   c->r.resize((size_t)n);
   c->z.reserve((size_t)n);
