@@ -8,9 +8,10 @@
 #include <cstring>
 #include <map>
 #include <mutex>
-#include <unordered_map>
 #include <sstream>
 #include <string>
+#include <unordered_map>
+#include <utility>
 #include <vector>
 
 #include "ngpb_internal.h"
@@ -145,6 +146,74 @@ void not_in_batch(const ngpb_ctx* c) {
 
 namespace ngpb {
 
+// ---- pool of idle blocks
+thread_local int IdleRelease::depth = 0;
+namespace {
+constexpr size_t kPoolMax = size_t(16) << 30;  // per device
+struct Pool {
+  std::multimap<size_t, void*> free;  // by size class
+  size_t bytes = 0;
+};
+std::mutex g_pool_mu;
+std::unordered_map<int, Pool> g_pool;  // by device
+
+size_t pool_class(size_t bytes) {
+  size_t step = 512;
+  while (step * 32 < bytes) step *= 2;  // step <= bytes / 16
+  return (bytes + step - 1) / step * step;
+}
+
+int current_device() {
+  int d = 0;
+  (void)hipGetDevice(&d);
+  return d;
+}
+}  // namespace
+
+void* pool_alloc(size_t bytes, size_t* cap) {
+  const size_t size = pool_class(bytes);
+  const int dev = current_device();
+  *cap = size;
+  {
+    std::lock_guard<std::mutex> g(g_pool_mu);
+    Pool& q = g_pool[dev];
+    auto f = q.free.find(size);
+    if (f != q.free.end()) {
+      void* p = f->second;
+      q.free.erase(f);
+      q.bytes -= size;
+      return p;
+    }
+  }
+  void* p = nullptr;
+  if (hipMalloc(&p, size) == hipSuccess) return p;
+  (void)hipGetLastError();
+  std::multimap<size_t, void*> all;  // give the pooled memory back and try once more
+  {
+    std::lock_guard<std::mutex> g(g_pool_mu);
+    Pool& q = g_pool[dev];
+    all.swap(q.free);
+    q.bytes = 0;
+  }
+  for (auto& f : all) (void)hipFree(f.second);
+  if (hipMalloc(&p, size) == hipSuccess) return p;
+  (void)hipGetLastError();
+  return nullptr;
+}
+
+void pool_free(void* p, size_t cap) {
+  {
+    std::lock_guard<std::mutex> g(g_pool_mu);
+    Pool& q = g_pool[current_device()];
+    if (q.bytes + cap <= kPoolMax) {
+      q.free.emplace(cap, p);
+      q.bytes += cap;
+      return;
+    }
+  }
+  (void)hipFree(p);
+}
+
 // ---- per-stream cache of released stream-ordered blocks
 // Bounds: a stream caches at most kCacheMax bytes during a call; at the end of an API
 // call it keeps at most kCacheKeep bytes, and none once the streams of all contexts
@@ -179,18 +248,23 @@ void* stream_cache_take(hipStream_t s, size_t bytes, size_t* cap) {
   return p;
 }
 
-bool stream_cache_put(hipStream_t s, void* p, size_t cap) {
-  std::lock_guard<std::mutex> g(g_cache_mu);
-  StreamBlocks& b = g_cache[s];
-  if (b.bytes + cap > kCacheMax) return false;
-  b.free.emplace(cap, p);
-  b.bytes += cap;
-  g_cached += cap;
-  return true;
+void stream_cache_put(hipStream_t s, void* p, size_t cap) {
+  {
+    std::lock_guard<std::mutex> g(g_cache_mu);
+    StreamBlocks& b = g_cache[s];
+    if (b.bytes + cap <= kCacheMax) {
+      b.free.emplace(cap, p);
+      b.bytes += cap;
+      g_cached += cap;
+      return;
+    }
+  }
+  if (hipStreamSynchronize(s) == hipSuccess) pool_free(p, cap);
+  else (void)hipFree(p);
 }
 
 void stream_cache_trim(hipStream_t s, size_t keep) {
-  std::vector<void*> out;
+  std::vector<std::pair<size_t, void*>> out;
   {
     std::lock_guard<std::mutex> g(g_cache_mu);
     auto it = g_cache.find(s);
@@ -199,13 +273,18 @@ void stream_cache_trim(hipStream_t s, size_t keep) {
     if (keep > 0 && g_cached > kGlobalKeep) keep = 0;
     while (b.bytes > keep && !b.free.empty()) {  // largest first
       auto f = std::prev(b.free.end());
-      out.push_back(f->second);
+      out.push_back(*f);
       b.bytes -= f->first;
       g_cached -= f->first;
       b.free.erase(f);
     }
   }
-  for (void* p : out) (void)hipFreeAsync(p, s);
+  if (out.empty()) return;
+  const bool idle = hipStreamSynchronize(s) == hipSuccess;
+  for (auto& f : out) {
+    if (idle) pool_free(f.second, f.first);
+    else (void)hipFree(f.second);
+  }
 }
 
 void stream_cache_end_call(hipStream_t s) { stream_cache_trim(s, kCacheKeep); }
@@ -266,17 +345,21 @@ int ngpb_destroy(ngpb_ctx* c) {
     return NGPB_E_STATE;
   }
   (void)hipSetDevice(c->device);
-  if (c->stream) (void)hipStreamSynchronize(c->stream);
+  const bool idle = c->stream && hipStreamSynchronize(c->stream) == hipSuccess;
   if (c->ks_host) (void)hipHostFree(c->ks_host);
   for (auto& p : c->kprof)
     for (hipEvent_t e : p.ev) (void)hipEventDestroy(e);
   c->ks_host = nullptr;
   if (c->stream) {
     ngpb::stream_cache_drop(c->stream);
-    (void)hipStreamSynchronize(c->stream);
     (void)hipStreamDestroy(c->stream);
   }
-  delete c;  // device buffers free themselves
+  if (idle) {  // every kernel on the context's buffers has ended: they go to the pool
+    ngpb::IdleRelease pool;
+    delete c;
+  } else {
+    delete c;
+  }
   return NGPB_OK;
 }
 
@@ -775,6 +858,8 @@ int ngpb_assemble_many(ngpb_ctx* const* cs, int n) {
     if (rc != NGPB_OK) return rc;
   }
   auto fail_all = [&](int code, const std::string& msg) {
+    // stages already enqueued use every context's arrays from the first one's stream
+    (void)hipStreamSynchronize(v[0]->stream);
     for (ngpb_ctx* c : v) c->err = msg;
     return code;
   };

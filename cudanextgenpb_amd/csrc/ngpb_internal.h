@@ -35,34 +35,52 @@ struct Error : std::runtime_error {
   } while (0)
 
 // --------------------------------------------------------------- device buffers
+// Process-wide pool of idle device blocks, by device and size class (16 classes per
+// power of two: a block is at most 6.25% larger than asked for). A destroyed context's
+// blocks and the blocks its stream's cache gives up go there once the stream is idle,
+// so the next context takes them without the driver: hipFree of a context's ~150
+// buffers took 10 ms (64^3 ligand) to 25 ms (8M unknowns), and a process that frees and
+// allocates gigabytes per request soon waits for the driver to clear the memory (160 ->
+// 395 ms per 8M-unknown request). A pooled block is idle: no stream has work pending on
+// it, whichever thread or stream takes it next. The pool holds at most 16 GiB per device
+// (more is freed) and gives everything back when an allocation fails.
+void* pool_alloc(size_t bytes, size_t* cap);  // nullptr: out of memory
+void pool_free(void* p, size_t cap);          // p must be idle
+// While an object of this type lives, this thread's plain buffers are released to the
+// pool: their users have been waited for.
+struct IdleRelease {
+  static thread_local int depth;
+  IdleRelease() { ++depth; }
+  ~IdleRelease() { --depth; }
+};
+
 // Blocks of stream-ordered buffers released on a stream are kept for later buffers on
 // the same stream (stream order makes the reuse safe: every use of the old buffer was
 // enqueued before every use of the new one), so a call's repeated temporaries (the
 // per-axis arrays of a ray cast, the per-level arrays of an octree build) are not
-// handed back to the driver and fetched again: a hipFreeAsync of a 64 MB block has
-// held the host for ~5 ms. No events are involved, so no thread ever waits on work
-// of another thread's stream. stream_cache_take returns a block of at least `bytes`
-// (and not much more) with its size in *cap, or nullptr; stream_cache_put returns
-// false when the stream's cache is full (the caller frees the block);
-// stream_cache_trim frees blocks until at most `keep` bytes stay cached;
+// fetched again. No events are involved, so no thread ever waits on work of another
+// thread's stream. stream_cache_take returns a block of at least `bytes` (and not much
+// more) with its size in *cap, or nullptr; stream_cache_put takes a block back, waiting
+// for the stream and passing it to the pool when the stream's cache is full;
+// stream_cache_trim passes blocks on until at most `keep` bytes stay cached;
 // stream_cache_end_call trims to the bound kept between API calls; and
-// stream_cache_drop frees them all (before the stream is destroyed).
+// stream_cache_drop passes all on (before the stream is destroyed).
 void* stream_cache_take(hipStream_t s, size_t bytes, size_t* cap);
-bool stream_cache_put(hipStream_t s, void* p, size_t cap);
+void stream_cache_put(hipStream_t s, void* p, size_t cap);
 void stream_cache_trim(hipStream_t s, size_t keep);
 void stream_cache_end_call(hipStream_t s);
 void stream_cache_drop(hipStream_t s);
 
-// A buffer constructed with a stream (or given one by order_on) is allocated and
-// freed in that stream's order (hipMallocAsync / hipFreeAsync, through the stream's
-// block cache): freeing it waits neither for the device nor for other streams, which
-// matters for the temporaries of one call while other contexts' work runs on the
-// same GPU. The others use hipMalloc / hipFree (the resident arrays of a context).
+// A buffer constructed with a stream (or given one by order_on) is released in that
+// stream's order, to the stream's block cache: releasing it waits neither for the device
+// nor for other streams, which matters for the temporaries of one call while other
+// contexts' work runs on the same GPU. The others are freed with hipFree (which waits for
+// the device), or to the pool under IdleRelease (the resident arrays of a context).
 template <class T>
 struct DBuf {
   T* p = nullptr;
   size_t n = 0;
-  size_t cap = 0;  // bytes of the block (stream-ordered buffers)
+  size_t cap = 0;  // bytes of the block
   hipStream_t os = nullptr;
   bool ordered = false;
   DBuf() = default;
@@ -77,8 +95,9 @@ struct DBuf {
   }
   void release() {
     if (p) {
-      if (!ordered) (void)hipFree(p);
-      else if (!stream_cache_put(os, p, cap)) (void)hipFreeAsync(p, os);
+      if (ordered) stream_cache_put(os, p, cap);
+      else if (IdleRelease::depth > 0) pool_free(p, cap);
+      else (void)hipFree(p);
     }
     p = nullptr;
     n = 0;
@@ -94,12 +113,10 @@ struct DBuf {
       n = count;
       return;
     }
-    cap = bytes;
-    hipError_t e = ordered ? hipMallocAsync((void**)&p, bytes, os) : hipMalloc((void**)&p, bytes);
-    if (e != hipSuccess) {
-      p = nullptr;
-      (void)hipGetLastError();
-      throw Error(NGPB_E_NOMEM, "hipMalloc of " + std::to_string(count * sizeof(T)) + " bytes failed");
+    p = static_cast<T*>(pool_alloc(bytes, &cap));
+    if (!p) {
+      cap = 0;
+      throw Error(NGPB_E_NOMEM, "hipMalloc of " + std::to_string(bytes) + " bytes failed");
     }
     n = count;
   }
