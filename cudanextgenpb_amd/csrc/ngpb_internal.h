@@ -486,14 +486,15 @@ double time_spmv_compact(ngpb_ctx* c, int reps);
 // mg_precondition, an SpMV on z, mg_direction, an SpMV on p and mg_update. par is the
 // parity of the iteration; every kernel returns at once after the stop flag.
 bool mg_setup(ngpb_ctx* c);
-// z0 from r and ar = Ahat r; stops first if (r, r) from the partials met the target
-void mg_precondition(ngpb_ctx* c, const float* r, const float* ar, float* z, const double* rr_part, int npr, int par,
-                     bool first);
-// z = z0 + omega (r - az), az = Ahat z0; p = z + beta p
-void mg_direction(ngpb_ctx* c, const float* r, const float* az, float* z, float* p, double* part, int par);
-// x += alpha p, r -= alpha ap, ap = Ahat p; per block (r, r)
-void mg_update(ngpb_ctx* c, float* x, float* r, const float* p, const float* ap, const double* pq_part, int npq,
-               double* part, int par);
+// z0 from r and ar = Ahat r, and (r, z) up to omega (r, r) in rz_part; stops first if
+// (r, r) from the partials met the target
+void mg_precondition(ngpb_ctx* c, const float* r, const float* ar, float* z, const double* rr_part, int npr,
+                     double* rz_part, int par, bool first);
+// x += alpha p of the iteration before; p = z + beta p, z = z0 + omega (r - az), az = Ahat z0
+void mg_direction(ngpb_ctx* c, const float* r, const float* az, const float* z, float* p, float* x,
+                  const double* rz_part, int par);
+// r -= alpha ap, ap = Ahat p; per block (r, r)
+void mg_update(ngpb_ctx* c, float* r, const float* ap, const double* pq_part, int npq, double* part, int par);
 
 // energy
 void run_energy(ngpb_ctx* c, ngpb_energy_out* out);

@@ -13,10 +13,6 @@ constexpr int kMgLevels = 10;  // 1022 cells an axis halve nine times
 // are ten or more times as many: at 18 per unknown (the 47,302-unknown mesh above) the
 // solve is still 1.5x faster, at twice that the two meet.
 constexpr int64_t kMgDenseRatio = 32;
-// largest level of the one-block bottom kernel and its LDS
-constexpr int64_t kMgBottomNodes = 9600;
-constexpr int64_t kMgBottomLds = 120 * 1024;
-
 // the finest lattice of the mesh's box
 struct MgBox {
   double x0[3] = {0, 0, 0};

@@ -24,9 +24,9 @@
 // positive definite operator and plain CG applies.
 //
 // Measured (tolerance 1e-10, solve alone, against Jacobi scaling): 8.04M unknowns 556 ->
-// 29 iterations, 57.8 -> 17.2 ms; 63.3M unknowns 892 iterations, 656 ms -> whole step 801
-// -> 283 ms; 274,625 unknowns (64^3 cells) 340 -> 22, 5.9 -> 2.4 ms; 47,302 unknowns 223
-// -> 26, 4.2 -> 2.8 ms. A cycle streams from HBM at the large sizes and is bound by the
+// 29 iterations, 57.8 -> 14.9 ms; 63.3M unknowns 892 iterations, 656 ms -> whole step 801
+// -> 283 ms; 274,625 unknowns (64^3 cells) 340 -> 22, 5.9 -> 2.1 ms; 47,302 unknowns 223
+// -> 26, 4.2 -> 2.6 ms. A cycle streams from HBM at the large sizes and is bound by the
 // latency of its ~20 launches at the small ones.
 //
 // All reductions have a fixed order and no kernel uses atomics on values: a repeated
@@ -37,7 +37,7 @@
 #include <vector>
 
 #include "ngpb_internal.h"
-#include "ngpb_mg.h"
+#include "ngpb_mg_dev.h"
 
 namespace ngpb {
 MeshView mesh_view_of(const ngpb_ctx* c);
@@ -45,10 +45,6 @@ MeshView mesh_view_of(const ngpb_ctx* c);
 namespace {
 
 constexpr int kBS = 256;
-// damping of the Jacobi smoother (22 and 27 iterations at 0.9, 23 and 28 at 0.8 on a
-// ligand and a 300-atom globule)
-constexpr float kOmega = 0.9f;
-constexpr int kBottomBS = 1024;
 
 // ------------------------------------------------------------------ setup
 __device__ __forceinline__ int axis_index(double x, double x0, double inv_h, int* bad) {
@@ -162,14 +158,14 @@ __global__ void __launch_bounds__(kBS) k_mg_rows(int64_t n, const double* __rest
   sd[r] = alone ? 0.f : (float)(1.0 / dscale[r]);
 }
 
-// coefficients of leaf l: per axis the mean of its four edges' permittivities, and the
-// mean screening term of its corners
-__device__ __forceinline__ float4 leaf_cell(const MeshView& m, int64_t l, const double* c_edge, const double* v8,
+// coefficients of leaf l of edge 1 / inv: per axis the mean of its four edges'
+// permittivities, and the mean screening term of its corners
+__device__ __forceinline__ float4 leaf_cell(const MeshView& m, int64_t l, double inv, const double* c_edge,
                                             const double* reac) {
   // edge order: x edges 0 2 4 6, y edges 1 3 5 7, z edges 8 .. 11; c_edge = eps h / 4
   const double* c = c_edge + 12 * l;
-  const double inv = 1.0 / cbrt(8.0 * v8[l]);
   double r = 0.0;
+#pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int32_t k = m.leaf_corner[8 * l + i];
     if (k >= 0) {
@@ -201,43 +197,50 @@ __device__ __forceinline__ float4 merge_cells(const float4* q) {
   return o;
 }
 
-// cells of level 1 (edge 2 hf) from the leaves: eight leaves of edge hf, or the one
-// larger leaf that holds the cell (found at its anchor)
+// Cells of level 1 (edge 2 hf) from the leaves, eight lanes a cell: eight leaves of edge
+// hf, one per lane, or the one larger leaf that holds the cell (found at its anchor). One
+// thread per cell took 1.0 ms on the 8M-node mesh, 96-byte leaf records read serially.
 __global__ void __launch_bounds__(kBS) k_mg_cells1(MeshView m, MgBox g, int cx, int cy, int cz,
                                                    const int32_t* __restrict__ map, const uint8_t* __restrict__ level,
-                                                   const double* __restrict__ c_edge, const double* __restrict__ v8,
+                                                   const double* __restrict__ c_edge,
                                                    const double* __restrict__ reac, float4* __restrict__ cells,
                                                    int* __restrict__ bad) {
-  const int64_t t = (int64_t)blockIdx.x * kBS + threadIdx.x;
-  if (t >= (int64_t)cx * cy * cz) return;
-  const int I = (int)(t % cx), J = (int)(t / cx % cy), K = (int)(t / ((int64_t)cx * cy));
-  auto at = [&](int i, int j, int k) { return map[((int64_t)k * g.n[1] + j) * g.n[0] + i]; };
-  const int32_t l0 = at(2 * I, 2 * J, 2 * K);
-  if (l0 >= 0 && level[l0] == 0) {
-    float4 q[8];
-    for (int c = 0; c < 8; ++c) {
-      const int32_t l = at(min(2 * I + (c & 1), g.n[0] - 1), min(2 * J + ((c >> 1) & 1), g.n[1] - 1),
-                           min(2 * K + (c >> 2), g.n[2] - 1));
-      if (l < 0) {
-        *bad = 1;
-        return;
+  const int64_t t = ((int64_t)blockIdx.x * kBS + threadIdx.x) >> 3;
+  const int c = threadIdx.x & 7;
+  const bool valid = t < (int64_t)cx * cy * cz;
+  float4 q = make_float4(1.f, 1.f, 1.f, 0.f);
+  if (valid) {
+    const int I = (int)(t % cx), J = (int)(t / cx % cy), K = (int)(t / ((int64_t)cx * cy));
+    auto at = [&](int i, int j, int k) { return map[((int64_t)k * g.n[1] + j) * g.n[0] + i]; };
+    int32_t l = at(min(2 * I + (c & 1), g.n[0] - 1), min(2 * J + ((c >> 1) & 1), g.n[1] - 1),
+                   min(2 * K + (c >> 2), g.n[2] - 1));
+    int s = 0;
+    if (l < 0 || level[l] != 0) {
+      l = -1;
+      for (s = 1; s <= 10 && l < 0; ++s) {
+        const int k = ~((1 << s) - 1);
+        const int32_t cand = at(2 * I & k, 2 * J & k, 2 * K & k);
+        if (cand >= 0 && level[cand] >= s) l = cand;
       }
-      q[c] = leaf_cell(m, l, c_edge, v8, reac);
+      if (l >= 0) s = level[l];
     }
-    cells[t] = merge_cells(q);
-    return;
+    if (l < 0) *bad = 1;
+    else q = leaf_cell(m, l, g.inv_h / (double)(1 << s), c_edge, reac);
   }
-  int32_t l = l0;
-  for (int s = 2; s <= 10 && l < 0; ++s) {
-    const int k = ~((1 << s) - 1);
-    const int32_t cand = at(2 * I & k, 2 * J & k, 2 * K & k);
-    if (cand >= 0 && level[cand] >= s) l = cand;
-  }
-  if (l < 0) {
-    *bad = 1;
-    return;
-  }
-  cells[t] = leaf_cell(m, l, c_edge, v8, reac);
+  // harmonic mean along the axis of the arithmetic means across it
+  auto axis = [&](float v, int along, int b0, int b1) {
+    v += __shfl_xor(v, b0, 64);
+    v += __shfl_xor(v, b1, 64);
+    return hmean(0.25f * v, 0.25f * __shfl_xor(v, along, 64));
+  };
+  float4 o;
+  o.x = axis(q.x, 1, 2, 4);
+  o.y = axis(q.y, 2, 1, 4);
+  o.z = axis(q.z, 4, 1, 2);
+  o.w = q.w;
+  for (int b = 1; b <= 4; b *= 2) o.w += __shfl_xor(o.w, b, 64);
+  o.w *= 0.125f;
+  if (valid && c == 0) cells[t] = o;
 }
 
 __global__ void __launch_bounds__(kBS) k_mg_cells(int fx, int fy, int fz, const float4* __restrict__ f, int cx, int cy,
@@ -290,169 +293,34 @@ __global__ void __launch_bounds__(kBS) k_mg_edges(MgGrid g, float h, const float
 }
 
 // ------------------------------------------------------------------ cycle
-__device__ __forceinline__ float nb_sum(const MgGrid& g, const float* v, int64_t o) {
-  const int64_t sy = g.pitch, sz = (int64_t)g.pitch * (g.cy + 1);
-  return g.ex[o] * v[o + 1] + g.ex[o - 1] * v[o - 1] + g.ey[o] * v[o + sy] + g.ey[o - sy] * v[o - sy] +
-         g.ez[o] * v[o + sz] + g.ez[o - sz] * v[o - sz];
-}
+// The levels' kernels: four nodes of a grid row per thread (mg_*_quad), one thread in a
+// flat index per quad.
 
-// residual after the first smoothing step x = omega b / d: t = b - A x
 __global__ void __launch_bounds__(kBS) k_mg_resid(MgGrid g, const KrylovScalars* ks) {
   if (ks->done) return;
-  const int i = blockIdx.x * 64 + (threadIdx.x & 63), j = blockIdx.y * 4 + (threadIdx.x >> 6), k = blockIdx.z;
-  if (!g.inner(i, j, k)) return;  // t stays 0 on the faces
-  const int64_t o = g.at(i, j, k);
-  g.t[o] = fmaf(1.f - kOmega, g.b[o], nb_sum(g, g.x, o));
+  mg_resid_quad(g, blockIdx.x * kBS + threadIdx.x);
 }
 
-// full weighting of t (fine grid, rows of `pitch`, `rows` rows per plane) around fine
-// node (2i, 2j, 2k); every index is inside the fine grid for interior coarse nodes
-__device__ __forceinline__ float weighted(const float* __restrict__ t, int64_t pitch, int64_t rows, int i, int j,
-                                          int k) {
-  float s = 0.f;
-#pragma unroll
-  for (int dk = -1; dk <= 1; ++dk) {
-#pragma unroll
-    for (int dj = -1; dj <= 1; ++dj) {
-      const float* r = t + ((int64_t)(2 * k + dk) * rows + 2 * j + dj) * pitch + 2 * i;
-      const float2 v = *reinterpret_cast<const float2*>(r);  // pitch is even
-      const float w = (dk ? 0.5f : 1.f) * (dj ? 0.5f : 1.f);
-      s = fmaf(w, fmaf(0.5f, r[-1] + v.y, v.x), s);
-    }
-  }
-  return s;
-}
-
-// b = R t + f, x = omega b / d
 __global__ void __launch_bounds__(kBS) k_mg_restrict(MgGrid g, const float* __restrict__ t, int pitch, int rows,
                                                      const KrylovScalars* ks) {
   if (ks->done) return;
-  const int i = blockIdx.x * 64 + (threadIdx.x & 63), j = blockIdx.y * 4 + (threadIdx.x >> 6), k = blockIdx.z;
-  if (!g.inner(i, j, k)) return;
-  const int64_t o = g.at(i, j, k);
-  float b = weighted(t, pitch, rows, i, j, k);
-  if (g.f) b += g.f[o];
-  g.b[o] = b;
-  g.x[o] = kOmega * g.dinv[o] * b;
-}
-
-// trilinear interpolation of coarse values e at fine position (i, j, k)
-template <class At>
-__device__ __forceinline__ float interpolate(int i, int j, int k, At&& e) {
-  const int I = i >> 1, J = j >> 1, K = k >> 1, a = i & 1, b = j & 1, c = k & 1;
-  auto ex = [&](int y, int z) { return a ? 0.5f * (e(I, y, z) + e(I + 1, y, z)) : e(I, y, z); };
-  auto ey = [&](int z) { return b ? 0.5f * (ex(J, z) + ex(J + 1, z)) : ex(J, z); };
-  return c ? 0.5f * (ey(K) + ey(K + 1)) : ey(K);
+  mg_restrict_pair(g, t, pitch, rows, blockIdx.x * kBS + threadIdx.x);
 }
 
 __global__ void __launch_bounds__(kBS) k_mg_prolong(MgGrid g, MgGrid c, const KrylovScalars* ks) {
   if (ks->done) return;
-  const int i = blockIdx.x * 64 + (threadIdx.x & 63), j = blockIdx.y * 4 + (threadIdx.x >> 6), k = blockIdx.z;
-  if (!g.inner(i, j, k)) return;
-  const int64_t o = g.at(i, j, k);
-  g.x[o] += interpolate(i, j, k, [&](int x, int y, int z) { return c.t[c.at(x, y, z)]; });
+  mg_prolong_quad(g, c, blockIdx.x * kBS + threadIdx.x);
 }
 
-// second smoothing step: t = x + omega (b - A x) / d
 __global__ void __launch_bounds__(kBS) k_mg_smooth(MgGrid g, const KrylovScalars* ks) {
   if (ks->done) return;
-  const int i = blockIdx.x * 64 + (threadIdx.x & 63), j = blockIdx.y * 4 + (threadIdx.x >> 6), k = blockIdx.z;
-  if (!g.inner(i, j, k)) return;
-  const int64_t o = g.at(i, j, k);
-  g.t[o] = fmaf(1.f - kOmega, g.x[o], kOmega * g.dinv[o] * (g.b[o] + nb_sum(g, g.x, o)));
+  mg_smooth_quad(g, blockIdx.x * kBS + threadIdx.x);
 }
 
-// The levels from `first` on, one cycle in one block: x and t of every level in LDS, b
-// in memory (a level's nodes belong to the same threads throughout). The last level has
-// one interior node (solved exactly) or, in a flat box, a few lines of them (16 steps).
-__global__ void __launch_bounds__(kBottomBS) k_mg_bottom(MgHierarchy h, int first, const KrylovScalars* ks) {
+__global__ void __launch_bounds__(kMgBottomBS) k_mg_bottom(MgHierarchy h, const KrylovScalars* ks) {
   extern __shared__ float s_mem[];
   if (ks->done) return;
-  float* xs[kMgLevels];
-  float* ts[kMgLevels];
-  {
-    float* p = s_mem;
-    for (int l = first; l < h.nlev; ++l) {
-      const int cnt = (int)h.lev[l].nodes();
-      xs[l] = p;
-      ts[l] = p + cnt;
-      p += 2 * cnt;
-    }
-    const int total = (int)(p - s_mem);
-    for (int q = threadIdx.x; q < total; q += kBottomBS) s_mem[q] = 0.f;
-  }
-  __syncthreads();
-  // visits the interior nodes of a level
-  auto each = [&](const MgGrid& g, auto&& fn) {
-    const int nx = g.cx - 1, ny = g.cy - 1, nz = g.cz - 1, cnt = nx * ny * nz;
-    for (int q = threadIdx.x; q < cnt; q += kBottomBS) {
-      const int i = q % nx + 1, j = q / nx % ny + 1, k = q / (nx * ny) + 1;
-      fn(i, j, k, (int)g.at(i, j, k));
-    }
-  };
-  {
-    const MgGrid& g = h.lev[first];
-    float* x = xs[first];
-    each(g, [&](int, int, int, int o) { x[o] = kOmega * g.dinv[o] * g.b[o]; });
-  }
-  __syncthreads();
-  for (int l = first; l + 1 < h.nlev; ++l) {
-    const MgGrid &g = h.lev[l], &c = h.lev[l + 1];
-    const float* x = xs[l];
-    float* t = ts[l];
-    each(g, [&](int, int, int, int o) { t[o] = fmaf(1.f - kOmega, g.b[o], nb_sum(g, x, o)); });
-    __syncthreads();
-    float* cxp = xs[l + 1];
-    const int rows = g.cy + 1, pitch = g.pitch;
-    each(c, [&](int i, int j, int k, int o) {
-      float b = weighted(t, pitch, rows, i, j, k);
-      if (c.f) b += c.f[o];
-      c.b[o] = b;
-      cxp[o] = kOmega * c.dinv[o] * b;
-    });
-    __syncthreads();
-  }
-  {
-    const int l = h.nlev - 1;
-    const MgGrid& g = h.lev[l];
-    float *x = xs[l], *t = ts[l];
-    if ((g.cx - 1) * (g.cy - 1) * (g.cz - 1) == 1) {
-      each(g, [&](int, int, int, int o) { t[o] = g.dinv[o] * g.b[o]; });
-      __syncthreads();
-    } else {
-      for (int it = 0; it < 8; ++it) {  // two steps each, x -> t -> x; the last leaves its result in t
-        each(g, [&](int, int, int, int o) {
-          t[o] = fmaf(1.f - kOmega, x[o], kOmega * g.dinv[o] * (g.b[o] + nb_sum(g, x, o)));
-        });
-        __syncthreads();
-        if (it == 7) break;
-        each(g, [&](int, int, int, int o) {
-          x[o] = fmaf(1.f - kOmega, t[o], kOmega * g.dinv[o] * (g.b[o] + nb_sum(g, t, o)));
-        });
-        __syncthreads();
-      }
-    }
-  }
-  for (int l = h.nlev - 2; l >= first; --l) {
-    const MgGrid &g = h.lev[l], &c = h.lev[l + 1];
-    float *x = xs[l], *t = ts[l];
-    const float* e = ts[l + 1];
-    each(g, [&](int i, int j, int k, int o) {
-      x[o] += interpolate(i, j, k, [&](int a, int b, int d) { return e[c.at(a, b, d)]; });
-    });
-    __syncthreads();
-    each(g, [&](int, int, int, int o) {
-      t[o] = fmaf(1.f - kOmega, x[o], kOmega * g.dinv[o] * (g.b[o] + nb_sum(g, x, o)));
-    });
-    __syncthreads();
-  }
-  // results that kernels outside read: the first level here, and levels with direct nodes
-  for (int l = first; l < h.nlev; ++l) {
-    const MgGrid& g = h.lev[l];
-    if (l != first && !g.f) continue;
-    const float* t = ts[l];
-    each(g, [&](int, int, int, int o) { g.t[o] = t[o]; });
-  }
+  mg_bottom(h, s_mem);
 }
 
 // ------------------------------------------------------------------ octree level
@@ -472,92 +340,94 @@ __global__ void __launch_bounds__(kBS) k_mgf_embed(MgHierarchy h, int64_t n, con
     if (blockIdx.x == 0 && threadIdx.x == 0) {
       ks->rr = RR;
       ks->iter = it;
-      if (stop) ks->done = 1;
+      if (stop) {
+        ks->done = 1;
+        ks->stop_par = par;
+      }
     }
     if (stop) return;
   }
-  for (int64_t q = (int64_t)blockIdx.x * kBS + threadIdx.x; q < n; q += (int64_t)gridDim.x * kBS) {
-    const float v = sd[q] * fmaf(-kOmega, ar[q], r[q]);
-    const uint32_t p = pos[q];
-    const int i = p & 1023, j = (p >> 10) & 1023, k = (p >> 20) & 1023, d = p >> 30;
-    if (d == 0) {
-      h.dense[((int64_t)k * h.drows + j) * h.dpitch + i] = v;
-    } else {
-      const MgGrid& g = h.lev[d];  // level d + 1
-      g.f[g.at(i >> (d + 1), j >> (d + 1), k >> (d + 1))] = v;
-    }
-  }
+  for (int64_t q = (int64_t)blockIdx.x * kBS + threadIdx.x; q < n; q += (int64_t)gridDim.x * kBS)
+    mg_embed(h, pos[q], sd[q] * fmaf(-kMgOmega, ar[q], r[q]));
 }
 
-// z0 = omega r + scaled coarse correction
+// rows a thread has in flight: a row's position leads to its coarse values, a chain of
+// two memory latencies (8M rows: 43 us with one row in flight, 38 with four)
+constexpr int kUnroll = 4;
+
+// z0 = omega r + scaled coarse correction; per block (z0, r - omega Ahat r), which with
+// omega (r, r) makes (r, z) of z = z0 + omega (r - Ahat z0): Ahat is symmetric
 __global__ void __launch_bounds__(kBS) k_mgf_correct(MgHierarchy h, int64_t n, const uint32_t* __restrict__ pos,
                                                      const float* __restrict__ sd, const float* __restrict__ r,
-                                                     float* __restrict__ z, const KrylovScalars* ks) {
-  if (ks->done) return;
-  for (int64_t q = (int64_t)blockIdx.x * kBS + threadIdx.x; q < n; q += (int64_t)gridDim.x * kBS) {
-    const uint32_t p = pos[q];
-    const int i = p & 1023, j = (p >> 10) & 1023, k = (p >> 20) & 1023, d = p >> 30;
-    float e = 0.f;
-    const float s = sd[q];
-    if (s != 0.f) {  // faces hold no correction (and may lie past the last coarse node's reach)
-      if (d == 0) {
-        const MgGrid& g = h.lev[0];
-        e = interpolate(i, j, k, [&](int x, int y, int zz) { return g.t[g.at(x, y, zz)]; });
-      } else {
-        const MgGrid& g = h.lev[d];
-        e = g.t[g.at(i >> (d + 1), j >> (d + 1), k >> (d + 1))];
-      }
-    }
-    z[q] = fmaf(s, e, kOmega * r[q]);
-  }
-}
-
-// z = z0 + omega (r - Ahat z0); per block (r, z)
-__global__ void __launch_bounds__(kBS) k_mgf_dot(int64_t n, const float* __restrict__ r, const float* __restrict__ az,
-                                                 float* __restrict__ z, const KrylovScalars* ks,
-                                                 double* __restrict__ part) {
+                                                     const float* __restrict__ ar, float* __restrict__ z,
+                                                     const KrylovScalars* ks, double* __restrict__ part) {
   __shared__ double s_red[kBS / 64];
   if (ks->done) return;
   double s = 0.0;
-  for (int64_t q = (int64_t)blockIdx.x * kBS + threadIdx.x; q < n; q += (int64_t)gridDim.x * kBS) {
-    const float ri = r[q];
-    const float zi = fmaf(kOmega, ri - az[q], z[q]);
-    z[q] = zi;
-    s += (double)ri * (double)zi;
+  const int64_t step = (int64_t)gridDim.x * kBS;
+  for (int64_t b = (int64_t)blockIdx.x * kBS; b < n; b += kUnroll * step) {
+    uint32_t p[kUnroll];
+    float ri[kUnroll], ai[kUnroll], si[kUnroll], e[kUnroll];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      const int64_t q = min(b + u * step + threadIdx.x, n - 1);
+      p[u] = pos[q];
+      ri[u] = r[q];
+      ai[u] = ar[q];
+      si[u] = sd[q];
+    }
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) e[u] = mg_correction(h, p[u], b + u * step + threadIdx.x < n);
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      const int64_t q = b + u * step + threadIdx.x;
+      if (q < n) {
+        const float zi = fmaf(si[u], e[u], kMgOmega * ri[u]);
+        z[q] = zi;
+        s += (double)zi * (double)fmaf(-kMgOmega, ai[u], ri[u]);
+      }
+    }
   }
   s = dev::block_sum<kBS>(s, s_red);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
+// xhat += alpha p of the previous iteration; z = z0 + omega (r - Ahat z0) and
 // p = z + beta p, beta = (r, z) / (r, z) of the previous iteration
-__global__ void __launch_bounds__(kBS) k_mgf_dir(int64_t n, const float* __restrict__ z, float* __restrict__ p,
-                                                 KrylovScalars* ks, const double* __restrict__ part, int np, int par) {
+__global__ void __launch_bounds__(kBS) k_mgf_dir(int64_t n, const float* __restrict__ z, const float* __restrict__ r,
+                                                 const float* __restrict__ az, float* __restrict__ p,
+                                                 float* __restrict__ x, KrylovScalars* ks,
+                                                 const double* __restrict__ part, int np, int par) {
   __shared__ double s_red[kBS / 64];
   if (ks->done) return;
-  const double rz = dev::sum_partials<kBS>(part, np, 1, s_red);
+  const double rz = dev::sum_partials<kBS>(part, np, 1, s_red) + (double)kMgOmega * ks->rr;
   const double old = ks->rho2[par];
   const float beta = old > 0.0 ? (float)(rz / old) : 0.f;
+  const float alpha = (float)ks->alpha2[par];
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     ks->rho2[par ^ 1] = rz;
     ks->iter2[par ^ 1] = ks->iter2[par] + 1;
   }
-  for (int64_t q = (int64_t)blockIdx.x * kBS + threadIdx.x; q < n; q += (int64_t)gridDim.x * kBS)
-    p[q] = fmaf(beta, p[q], z[q]);
+  for (int64_t q = (int64_t)blockIdx.x * kBS + threadIdx.x; q < n; q += (int64_t)gridDim.x * kBS) {
+    const float pi = p[q];
+    // xhat and Ahat z0 are not read again before everything else has passed the caches
+    __builtin_nontemporal_store(fmaf(alpha, pi, __builtin_nontemporal_load(&x[q])), &x[q]);
+    p[q] = fmaf(beta, pi, fmaf(kMgOmega, r[q] - __builtin_nontemporal_load(&az[q]), z[q]));
+  }
 }
 
-// alpha = (r, z) / (p, Ahat p); x += alpha p, r -= alpha Ahat p; per block (r, r)
-__global__ void __launch_bounds__(kBS) k_mgf_update(int64_t n, float* __restrict__ x, float* __restrict__ r,
-                                                    const float* __restrict__ p, const float* __restrict__ ap,
-                                                    const KrylovScalars* ks, const double* __restrict__ pq_part,
-                                                    int npq, double* __restrict__ part, int par) {
+// alpha = (r, z) / (p, Ahat p); r -= alpha Ahat p; per block (r, r)
+__global__ void __launch_bounds__(kBS) k_mgf_update(int64_t n, float* __restrict__ r, const float* __restrict__ ap,
+                                                    KrylovScalars* ks, const double* __restrict__ pq_part, int npq,
+                                                    double* __restrict__ part, int par) {
   __shared__ double s_red[kBS / 64];
   if (ks->done) return;
   const double pq = dev::sum_partials<kBS>(pq_part, npq, 1, s_red);
-  const float alpha = (float)(ks->rho2[par ^ 1] / pq);
+  const double a = ks->rho2[par ^ 1] / pq;
+  const float alpha = (float)a;
+  if (blockIdx.x == 0 && threadIdx.x == 0) ks->alpha2[par ^ 1] = a;
   double rr = 0.0;
   for (int64_t q = (int64_t)blockIdx.x * kBS + threadIdx.x; q < n; q += (int64_t)gridDim.x * kBS) {
-    // x and Ahat p are not read again before everything else has passed the caches
-    __builtin_nontemporal_store(fmaf(alpha, p[q], __builtin_nontemporal_load(&x[q])), &x[q]);
     const float ri = fmaf(-alpha, __builtin_nontemporal_load(&ap[q]), r[q]);
     r[q] = ri;
     rr += (double)ri * (double)ri;
@@ -568,12 +438,6 @@ __global__ void __launch_bounds__(kBS) k_mgf_update(int64_t n, float* __restrict
 
 dim3 grid_of(const MgGrid& g) {
   return dim3((unsigned)((g.pitch + 63) / 64), (unsigned)((g.cy + 4) / 4), (unsigned)(g.cz + 1));
-}
-
-int64_t lds_bytes_from(const MgHierarchy& h, int first) {
-  int64_t n = 0;
-  for (int l = first; l < h.nlev; ++l) n += h.lev[l].nodes();
-  return n * 2 * (int64_t)sizeof(float);
 }
 
 }  // namespace
@@ -688,8 +552,8 @@ bool mg_setup(ngpb_ctx* c) {
     const int64_t nc = (int64_t)l.cx * l.cy * l.cz;
     ca.resize((size_t)nc);
     cb.resize((size_t)(nc / 8 + 2 * (int64_t)(l.cx + 2) * (l.cy + 2) + 2 * (int64_t)(l.cz + 2) * (l.cx + l.cy + 4)));
-    hipLaunchKernelGGL(k_mg_cells1, dim3(blocks_for(nc, kBS)), dim3(kBS), 0, st, m, g, l.cx, l.cy, l.cz, map, level.p,
-                       c->c_edge.p, c->v8.p, c->reac.p, ca.p, bad.p);
+    hipLaunchKernelGGL(k_mg_cells1, dim3(blocks_for(8 * nc, kBS)), dim3(kBS), 0, st, m, g, l.cx, l.cy, l.cz, map, level.p,
+                       c->c_edge.p, c->reac.p, ca.p, bad.p);
   }
   if (is_bad()) return false;
   NGPB_HIP(hipMemsetAsync(c->mg_dense.p, 0, (size_t)dense * 4, st));
@@ -708,21 +572,18 @@ bool mg_setup(ngpb_ctx* c) {
   }
   NGPB_HIP(hipGetLastError());
   // the bottom kernel takes the levels that fit one block
-  H.bottom = H.nlev - 1;
-  while (H.bottom > 0 && H.lev[H.bottom - 1].nodes() <= kMgBottomNodes &&
-         lds_bytes_from(H, H.bottom - 1) <= kMgBottomLds)
-    --H.bottom;
-  if (lds_bytes_from(H, H.bottom) > kMgBottomLds) return false;
+  H.bottom = mg_bottom_level(H);
+  if (H.bottom < 0) return false;
   NGPB_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mg_bottom), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)kMgBottomLds));
+                               kMgBottomLds));
   NGPB_HIP(hipStreamSynchronize(st));
   c->mg_state = 1;
   return true;
 }
 
 // ------------------------------------------------------------------ launches
-void mg_precondition(ngpb_ctx* c, const float* r, const float* ar, float* z, const double* rr_part, int npr, int par,
-                     bool first) {
+void mg_precondition(ngpb_ctx* c, const float* r, const float* ar, float* z, const double* rr_part, int npr,
+                     double* rz_part, int par, bool first) {
   const MgHierarchy& H = c->mg;
   const int64_t n = c->n;
   const unsigned gv = vec_grid(n);
@@ -732,33 +593,34 @@ void mg_precondition(ngpb_ctx* c, const float* r, const float* ar, float* z, con
                      par, first ? 1 : 0);
   for (int l = 0; l <= H.bottom; ++l) {
     const MgGrid& q = H.lev[l];
+    const dim3 gp(blocks_for(mg_pairs(q), kBS));
     if (l == 0)
-      hipLaunchKernelGGL(k_mg_restrict, grid_of(q), dim3(kBS), 0, st, q, H.dense, H.dpitch, H.drows, ks);
+      hipLaunchKernelGGL(k_mg_restrict, gp, dim3(kBS), 0, st, q, H.dense, H.dpitch, H.drows, ks);
     else
-      hipLaunchKernelGGL(k_mg_restrict, grid_of(q), dim3(kBS), 0, st, q, H.lev[l - 1].t, H.lev[l - 1].pitch,
+      hipLaunchKernelGGL(k_mg_restrict, gp, dim3(kBS), 0, st, q, H.lev[l - 1].t, H.lev[l - 1].pitch,
                          H.lev[l - 1].cy + 1, ks);
-    if (l < H.bottom) hipLaunchKernelGGL(k_mg_resid, grid_of(q), dim3(kBS), 0, st, q, ks);
+    if (l < H.bottom) hipLaunchKernelGGL(k_mg_resid, dim3(blocks_for(mg_quads(q), kBS)), dim3(kBS), 0, st, q, ks);
   }
-  hipLaunchKernelGGL(k_mg_bottom, dim3(1), dim3(kBottomBS), (unsigned)lds_bytes_from(H, H.bottom), st, H, H.bottom, ks);
+  hipLaunchKernelGGL(k_mg_bottom, dim3(1), dim3(kMgBottomBS), (unsigned)mg_bottom_lds(H, H.bottom), st, H, ks);
   for (int l = H.bottom - 1; l >= 0; --l) {
-    hipLaunchKernelGGL(k_mg_prolong, grid_of(H.lev[l]), dim3(kBS), 0, st, H.lev[l], H.lev[l + 1], ks);
-    hipLaunchKernelGGL(k_mg_smooth, grid_of(H.lev[l]), dim3(kBS), 0, st, H.lev[l], ks);
+    const dim3 gq(blocks_for(mg_quads(H.lev[l]), kBS));
+    hipLaunchKernelGGL(k_mg_prolong, gq, dim3(kBS), 0, st, H.lev[l], H.lev[l + 1], ks);
+    hipLaunchKernelGGL(k_mg_smooth, gq, dim3(kBS), 0, st, H.lev[l], ks);
   }
-  hipLaunchKernelGGL(k_mgf_correct, dim3(gv), dim3(kBS), 0, st, H, n, c->mg_pos.p, c->mg_sd.p, r, z, ks);
+  hipLaunchKernelGGL(k_mgf_correct, dim3(gv), dim3(kBS), 0, st, H, n, c->mg_pos.p, c->mg_sd.p, r, ar, z, ks, rz_part);
 }
 
-void mg_direction(ngpb_ctx* c, const float* r, const float* az, float* z, float* p, double* part, int par) {
+void mg_direction(ngpb_ctx* c, const float* r, const float* az, const float* z, float* p, float* x,
+                  const double* rz_part, int par) {
   const int64_t n = c->n;
   const unsigned gv = vec_grid(n);
-  hipLaunchKernelGGL(k_mgf_dot, dim3(gv), dim3(kBS), 0, c->stream, n, r, az, z, c->ks.p, part);
-  hipLaunchKernelGGL(k_mgf_dir, dim3(gv), dim3(kBS), 0, c->stream, n, z, p, c->ks.p, part, (int)gv, par);
+  hipLaunchKernelGGL(k_mgf_dir, dim3(gv), dim3(kBS), 0, c->stream, n, z, r, az, p, x, c->ks.p, rz_part, (int)gv, par);
 }
 
-void mg_update(ngpb_ctx* c, float* x, float* r, const float* p, const float* ap, const double* pq_part, int npq,
-               double* part, int par) {
+void mg_update(ngpb_ctx* c, float* r, const float* ap, const double* pq_part, int npq, double* part, int par) {
   const int64_t n = c->n;
-  hipLaunchKernelGGL(k_mgf_update, dim3(vec_grid(n)), dim3(kBS), 0, c->stream, n, x, r, p, ap, c->ks.p, pq_part, npq,
-                     part, par);
+  hipLaunchKernelGGL(k_mgf_update, dim3(vec_grid(n)), dim3(kBS), 0, c->stream, n, r, ap, c->ks.p, pq_part, npq, part,
+                     par);
 }
 
 }  // namespace ngpb

@@ -1502,7 +1502,7 @@ void solve_mixed(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
       h->done = 0;
       h->rho2[launch & 1] = mg ? mg_rho : h->rho;
       h->iter2[launch & 1] = iters;
-      if (mg) {  // xhat is complete when the flag is raised: k_mx_accum adds nothing to it
+      if (mg) {  // the cycle's first direction kernel has no step to add to xhat
         h->alpha2[0] = h->alpha2[1] = 0.0;
         h->stop_par = 0;
       }
@@ -1515,15 +1515,15 @@ void solve_mixed(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
           const int par = (int)(launch & 1);
           if (mg) {
             launch_sell(c, true, rv, c->qs.p, pun);
-            mg_precondition(c, rv, c->qs.p, zv, pup, (int)gv, par, launch == cycle_start);
+            mg_precondition(c, rv, c->qs.p, zv, pup, (int)gv, prz, par, launch == cycle_start);
             launch_sell(c, true, zv, c->qs.p, pun);
-            mg_direction(c, rv, c->qs.p, zv, pv, prz, par);
+            mg_direction(c, rv, c->qs.p, zv, pv, c->xs.p, prz, par);
           }
           prof_begin(c, 1, launch);
           launch_sell(c, true, pv, c->qs.p, ppq);
           prof_end(c, 1);
           if (mg) {
-            mg_update(c, c->xs.p, rv, pv, c->qs.p, ppq, (int)gs, pup, par);
+            mg_update(c, rv, c->qs.p, ppq, (int)gs, pup, par);
             continue;
           }
           hipLaunchKernelGGL(k_mx_update, dim3(gv), dim3(kBS), 0, c->stream, n, rv, c->qs.p, ks, ppq, (int)gs, pup, par);
@@ -1594,10 +1594,10 @@ void solve_mixed(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
   st.relres = bb > 0 ? std::sqrt(true_rr / bb) : 0.0;
   st.ms_solve = ms;
   // SpMV + update (rhat, q read; rhat written) + direction (rhat, p, xhat read; p, xhat
-  // written); with the preconditioner three SpMVs, the vector streams of its five row
-  // kernels (25 x 4 bytes) and the uniform levels (the dense array twice, then some 100
+  // written); with the preconditioner three SpMVs, the vector streams of its four row
+  // kernels (20 x 4 bytes) and the uniform levels (the dense array twice, then some 100
   // bytes per node of the first level and an eighth of that for each further one)
-  st.bytes_per_iter = mg ? 3.0 * spmv_compact_bytes(c) + (double)n * 100.0 + 4.0 * (double)c->mg_dense.n +
+  st.bytes_per_iter = mg ? 3.0 * spmv_compact_bytes(c) + (double)n * 80.0 + 4.0 * (double)c->mg_dense.n +
                                115.0 * (double)c->mg.lev[0].nodes()
                          : spmv_compact_bytes(c) + (double)n * 4.0 * (3.0 + 5.0);
   c->have_phi = true;
