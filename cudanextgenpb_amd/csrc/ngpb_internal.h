@@ -477,6 +477,7 @@ double time_spmv_fp64(ngpb_ctx* c, int reps);
 // mixed
 void build_compact(ngpb_ctx* c, bool allow_band = true);  // allow_band: banded row order may apply
 float* spmv_input(ngpb_ctx* c);  // FP32 SpMV input vector (zero guard entries either side)
+float* guarded_vector(ngpb_ctx* c, DBuf<float>& v);  // n entries between such guards
 void spmv_compact(ngpb_ctx* c, const double* x, double* y);
 void solve_mixed(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st);
 double spmv_compact_bytes(const ngpb_ctx* c);
