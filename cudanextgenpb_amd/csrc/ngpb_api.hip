@@ -89,7 +89,7 @@ int64_t ngpb_ctx::device_bytes() const {
   b += lis_rt.bytes() + lis_u.bytes() + lis_v.bytes() + lis_ph.bytes() + lis_uh.bytes() + lis_t.bytes() +
        diag_pos.bytes() + ssor_f.bytes() + ssor_b.bytes();
   b += xs.bytes() + rs.bytes() + ps.bytes() + qs.bytes() + ks.bytes();
-  b += mg_pool.bytes() + mg_dense.bytes() + mg_sd.bytes() + mg_r.bytes() + mg_z.bytes() + mg_pos.bytes();
+  b += mg_pool.bytes() + mg_dense.bytes() + mg_sd.bytes() + mg_r.bytes() + mg_z.bytes() + mg_pos.bytes() + slice_rec.bytes();
   b += red.partials.bytes() + scan_tmp.bytes();
   for (const auto& t : tmp) b += t.bytes();
   return b;

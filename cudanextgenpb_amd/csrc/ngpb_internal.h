@@ -327,6 +327,7 @@ struct ngpb_ctx {
   int sell_band = 0;  // band of the built operator when sell_banded
   ngpb::DBuf<int32_t> row_perm;
   ngpb::DBuf<int64_t> sell_pk_hdr_list;
+  ngpb::DBuf<uint8_t> slice_rec;     // FP64 solves: diagonals of each 64-row slice
   ngpb::DBuf<double> dscale;         // 1/sqrt(diag)
   // multigrid preconditioner of the mixed solve, built with the compact operator
   int mg_state = 0;  // 0 not built, 1 in use, -1 does not apply to this operator
@@ -457,7 +458,9 @@ void check_operator(ngpb_ctx* c);
 void ensure_reduce(ngpb_ctx* c, int64_t blocks);
 // FP64 CSR SpMV y = A x that also writes per-block (x, y) partials and returns at once
 // once the stop flag of c->ks is raised; grid size of its launches
-void spmv_fp64_dot(ngpb_ctx* c, const double* x, double* y, double* partials);
+// FP64 CSR products by per-slice diagonals: the system's records, built anew on each call
+const void* slice_records(ngpb_ctx* c);
+void spmv_fp64_dot(ngpb_ctx* c, const double* x, double* y, double* partials, const void* rec);
 unsigned spmv_fp64_grid(ngpb_ctx* c);
 void check_operator(ngpb_ctx* c);
 // other LIS solvers (ngpb_lis.hip)

@@ -37,16 +37,12 @@ constexpr int kFin = 1024;  // finalize block size
 // range of chunks, with blocks renumbered so that the blocks on one XCD (block id
 // mod 8) cover one contiguous eighth of the rows (L2 reuse of the x gathers); the
 // grid is then the number of blocks resident at once.
-template <bool DOT, int SCHED>
+template <int SCHED>
 __global__ void __launch_bounds__(kBS) k_spmv64(int64_t n, const int32_t* __restrict__ rowptr,
                                                  const int32_t* __restrict__ col, const double* __restrict__ val,
-                                                 const double* __restrict__ x, double* __restrict__ y,
-                                                 const KrylovScalars* ks, double* __restrict__ partials) {
+                                                 const double* __restrict__ x, double* __restrict__ y) {
   __shared__ double s_val[kCap];
   __shared__ double s_x[kCap];
-  __shared__ double s_red[kBS / 64];
-  if (DOT && ks->done) return;
-  double part = 0.0;
   const int64_t nchunks = (n + kBS - 1) / kBS;
   int64_t c_begin = blockIdx.x, c_end = nchunks, c_step = gridDim.x;
   if (SCHED == 1) {
@@ -93,12 +89,165 @@ __global__ void __launch_bounds__(kBS) k_spmv64(int64_t n, const int32_t* __rest
       for (int64_t k = kb; k < ke; ++k) sum = fma(s_val[k - p0], s_x[k - p0], sum);
     }
     if (row < n) y[row] = sum;
-    if (DOT && row < n) part += x[row] * sum;
   }
-  if (DOT) {
-    part = dev::block_sum<kBS>(part, s_red);
-    if (threadIdx.x == 0) partials[blockIdx.x] = part;
+}
+
+// ---- slice records
+// Most rows of a mesh operator belong to 64-row slices whose entries lie on a few
+// diagonals (column - row), with the same value along a diagonal wherever the medium is
+// uniform. A record lists a slice's diagonals in ascending order, which rows have an
+// entry there and, unless it varies, the value: the product then reads 288 bytes of
+// record and contiguous runs of x instead of 12 bytes per entry. Values that vary are
+// read from the CSR, and slices with more diagonals are staged as in k_spmv64. Every row
+// still sums its entries in column order, so the results are the same bit for bit.
+constexpr int kDiags = 14;
+struct SliceRec {
+  int32_t count;  // diagonals, -1: more than kDiags
+  uint32_t vary;  // bit k: diagonal k's values differ
+  int32_t delta[kDiags];
+  uint64_t rows[kDiags];  // bit per row
+  double val[kDiags];
+};
+static_assert(sizeof(SliceRec) == 288, "SliceRec is 288 bytes");
+
+// one wave per slice
+__global__ void __launch_bounds__(kBS) k_slice_rec(int64_t n, const int32_t* __restrict__ rowptr,
+                                                   const int32_t* __restrict__ col, const double* __restrict__ val,
+                                                   SliceRec* __restrict__ recs) {
+  const int64_t s = (int64_t)blockIdx.x * (kBS / 64) + (threadIdx.x >> 6);
+  if (s * 64 >= n) return;
+  const int lane = threadIdx.x & 63;
+  const int64_t row = s * 64 + lane;
+  int64_t e = 0, end = 0;
+  if (row < n) {
+    e = rowptr[row];
+    end = rowptr[row + 1];
   }
+  SliceRec& R = recs[s];
+  int k = 0;
+  uint32_t vary = 0;
+  while (true) {
+    int d = e < end ? (int)((int64_t)col[e] - row) : INT32_MAX;
+    int m = d;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) m = min(m, __shfl_xor(m, off, 64));
+    if (m == INT32_MAX) break;
+    if (k == kDiags) {
+      k = -1;
+      break;
+    }
+    const bool has = d == m;
+    const uint64_t rows = __ballot(has);
+    const double v = has ? val[e] : 0.0;
+    const long long bits = __double_as_longlong(v);
+    const long long first = __shfl(bits, __ffsll((unsigned long long)rows) - 1, 64);
+    if (__ballot(has && bits != first)) vary |= 1u << k;
+    if (lane == 0) {
+      R.delta[k] = m;
+      R.rows[k] = rows;
+      R.val[k] = __longlong_as_double(first);
+    }
+    if (has) ++e;
+    ++k;
+  }
+  if (lane == 0) {
+    R.count = k;
+    R.vary = vary;
+  }
+}
+
+// k_spmv64 from slice records: the same rows per thread and the same partial sums.
+// Diagonals are taken kGo at a time, their loads in flight together.
+template <int SCHED>
+__global__ void __launch_bounds__(kBS) k_spmv64_rec(int64_t n, const int32_t* __restrict__ rowptr,
+                                                     const int32_t* __restrict__ col, const double* __restrict__ val,
+                                                     const SliceRec* __restrict__ recs, const double* __restrict__ x,
+                                                     double* __restrict__ y, const KrylovScalars* ks,
+                                                     double* __restrict__ partials) {
+  constexpr int kWaveCap = 256, kGo = 7;
+  __shared__ double s_val[kBS / 64 * kWaveCap];
+  __shared__ double s_x[kBS / 64 * kWaveCap];
+  __shared__ double s_red[kBS / 64];
+  if (ks->done) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double part = 0.0;
+  const int64_t nchunks = (n + kBS - 1) / kBS;
+  int64_t c_begin = blockIdx.x, c_end = nchunks, c_step = gridDim.x;
+  if (SCHED == 1) {
+    const unsigned nb = gridDim.x, b = blockIdx.x;
+    const int64_t lb = (nb % 8u == 0u) ? (int64_t)((b % 8u) * (nb / 8u) + b / 8u) : (int64_t)b;
+    c_begin = lb * nchunks / nb;
+    c_end = (lb + 1) * nchunks / nb;
+    c_step = 1;
+  }
+  for (int64_t chunk = c_begin; chunk < c_end; chunk += c_step) {
+    const int64_t s = __builtin_amdgcn_readfirstlane((int)(chunk * (kBS / 64) + wave));
+    if (s * 64 >= n) continue;
+    const int64_t row = s * 64 + lane;
+    const SliceRec& R = recs[s];
+    const int count = R.count;
+    double sum = 0.0;
+    if (count >= 0) {
+      const uint32_t vary = R.vary;
+      int64_t e = vary && row < n ? (int64_t)rowptr[row] : 0;  // the row's next entry
+      const int64_t safe = min(row, n - 1);
+      for (int k0 = 0; k0 < count; k0 += kGo) {
+        double xv[kGo], v[kGo];
+        bool has[kGo];
+#pragma unroll
+        for (int u = 0; u < kGo; ++u) {
+          const int k = min(k0 + u, kDiags - 1);
+          const bool in = k0 + u < count;
+          has[u] = in && ((R.rows[k] >> lane) & 1);
+          xv[u] = x[has[u] ? row + R.delta[k] : safe];
+          v[u] = R.val[k];
+          if (in && ((vary >> k) & 1)) {
+            if (has[u]) v[u] = val[e];
+          }
+          if (has[u]) ++e;
+        }
+#pragma unroll
+        for (int u = 0; u < kGo; ++u)
+          if (has[u]) sum = fma(v[u], xv[u], sum);
+      }
+    } else {
+      // a slice of its own shape: its entries staged in the wave's part of the LDS
+      const int64_t last = min(s * 64 + 63, n - 1);
+      const int64_t e0 = rowptr[s * 64], e1 = rowptr[last + 1];
+      const int64_t rb = row < n ? (int64_t)rowptr[row] : e1, re = row < n ? (int64_t)rowptr[row + 1] : e1;
+      double* wv = s_val + wave * kWaveCap;
+      double* wx = s_x + wave * kWaveCap;
+      for (int64_t p0 = e0; p0 < e1; p0 += kWaveCap) {
+        const int64_t p1 = min(p0 + (int64_t)kWaveCap, e1);
+        constexpr int kU = kWaveCap / 64;
+        double v[kU];
+        int c[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+          const int64_t k = min(p0 + lane + u * 64, p1 - 1);
+          v[u] = __builtin_nontemporal_load(&val[k]);
+          c[u] = __builtin_nontemporal_load(&col[k]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();  // the previous piece has been read
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+          wv[lane + u * 64] = v[u];
+          wx[lane + u * 64] = x[c[u]];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const int64_t kb = max(rb, p0), ke = min(re, p1);
+        for (int64_t k = kb; k < ke; ++k) sum = fma(wv[k - p0], wx[k - p0], sum);
+      }
+    }
+    if (row < n) {
+      y[row] = sum;
+      part += x[row] * sum;
+    }
+  }
+  part = dev::block_sum<kBS>(part, s_red);
+  if (threadIdx.x == 0) partials[blockIdx.x] = part;
 }
 
 unsigned spmv64_grid(ngpb_ctx* c) {
@@ -107,20 +256,20 @@ unsigned spmv64_grid(ngpb_ctx* c) {
   if (c->csr_resident <= 0) {
     int cus = 0, per_cu = 0;
     NGPB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
-    NGPB_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_spmv64<true, 1>, kBS, 0));
+    NGPB_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_spmv64_rec<1>, kBS, 0));
     c->csr_resident = std::max(8, (std::max(cus, 1) * std::max(per_cu, 1)) / 8 * 8);
   }
   if (need >= c->csr_resident) return (unsigned)c->csr_resident;
   return (unsigned)(c->spmv_sched == 1 ? (need + 7) / 8 * 8 : need);
 }
 
-template <bool DOT>
-void launch_spmv64(ngpb_ctx* c, unsigned grid, const double* x, double* y, double* part) {
-  const KrylovScalars* ks = DOT ? c->ks.p : nullptr;
+// y = A x from the slice records, with the (x, y) partials
+void launch_spmv64_rec(ngpb_ctx* c, unsigned grid, const double* x, double* y, double* part, const void* rec) {
+  const SliceRec* R = static_cast<const SliceRec*>(rec);
   if (c->spmv_sched == 1)
-    spmv_launch(c, k_spmv64<DOT, 1>, dim3(grid), dim3(kBS), c->n, c->rowptr.p, c->col.p, c->val.p, x, y, ks, part);
+    spmv_launch(c, k_spmv64_rec<1>, dim3(grid), dim3(kBS), c->n, c->rowptr.p, c->col.p, c->val.p, R, x, y, c->ks.p, part);
   else
-    spmv_launch(c, k_spmv64<DOT, 0>, dim3(grid), dim3(kBS), c->n, c->rowptr.p, c->col.p, c->val.p, x, y, ks, part);
+    spmv_launch(c, k_spmv64_rec<0>, dim3(grid), dim3(kBS), c->n, c->rowptr.p, c->col.p, c->val.p, R, x, y, c->ks.p, part);
 }
 
 // x = 0, r = b, p = D^-1 b; per block (r, D^-1 r), (b, b)
@@ -166,9 +315,8 @@ __global__ void __launch_bounds__(kFin) k_fin_init(KrylovScalars* ks, const doub
 
 // Iteration of parity par. Every block forms (p, q) from the SpMV partials in the
 // same fixed order, so all blocks use the same alpha = rho / (p, q).
-// x += alpha p; r -= alpha q; per block (r, D^-1 r), (r, r)
-__global__ void __launch_bounds__(kBS) k_pcg_update(int64_t n, const double* __restrict__ dinv, double* __restrict__ x,
-                                                    double* __restrict__ r, const double* __restrict__ p,
+// r -= alpha q; per block (r, D^-1 r), (r, r)
+__global__ void __launch_bounds__(kBS) k_pcg_update(int64_t n, const double* __restrict__ dinv, double* __restrict__ r,
                                                     const double* __restrict__ q, KrylovScalars* ks,
                                                     const double* __restrict__ pq_part, int npq,
                                                     double* __restrict__ partials, int par) {
@@ -182,7 +330,6 @@ __global__ void __launch_bounds__(kBS) k_pcg_update(int64_t n, const double* __r
   }
   double rz = 0.0, rr = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * kBS + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBS) {
-    x[i] += alpha * p[i];
     const double ri = r[i] - alpha * q[i];
     r[i] = ri;
     rz += ri * (dinv[i] * ri);
@@ -196,10 +343,11 @@ __global__ void __launch_bounds__(kBS) k_pcg_update(int64_t n, const double* __r
   }
 }
 
-// Stop test on ||r||^2 (every block decides alike), then beta = (r', z') / (r, z) and
-// p = D^-1 r + beta p. Block 0 records the scalars for the next iteration and the host.
-__global__ void __launch_bounds__(kBS) k_pcg_dir(int64_t n, const double* __restrict__ dinv, const double* __restrict__ r,
-                                                 double* __restrict__ p, KrylovScalars* ks,
+// x += alpha p (here, where p is read for its own update too), the stop test on ||r||^2
+// (every block decides alike), then beta = (r', z') / (r, z) and p = D^-1 r + beta p.
+// Block 0 records the scalars for the next iteration and the host.
+__global__ void __launch_bounds__(kBS) k_pcg_dir(int64_t n, const double* __restrict__ dinv, double* __restrict__ x,
+                                                 const double* __restrict__ r, double* __restrict__ p, KrylovScalars* ks,
                                                  const double* __restrict__ part, int np, int par) {
   __shared__ double s_red[kBS / 64];
   if (ks->done) return;
@@ -223,10 +371,12 @@ __global__ void __launch_bounds__(kBS) k_pcg_dir(int64_t n, const double* __rest
       ks->rho2[par ^ 1] = RZ;
     }
   }
-  if (stop) return;
-  const double beta = RZ / rho;
-  for (int64_t i = (int64_t)blockIdx.x * kBS + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBS)
-    p[i] = dinv[i] * r[i] + beta * p[i];
+  const double alpha = ks->alpha2[par], beta = RZ / rho;
+  for (int64_t i = (int64_t)blockIdx.x * kBS + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBS) {
+    const double pi = p[i];
+    x[i] += alpha * pi;
+    if (!stop) p[i] = dinv[i] * r[i] + beta * pi;
+  }
 }
 
 __global__ void k_diag_inv(int64_t n, const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
@@ -339,8 +489,18 @@ void ensure_reduce(ngpb_ctx* c, int64_t blocks) {
   if (!c->ks_host) NGPB_HIP(hipHostMalloc((void**)&c->ks_host, sizeof(KrylovScalars), hipHostMallocDefault));
 }
 
-void spmv_fp64_dot(ngpb_ctx* c, const double* x, double* y, double* partials) {
-  launch_spmv64<true>(c, spmv64_grid(c), x, y, partials);
+const void* slice_records(ngpb_ctx* c) {
+  const int64_t ns = (c->n + 63) / 64;
+  c->slice_rec.reserve((size_t)ns * sizeof(SliceRec));
+  SliceRec* R = reinterpret_cast<SliceRec*>(c->slice_rec.p);
+  hipLaunchKernelGGL(k_slice_rec, dim3(blocks_for(ns, kBS / 64)), dim3(kBS), 0, c->stream, c->n, c->rowptr.p, c->col.p,
+                     c->val.p, R);
+  NGPB_HIP(hipGetLastError());
+  return R;
+}
+
+void spmv_fp64_dot(ngpb_ctx* c, const double* x, double* y, double* partials, const void* rec) {
+  launch_spmv64_rec(c, spmv64_grid(c), x, y, partials, rec);
 }
 
 unsigned spmv_fp64_grid(ngpb_ctx* c) { return spmv64_grid(c); }
@@ -351,7 +511,11 @@ double spmv_fp64_bytes(const ngpb_ctx* c) {
 }
 
 void spmv_fp64(ngpb_ctx* c, const double* x, double* y) {
-  launch_spmv64<false>(c, spmv64_grid(c), x, y, nullptr);
+  const unsigned grid = spmv64_grid(c);
+  if (c->spmv_sched == 1)
+    spmv_launch(c, k_spmv64<1>, dim3(grid), dim3(kBS), c->n, c->rowptr.p, c->col.p, c->val.p, x, y);
+  else
+    spmv_launch(c, k_spmv64<0>, dim3(grid), dim3(kBS), c->n, c->rowptr.p, c->col.p, c->val.p, x, y);
   NGPB_HIP(hipGetLastError());
 }
 
@@ -404,6 +568,7 @@ void solve_fp64(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
   NGPB_HIP(hipEventCreate(&e0));
   NGPB_HIP(hipEventCreate(&e1));
   NGPB_HIP(hipEventRecord(e0, c->stream));
+  const void* rec = slice_records(c);
   hipLaunchKernelGGL(k_pcg_init, dim3(gv), dim3(kBS), 0, c->stream, n, c->rhs.p, c->dinv.p, c->x.p, c->r.p, c->p.p, part);
   hipLaunchKernelGGL(k_fin_init, dim3(1), dim3(kFin), 0, c->stream, ks, part, (int)gv, o.tol * o.tol, o.maxiter);
   NGPB_HIP(hipGetLastError());
@@ -416,12 +581,11 @@ void solve_fp64(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
     for (int k = 0; k < chunk; ++k, ++launch) {
       const int par = (int)(launch & 1);
       prof_begin(c, 0, launch);
-      launch_spmv64<true>(c, gs, c->p.p, c->q.p, ppq);
+      launch_spmv64_rec(c, gs, c->p.p, c->q.p, ppq, rec);
       prof_end(c, 0);
-      hipLaunchKernelGGL(k_pcg_update, dim3(gv), dim3(kBS), 0, c->stream, n, c->dinv.p, c->x.p, c->r.p, c->p.p, c->q.p,
-                         ks, ppq, (int)gs, pup, par);
-      hipLaunchKernelGGL(k_pcg_dir, dim3(gv), dim3(kBS), 0, c->stream, n, c->dinv.p, c->r.p, c->p.p, ks, pup, (int)gv,
-                         par);
+      hipLaunchKernelGGL(k_pcg_update, dim3(gv), dim3(kBS), 0, c->stream, n, c->dinv.p, c->r.p, c->q.p, ks, ppq, (int)gs, pup, par);
+      hipLaunchKernelGGL(k_pcg_dir, dim3(gv), dim3(kBS), 0, c->stream, n, c->dinv.p, c->x.p, c->r.p, c->p.p, ks, pup,
+                         (int)gv, par);
     }
     NGPB_HIP(hipGetLastError());
     NGPB_HIP(hipMemcpyAsync(c->ks_host, ks, sizeof(KrylovScalars), hipMemcpyDeviceToHost, c->stream));
@@ -441,15 +605,15 @@ void solve_fp64(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
   st.replacements = 0;
   st.relres = h.bb > 0 ? std::sqrt(h.rr / h.bb) : 0.0;
   st.ms_solve = ms;
-  // SpMV + update (x, p, r, q, dinv read; x, r written) + direction (dinv, r, p read; p written)
-  st.bytes_per_iter = spmv_fp64_bytes(c) + (double)n * 8.0 * (7.0 + 4.0);
+  // SpMV in CSR form + update (r, q, dinv read; r written) + direction (x, dinv, r, p read; x, p written)
+  st.bytes_per_iter = spmv_fp64_bytes(c) + (double)n * 8.0 * (4.0 + 6.0);
   c->have_phi = true;
   c->phi_len = c->n;
 }
 
 // ------------------------------------------------------------ allocation-free entry point
 // ngpb_solve_csr_noalloc runs the CG-Jacobi above on a CSR system the caller keeps in
-// device memory, with its work vectors, partial sums, scalars and flags in one
+// device memory, with its work vectors, partial sums, scalars, flags and slice records in one
 // file-scope device array: the call allocates nothing (no hipMalloc / hipFree, no
 // pinned host memory, no events), for callers that cannot allocate. Each GPU holds
 // its own copy of the array until the process ends; its address on a device is taken
@@ -458,7 +622,8 @@ void solve_fp64(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
 // (from several host threads or streams) race; each call initializes what it reads.
 constexpr int64_t kNoAllocMaxRows = int64_t(1) << 20;  // 1,048,576 rows
 constexpr int64_t kNoAllocPartials = 8192;             // >= 2048 + 2 * 2048
-constexpr int64_t kNoAllocDoubles = 4 * kNoAllocMaxRows + kNoAllocPartials + 64;
+constexpr int64_t kNoAllocRecs = (kNoAllocMaxRows / 64) * (int64_t)(sizeof(SliceRec) / 8);  // in doubles
+constexpr int64_t kNoAllocDoubles = 4 * kNoAllocMaxRows + kNoAllocPartials + 64 + kNoAllocRecs;
 static __device__ __align__(256) double scratch[kNoAllocDoubles];
 
 namespace {
@@ -516,6 +681,7 @@ void solve_csr_noalloc(int device, hipStream_t s, int64_t n, int64_t nnz, const 
   double* part = base + 4 * kNoAllocMaxRows;
   KrylovScalars* ks = reinterpret_cast<KrylovScalars*>(part + kNoAllocPartials);
   int* bad = reinterpret_cast<int*>(ks + 1);
+  SliceRec* recs = reinterpret_cast<SliceRec*>(part + kNoAllocPartials + 64);
   static_assert(sizeof(KrylovScalars) + sizeof(int) <= 64 * sizeof(double), "scalar area too small");
   const auto t0 = std::chrono::steady_clock::now();
   hipLaunchKernelGGL(k_clear_int, dim3(1), dim3(1), 0, s, bad);
@@ -536,6 +702,7 @@ void solve_csr_noalloc(int device, hipStream_t s, int64_t n, int64_t nnz, const 
   const unsigned gv = vec_grid(n);
   double* ppq = part;
   double* pup = part + 2048;
+  hipLaunchKernelGGL(k_slice_rec, dim3(blocks_for((n + 63) / 64, kBS / 64)), dim3(kBS), 0, s, n, rowptr, col, val, recs);
   hipLaunchKernelGGL(k_pcg_init, dim3(gv), dim3(kBS), 0, s, n, b, dinv, x, r, p, pup);
   hipLaunchKernelGGL(k_fin_init, dim3(1), dim3(kFin), 0, s, ks, pup, (int)gv, tol * tol, maxiter);
   NGPB_HIP(hipGetLastError());
@@ -545,9 +712,9 @@ void solve_csr_noalloc(int device, hipStream_t s, int64_t n, int64_t nnz, const 
   for (int64_t launch = 0;;) {
     for (int k = 0; k < chunk; ++k, ++launch) {
       const int par = (int)(launch & 1);
-      hipLaunchKernelGGL((k_spmv64<true, 0>), dim3(gs), dim3(kBS), 0, s, n, rowptr, col, val, p, q, ks, ppq);
-      hipLaunchKernelGGL(k_pcg_update, dim3(gv), dim3(kBS), 0, s, n, dinv, x, r, p, q, ks, ppq, (int)gs, pup, par);
-      hipLaunchKernelGGL(k_pcg_dir, dim3(gv), dim3(kBS), 0, s, n, dinv, r, p, ks, pup, (int)gv, par);
+      hipLaunchKernelGGL(k_spmv64_rec<0>, dim3(gs), dim3(kBS), 0, s, n, rowptr, col, val, recs, p, q, ks, ppq);
+      hipLaunchKernelGGL(k_pcg_update, dim3(gv), dim3(kBS), 0, s, n, dinv, r, q, ks, ppq, (int)gs, pup, par);
+      hipLaunchKernelGGL(k_pcg_dir, dim3(gv), dim3(kBS), 0, s, n, dinv, x, r, p, ks, pup, (int)gv, par);
     }
     NGPB_HIP(hipGetLastError());
     NGPB_HIP(hipMemcpyAsync(&h, ks, sizeof(KrylovScalars), hipMemcpyDeviceToHost, s));
@@ -560,7 +727,7 @@ void solve_csr_noalloc(int device, hipStream_t s, int64_t n, int64_t nnz, const 
   st.relres = h.bb > 0 ? std::sqrt(h.rr / h.bb) : 0.0;
   st.ms_solve = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   // SpMV (12 nnz + 4 (n + 1) + 16 n) + update and direction vector streams, as ngpb_solve
-  st.bytes_per_iter = 12.0 * (double)nnz + 4.0 * (double)(n + 1) + 16.0 * (double)n + (double)n * 8.0 * (7.0 + 4.0);
+  st.bytes_per_iter = 12.0 * (double)nnz + 4.0 * (double)(n + 1) + 16.0 * (double)n + (double)n * 8.0 * (4.0 + 6.0);
 }
 
 }  // namespace ngpb

@@ -756,6 +756,7 @@ void solve_lis(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
   NGPB_HIP(hipEventCreate(&e0));
   NGPB_HIP(hipEventCreate(&e1));
   NGPB_HIP(hipEventRecord(e0, c->stream));
+  const void* rec = slice_records(c);
   hipLaunchKernelGGL(k_lis_init, G, B, 0, c->stream, n, c->rhs.p, x, r, rt, p, q, v, dpart);
   hipLaunchKernelGGL(k_lis_fin_init, F, BF, 0, c->stream, ks, dpart, np, o.tol * o.tol, o.maxiter);
   if (o.solver == NGPB_SOLVER_CG) {
@@ -769,7 +770,7 @@ void solve_lis(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
   while (true) {
     for (int k = 0; k < chunk; ++k) {
       if (o.solver == NGPB_SOLVER_CG) {
-        spmv_fp64_dot(c, p, q, spart);  // q = A p with (p, q) partials
+        spmv_fp64_dot(c, p, q, spart, rec);  // q = A p with (p, q) partials
         fin(spart, nsp, 1, kFinAlpha);
         hipLaunchKernelGGL(k_xr_update, G, B, 0, c->stream, n, x, p, r, q, ks, dpart);
         fin(dpart, np, 2, kFinResid);
@@ -782,12 +783,12 @@ void solve_lis(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
         fin(dpart, np, 2, kFinRho);
         hipLaunchKernelGGL(k_cgs_up, G, B, 0, c->stream, n, r, q, u, p, ks);
         const double* pp = psolve(c, o.precon, w, p, ph);
-        spmv_fp64_dot(c, pp, v, spart);
+        spmv_fp64_dot(c, pp, v, spart, rec);
         hipLaunchKernelGGL(k_dots<false>, G, B, 0, c->stream, n, rt, v, nullptr, nullptr, ks, dpart);
         fin(dpart, np, 2, kFinAlpha);
         hipLaunchKernelGGL(k_cgs_q, G, B, 0, c->stream, n, u, v, q, t, ks);
         const double* uu = psolve(c, o.precon, w, t, uh);
-        spmv_fp64_dot(c, uu, ph, spart);  // A uh into ph, free once v = A ph was formed
+        spmv_fp64_dot(c, uu, ph, spart, rec);  // A uh into ph, free once v = A ph was formed
         hipLaunchKernelGGL(k_xr_update, G, B, 0, c->stream, n, x, uu, r, ph, ks, dpart);
         fin(dpart, np, 2, kFinResid);
       } else {  // BiCGSTAB; s lives in u, its preconditioned copy in uh
@@ -795,13 +796,13 @@ void solve_lis(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
         fin(dpart, np, 2, kFinRho);
         hipLaunchKernelGGL(k_bicg_p, G, B, 0, c->stream, n, r, v, p, ks);
         const double* pp = psolve(c, o.precon, w, p, ph);
-        spmv_fp64_dot(c, pp, v, spart);
+        spmv_fp64_dot(c, pp, v, spart, rec);
         hipLaunchKernelGGL(k_dots<false>, G, B, 0, c->stream, n, rt, v, nullptr, nullptr, ks, dpart);
         fin(dpart, np, 2, kFinAlpha);
         hipLaunchKernelGGL(k_bicg_s, G, B, 0, c->stream, n, r, v, u, ks, dpart);
         fin(dpart, np, 2, kFinBicgS);
         const double* ss = psolve(c, o.precon, w, u, uh);
-        spmv_fp64_dot(c, ss, t, spart);
+        spmv_fp64_dot(c, ss, t, spart, rec);
         hipLaunchKernelGGL(k_dots<true>, G, B, 0, c->stream, n, t, u, t, t, ks, dpart);
         fin(dpart, np, 2, kFinOmega);
         hipLaunchKernelGGL(k_bicg_x, G, B, 0, c->stream, n, x, pp, ss, r, u, t, ks, dpart);
