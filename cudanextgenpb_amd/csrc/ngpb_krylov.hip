@@ -156,19 +156,23 @@ __global__ void __launch_bounds__(kBS) k_slice_rec(int64_t n, const int32_t* __r
   }
 }
 
-// k_spmv64 from slice records: the same rows per thread and the same partial sums.
-// Diagonals are taken kGo at a time, their loads in flight together.
+// k_spmv64 from slice records: the same rows per thread and the same partial sums. A
+// record is read one word per lane, the next slice's while this one is worked on, and
+// its fields are broadcast from there; kGo diagonals' loads of x are in flight together.
+// Bound by the latency of record, x and store at one or two slices per wave. 1 million
+// rows of a uniform grid: 26 us from the CSR, 12.4 with each field a scalar load when it
+// is needed, 11.1 so; 2.1 million rows: 50, 24.2, 22.0 us.
 template <int SCHED>
 __global__ void __launch_bounds__(kBS) k_spmv64_rec(int64_t n, const int32_t* __restrict__ rowptr,
                                                      const int32_t* __restrict__ col, const double* __restrict__ val,
                                                      const SliceRec* __restrict__ recs, const double* __restrict__ x,
                                                      double* __restrict__ y, const KrylovScalars* ks,
                                                      double* __restrict__ partials) {
-  constexpr int kWaveCap = 256, kGo = 7;
-  __shared__ double s_val[kBS / 64 * kWaveCap];
-  __shared__ double s_x[kBS / 64 * kWaveCap];
-  __shared__ double s_red[kBS / 64];
-  if (ks->done) return;
+  constexpr int kWaveCap = 256, kGo = 7, kSW = kBS / 64;
+  constexpr int kRows = 2 + kDiags, kVal = kRows + 2 * kDiags;  // words before the fields
+  __shared__ double s_val[kSW * kWaveCap];
+  __shared__ double s_x[kSW * kWaveCap];
+  __shared__ double s_red[kSW];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   double part = 0.0;
   const int64_t nchunks = (n + kBS - 1) / kBS;
@@ -180,31 +184,50 @@ __global__ void __launch_bounds__(kBS) k_spmv64_rec(int64_t n, const int32_t* __
     c_end = (lb + 1) * nchunks / nb;
     c_step = 1;
   }
+  const int64_t nslices = (n + 63) / 64;
+  const int32_t* const words = reinterpret_cast<const int32_t*>(recs);
+  // words l and 64 + l of a record (72 in all; lanes 8.. repeat the last)
+  auto word_at = [&](int64_t chunk, int w) {
+    const int64_t s = min(min(chunk, nchunks - 1) * kSW + wave, nslices - 1);
+    return words[s * 72 + min(w, 71)];
+  };
+  int n0 = word_at(c_begin, lane), n1 = word_at(c_begin, 64 + lane);
+  if (ks->done) return;
   for (int64_t chunk = c_begin; chunk < c_end; chunk += c_step) {
-    const int64_t s = __builtin_amdgcn_readfirstlane((int)(chunk * (kBS / 64) + wave));
-    if (s * 64 >= n) continue;
+    const int w0 = n0, w1 = n1;
+    n0 = word_at(chunk + c_step, lane);
+    n1 = word_at(chunk + c_step, 64 + lane);
+    const int64_t s = __builtin_amdgcn_readfirstlane((int)(chunk * kSW + wave));
+    if (s >= nslices) continue;
     const int64_t row = s * 64 + lane;
-    const SliceRec& R = recs[s];
-    const int count = R.count;
+    auto word = [&](int k) {
+      return (uint32_t)(k < 64 ? __builtin_amdgcn_readlane(w0, k) : __builtin_amdgcn_readlane(w1, k - 64));
+    };
+    auto pair = [&](int k) { return (uint64_t)word(k) | (uint64_t)word(k + 1) << 32; };
+    const int count = (int)word(0);
     double sum = 0.0;
     if (count >= 0) {
-      const uint32_t vary = R.vary;
+      const uint32_t vary = word(1);
       int64_t e = vary && row < n ? (int64_t)rowptr[row] : 0;  // the row's next entry
       const int64_t safe = min(row, n - 1);
-      for (int k0 = 0; k0 < count; k0 += kGo) {
+#pragma unroll
+      for (int k0 = 0; k0 < kDiags; k0 += kGo) {
+        if (k0 >= count) break;
         double xv[kGo], v[kGo];
         bool has[kGo];
 #pragma unroll
         for (int u = 0; u < kGo; ++u) {
-          const int k = min(k0 + u, kDiags - 1);
-          const bool in = k0 + u < count;
-          has[u] = in && ((R.rows[k] >> lane) & 1);
-          xv[u] = x[has[u] ? row + R.delta[k] : safe];
-          v[u] = R.val[k];
-          if (in && ((vary >> k) & 1)) {
-            if (has[u]) v[u] = val[e];
+          const int k = k0 + u;
+          has[u] = k < count && ((pair(kRows + 2 * k) >> lane) & 1);
+          xv[u] = x[has[u] ? row + (int)word(2 + k) : safe];
+          v[u] = __longlong_as_double((long long)pair(kVal + 2 * k));
+        }
+        if (vary) {
+#pragma unroll
+          for (int u = 0; u < kGo; ++u) {
+            if (has[u] && ((vary >> (k0 + u)) & 1)) v[u] = val[e];
+            if (has[u]) ++e;
           }
-          if (has[u]) ++e;
         }
 #pragma unroll
         for (int u = 0; u < kGo; ++u)
