@@ -458,8 +458,9 @@ void check_operator(ngpb_ctx* c);
 void ensure_reduce(ngpb_ctx* c, int64_t blocks);
 // FP64 CSR SpMV y = A x that also writes per-block (x, y) partials and returns at once
 // once the stop flag of c->ks is raised; grid size of its launches
-// FP64 CSR products by per-slice diagonals: the system's records, built anew on each call
-const void* slice_records(ngpb_ctx* c);
+// FP64 CSR products by per-slice diagonals: check_operator, and the system's records,
+// built anew on each call; *block: the system suits the one-block CG
+const void* slice_records(ngpb_ctx* c, bool* block);
 void spmv_fp64_dot(ngpb_ctx* c, const double* x, double* y, double* partials, const void* rec);
 unsigned spmv_fp64_grid(ngpb_ctx* c);
 void check_operator(ngpb_ctx* c);

@@ -101,6 +101,10 @@ __global__ void __launch_bounds__(kBS) k_spmv64(int64_t n, const int32_t* __rest
 // read from the CSR, and slices with more diagonals are staged as in k_spmv64. Every row
 // still sums its entries in column order, so the results are the same bit for bit.
 constexpr int kDiags = 14;
+// Most rows of k_pcg_block. Whole solves of uniform grids: 4,096 rows 1,340 us with three
+// launches per iteration, 822 in one block; 512 rows 863 and 239; 8,000 rows 1,774 and
+// 1,708 (8 rows per thread, which spill), so the line lies at 4 rows per thread.
+constexpr int kBlockRows = 4096;
 struct SliceRec {
   int32_t count;  // diagonals, -1: more than kDiags
   uint32_t vary;  // bit k: diagonal k's values differ
@@ -110,10 +114,11 @@ struct SliceRec {
 };
 static_assert(sizeof(SliceRec) == 288, "SliceRec is 288 bytes");
 
-// one wave per slice
+// one wave per slice; at up to kBlockRows rows bit 8 of *flags is set when a slice has
+// more than kDiags diagonals
 __global__ void __launch_bounds__(kBS) k_slice_rec(int64_t n, const int32_t* __restrict__ rowptr,
                                                    const int32_t* __restrict__ col, const double* __restrict__ val,
-                                                   SliceRec* __restrict__ recs) {
+                                                   SliceRec* __restrict__ recs, int* __restrict__ flags) {
   const int64_t s = (int64_t)blockIdx.x * (kBS / 64) + (threadIdx.x >> 6);
   if (s * 64 >= n) return;
   const int lane = threadIdx.x & 63;
@@ -153,6 +158,7 @@ __global__ void __launch_bounds__(kBS) k_slice_rec(int64_t n, const int32_t* __r
   if (lane == 0) {
     R.count = k;
     R.vary = vary;
+    if (k < 0 && n <= kBlockRows) atomicOr(flags, 8);
   }
 }
 
@@ -271,6 +277,179 @@ __global__ void __launch_bounds__(kBS) k_spmv64_rec(int64_t n, const int32_t* __
   }
   part = dev::block_sum<kBS>(part, s_red);
   if (threadIdx.x == 0) partials[blockIdx.x] = part;
+}
+
+// ---- small systems: the whole CG in one block
+// An iteration of three launches takes 11 us however few the rows: their latency. For at
+// most kBlockRows rows, in slices that all have a record (own entry lists would be read
+// from memory in every iteration: a 5,559-row octree operator took 3.7 ms for 1.8), one
+// block keeps p and A p in LDS and r and 1 / diag of its R rows per thread in registers,
+// and takes up to `steps` iterations per launch with three barriers each: 2.3 us per
+// iteration at 512 rows, 6.3 at 4,096, where reading varying values is most of it.
+constexpr int kBlk = 1024;
+
+// sums of a and b over the block, in every thread; slot alternates between calls
+__device__ __forceinline__ double2 blk_sum2(double a, double b, double2* slot) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    a += __shfl_xor(a, off, 64);
+    b += __shfl_xor(b, off, 64);
+  }
+  if ((threadIdx.x & 63) == 0) slot[threadIdx.x >> 6] = make_double2(a, b);
+  __syncthreads();
+  double2 t = make_double2(0.0, 0.0);
+#pragma unroll
+  for (int w = 0; w < kBlk / 64; ++w) {
+    t.x += slot[w].x;
+    t.y += slot[w].y;
+  }
+  return t;
+}
+
+template <int R>
+__global__ void __launch_bounds__(kBlk) k_pcg_block(int n, const int32_t* __restrict__ rowptr, const double* __restrict__ val,
+                                                     const SliceRec* __restrict__ recs, const double* __restrict__ dinv,
+                                                     const double* __restrict__ b, double* __restrict__ x,
+                                                     double* __restrict__ r, double* __restrict__ p, KrylovScalars* ks,
+                                                     double tol2, int maxiter, int first, int steps) {
+  constexpr int kGo = 7;
+  __shared__ double s_p[R * kBlk], s_q[R * kBlk];
+  __shared__ int s_e[R * kBlk];
+  __shared__ double2 s_red[2][kBlk / 64];
+  const int t = threadIdx.x, lane = t & 63;
+  double xr[R], rr[R], di[R];
+  double rho, stop_rr, RR = 0.0;
+  int it = 0, done = 0, status = 0;
+#pragma unroll
+  for (int j = 0; j < R; ++j) s_e[j * kBlk + t] = j * kBlk + t < n ? rowptr[j * kBlk + t] : 0;
+  if (first) {
+    double rz = 0.0, bb = 0.0;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const int row = j * kBlk + t;
+      const double bi = row < n ? b[row] : 0.0;
+      di[j] = row < n ? dinv[row] : 0.0;
+      const double zi = di[j] * bi;
+      xr[j] = 0.0;
+      rr[j] = bi;
+      s_p[row] = zi;
+      rz += bi * zi;
+      bb += bi * bi;
+    }
+    const double2 S = blk_sum2(rz, bb, s_red[1]);
+    rho = S.x;
+    RR = S.y;
+    stop_rr = tol2 * S.y;
+    done = S.y == 0.0;
+    if (t == 0) {
+      ks->bb = S.y;
+      ks->stop_rr = stop_rr;
+    }
+  } else {
+    if (ks->done) return;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const int row = j * kBlk + t;
+      xr[j] = row < n ? x[row] : 0.0;
+      rr[j] = row < n ? r[row] : 0.0;
+      di[j] = row < n ? dinv[row] : 0.0;
+      s_p[row] = row < n ? p[row] : 0.0;
+    }
+    rho = ks->rho;
+    stop_rr = ks->stop_rr;
+    it = ks->iter;
+    __syncthreads();
+  }
+  for (int k = 0; k < steps && !done; ++k) {
+    double pq = 0.0;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const int s = __builtin_amdgcn_readfirstlane(j * (kBlk / 64) + (t >> 6));
+      const int row = j * kBlk + t;
+      if (s * 64 >= n) break;
+      const SliceRec& S = recs[s];
+      double sum = 0.0;
+      const uint32_t vary = S.vary;
+      int e = s_e[row];  // the row's next entry
+#pragma unroll
+      for (int k0 = 0; k0 < kDiags; k0 += kGo) {
+        if (k0 >= S.count) break;
+        double pv[kGo], v[kGo];
+        bool has[kGo];
+#pragma unroll
+        for (int u = 0; u < kGo; ++u) {
+          has[u] = k0 + u < S.count && ((S.rows[k0 + u] >> lane) & 1);
+          pv[u] = s_p[has[u] ? row + S.delta[k0 + u] : row];
+          v[u] = S.val[k0 + u];
+        }
+        if (vary) {
+#pragma unroll
+          for (int u = 0; u < kGo; ++u) {
+            if (has[u] && ((vary >> (k0 + u)) & 1)) v[u] = val[e];
+            if (has[u]) ++e;
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < kGo; ++u)
+          if (has[u]) sum = fma(v[u], pv[u], sum);
+      }
+      s_q[row] = sum;
+      pq += s_p[row] * sum;  // rows past n: p and sum are 0
+    }
+    const double alpha = rho / blk_sum2(pq, 0.0, s_red[0]).x;
+    double rz = 0.0, r2 = 0.0;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      if ((j * kBlk + (t & ~63)) >= n) break;
+      xr[j] += alpha * s_p[j * kBlk + t];
+      rr[j] -= alpha * s_q[j * kBlk + t];
+      rz += rr[j] * (di[j] * rr[j]);
+      r2 += rr[j] * rr[j];
+    }
+    const double2 S = blk_sum2(rz, r2, s_red[1]);
+    RR = S.y;
+    ++it;
+    const bool conv = RR <= stop_rr;
+    if (conv || it >= maxiter) {
+      done = 1;
+      status = conv ? 0 : NGPB_E_NOCONV;
+      break;
+    }
+    const double beta = S.x / rho;
+    rho = S.x;
+#pragma unroll
+    for (int j = 0; j < R; ++j) s_p[j * kBlk + t] = di[j] * rr[j] + beta * s_p[j * kBlk + t];
+    __syncthreads();
+  }
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const int row = j * kBlk + t;
+    if (row < n) {
+      x[row] = xr[j];
+      r[row] = rr[j];
+      p[row] = s_p[row];
+    }
+  }
+  if (t == 0) {
+    ks->rho = rho;
+    ks->rr = RR;
+    ks->iter = it;
+    ks->done = done;
+    ks->status = status;
+  }
+}
+
+// runs a system to its end; poll copies *ks to the host and says whether it is done
+template <typename Poll>
+void run_pcg_block(hipStream_t s, int64_t n, const int32_t* rowptr, const double* val, const SliceRec* recs,
+                   const double* dinv, const double* b, double* x, double* r, double* p, KrylovScalars* ks, double tol, int maxiter, Poll poll) {
+  const auto k = n <= kBlk ? k_pcg_block<1> : n <= 2 * kBlk ? k_pcg_block<2> : k_pcg_block<4>;
+  for (int first = 1;; first = 0) {
+    hipLaunchKernelGGL(k, dim3(1), dim3(kBlk), 0, s, (int)n, rowptr, val, recs, dinv, b, x, r, p, ks, tol * tol,
+                       maxiter, first, 1024);
+    NGPB_HIP(hipGetLastError());
+    if (poll()) return;
+  }
 }
 
 unsigned spmv64_grid(ngpb_ctx* c) {
@@ -512,15 +691,30 @@ void ensure_reduce(ngpb_ctx* c, int64_t blocks) {
   if (!c->ks_host) NGPB_HIP(hipHostMalloc((void**)&c->ks_host, sizeof(KrylovScalars), hipHostMallocDefault));
 }
 
-const void* slice_records(ngpb_ctx* c) {
-  const int64_t ns = (c->n + 63) / 64;
-  c->slice_rec.reserve((size_t)ns * sizeof(SliceRec));
-  SliceRec* R = reinterpret_cast<SliceRec*>(c->slice_rec.p);
-  hipLaunchKernelGGL(k_slice_rec, dim3(blocks_for(ns, kBS / 64)), dim3(kBS), 0, c->stream, c->n, c->rowptr.p, c->col.p,
-                     c->val.p, R);
+namespace {
+// 1 / diagonal, its checks and, if asked for, the slice records; returns the flags
+int check_operator_records(ngpb_ctx* c, bool records) {
+  c->dinv.resize((size_t)c->n);
+  DBuf<int> bad;
+  bad.resize(1);
+  NGPB_HIP(hipMemsetAsync(bad.p, 0, sizeof(int), c->stream));
+  hipLaunchKernelGGL(k_diag_inv, dim3(blocks_for(c->n, 256)), dim3(256), 0, c->stream, c->n, c->rowptr.p, c->col.p,
+                     c->val.p, c->dinv.p, bad.p);
+  if (records) {
+    const int64_t ns = (c->n + 63) / 64;
+    c->slice_rec.reserve((size_t)ns * sizeof(SliceRec));
+    hipLaunchKernelGGL(k_slice_rec, dim3(blocks_for(ns, kBS / 64)), dim3(kBS), 0, c->stream, c->n, c->rowptr.p,
+                       c->col.p, c->val.p, reinterpret_cast<SliceRec*>(c->slice_rec.p), bad.p);
+  }
   NGPB_HIP(hipGetLastError());
-  return R;
+  int hb = 0;
+  NGPB_HIP(hipMemcpyAsync(&hb, bad.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  NGPB_HIP(hipStreamSynchronize(c->stream));
+  NGPB_REQUIRE(!(hb & 2), NGPB_E_NUMERIC, "operator holds NaN or Inf entries");
+  NGPB_REQUIRE(!(hb & 1), NGPB_E_NUMERIC, "operator has a zero or negative diagonal entry");
+  return hb;
 }
+}  // namespace
 
 void spmv_fp64_dot(ngpb_ctx* c, const double* x, double* y, double* partials, const void* rec) {
   launch_spmv64_rec(c, spmv64_grid(c), x, y, partials, rec);
@@ -561,24 +755,18 @@ double time_spmv_fp64(ngpb_ctx* c, int reps) {
   return (double)ms / std::max(reps, 1);
 }
 
-void check_operator(ngpb_ctx* c) {
-  c->dinv.resize((size_t)c->n);
-  DBuf<int> bad;
-  bad.resize(1);
-  NGPB_HIP(hipMemsetAsync(bad.p, 0, sizeof(int), c->stream));
-  hipLaunchKernelGGL(k_diag_inv, dim3(blocks_for(c->n, 256)), dim3(256), 0, c->stream, c->n, c->rowptr.p, c->col.p,
-                     c->val.p, c->dinv.p, bad.p);
-  NGPB_HIP(hipGetLastError());
-  int hb = 0;
-  NGPB_HIP(hipMemcpyAsync(&hb, bad.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  NGPB_HIP(hipStreamSynchronize(c->stream));
-  NGPB_REQUIRE(!(hb & 2), NGPB_E_NUMERIC, "operator holds NaN or Inf entries");
-  NGPB_REQUIRE(!(hb & 1), NGPB_E_NUMERIC, "operator has a zero or negative diagonal entry");
+void check_operator(ngpb_ctx* c) { (void)check_operator_records(c, false); }
+
+const void* slice_records(ngpb_ctx* c, bool* block) {
+  const int flags = check_operator_records(c, true);
+  if (block) *block = c->n <= kBlockRows && !(flags & 8);
+  return c->slice_rec.p;
 }
 
 void solve_fp64(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
   const int64_t n = c->n;
-  check_operator(c);
+  bool block = false;
+  const void* rec = slice_records(c, &block);
   c->x.resize((size_t)n);
   c->r.resize((size_t)n);
   c->p.reserve((size_t)n);
@@ -591,30 +779,37 @@ void solve_fp64(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
   NGPB_HIP(hipEventCreate(&e0));
   NGPB_HIP(hipEventCreate(&e1));
   NGPB_HIP(hipEventRecord(e0, c->stream));
-  const void* rec = slice_records(c);
-  hipLaunchKernelGGL(k_pcg_init, dim3(gv), dim3(kBS), 0, c->stream, n, c->rhs.p, c->dinv.p, c->x.p, c->r.p, c->p.p, part);
-  hipLaunchKernelGGL(k_fin_init, dim3(1), dim3(kFin), 0, c->stream, ks, part, (int)gv, o.tol * o.tol, o.maxiter);
-  NGPB_HIP(hipGetLastError());
-  // partial-sum regions: SpMV (p, q) and update (r, z), (r, r)
-  double* ppq = part;
-  double* pup = part + std::max<int64_t>(gs, 2048);
-  const int chunk = std::max(1, o.check_every);
-  int64_t launch = 0;
-  while (true) {
-    for (int k = 0; k < chunk; ++k, ++launch) {
-      const int par = (int)(launch & 1);
-      prof_begin(c, 0, launch);
-      launch_spmv64_rec(c, gs, c->p.p, c->q.p, ppq, rec);
-      prof_end(c, 0);
-      hipLaunchKernelGGL(k_pcg_update, dim3(gv), dim3(kBS), 0, c->stream, n, c->dinv.p, c->r.p, c->q.p, ks, ppq, (int)gs, pup, par);
-      hipLaunchKernelGGL(k_pcg_dir, dim3(gv), dim3(kBS), 0, c->stream, n, c->dinv.p, c->x.p, c->r.p, c->p.p, ks, pup,
-                         (int)gv, par);
-    }
-    NGPB_HIP(hipGetLastError());
+  const auto poll = [&]() {
     NGPB_HIP(hipMemcpyAsync(c->ks_host, ks, sizeof(KrylovScalars), hipMemcpyDeviceToHost, c->stream));
     NGPB_HIP(hipStreamSynchronize(c->stream));
-    prof_collect(c, 0, c->ks_host->iter);
-    if (c->ks_host->done) break;
+    return c->ks_host->done != 0;
+  };
+  if (block && !c->profile) {  // profiling times the products of the general path
+    run_pcg_block(c->stream, n, c->rowptr.p, c->val.p, static_cast<const SliceRec*>(rec), c->dinv.p, c->rhs.p,
+                  c->x.p, c->r.p, c->p.p, ks, o.tol, o.maxiter, poll);
+  } else {
+    hipLaunchKernelGGL(k_pcg_init, dim3(gv), dim3(kBS), 0, c->stream, n, c->rhs.p, c->dinv.p, c->x.p, c->r.p, c->p.p, part);
+    hipLaunchKernelGGL(k_fin_init, dim3(1), dim3(kFin), 0, c->stream, ks, part, (int)gv, o.tol * o.tol, o.maxiter);
+    NGPB_HIP(hipGetLastError());
+    // partial-sum regions: SpMV (p, q) and update (r, z), (r, r)
+    double* ppq = part;
+    double* pup = part + std::max<int64_t>(gs, 2048);
+    const int chunk = std::max(1, o.check_every);
+    for (int64_t launch = 0;;) {
+      for (int k = 0; k < chunk; ++k, ++launch) {
+        const int par = (int)(launch & 1);
+        prof_begin(c, 0, launch);
+        launch_spmv64_rec(c, gs, c->p.p, c->q.p, ppq, rec);
+        prof_end(c, 0);
+        hipLaunchKernelGGL(k_pcg_update, dim3(gv), dim3(kBS), 0, c->stream, n, c->dinv.p, c->r.p, c->q.p, ks, ppq, (int)gs, pup, par);
+        hipLaunchKernelGGL(k_pcg_dir, dim3(gv), dim3(kBS), 0, c->stream, n, c->dinv.p, c->x.p, c->r.p, c->p.p, ks, pup,
+                           (int)gv, par);
+      }
+      NGPB_HIP(hipGetLastError());
+      const bool done = poll();
+      prof_collect(c, 0, c->ks_host->iter);
+      if (done) break;
+    }
   }
   NGPB_HIP(hipEventRecord(e1, c->stream));
   NGPB_HIP(hipEventSynchronize(e1));
@@ -715,34 +910,42 @@ void solve_csr_noalloc(int device, hipStream_t s, int64_t n, int64_t nnz, const 
   NGPB_HIP(hipStreamSynchronize(s));
   NGPB_REQUIRE(!(hb & 4), NGPB_E_ARG, "row pointers must run from 0 to nnz without decreasing, columns in [0, n)");
   hipLaunchKernelGGL(k_diag_inv, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, rowptr, col, val, dinv, bad);
+  hipLaunchKernelGGL(k_slice_rec, dim3(blocks_for((n + 63) / 64, kBS / 64)), dim3(kBS), 0, s, n, rowptr, col, val, recs,
+                     bad);
   NGPB_HIP(hipGetLastError());
   NGPB_HIP(hipMemcpyAsync(&hb, bad, sizeof(int), hipMemcpyDeviceToHost, s));
   NGPB_HIP(hipStreamSynchronize(s));
   NGPB_REQUIRE(!(hb & 2), NGPB_E_NUMERIC, "operator holds NaN or Inf entries");
   NGPB_REQUIRE(!(hb & 1), NGPB_E_NUMERIC, "operator has a zero or negative diagonal entry");
-  // the launch shapes of ngpb_solve under SpMV schedule 0
-  const unsigned gs = (unsigned)std::min<int64_t>(std::max<int64_t>(1, (n + kBS - 1) / kBS), 2048);
-  const unsigned gv = vec_grid(n);
-  double* ppq = part;
-  double* pup = part + 2048;
-  hipLaunchKernelGGL(k_slice_rec, dim3(blocks_for((n + 63) / 64, kBS / 64)), dim3(kBS), 0, s, n, rowptr, col, val, recs);
-  hipLaunchKernelGGL(k_pcg_init, dim3(gv), dim3(kBS), 0, s, n, b, dinv, x, r, p, pup);
-  hipLaunchKernelGGL(k_fin_init, dim3(1), dim3(kFin), 0, s, ks, pup, (int)gv, tol * tol, maxiter);
-  NGPB_HIP(hipGetLastError());
-  const int chunk = std::max(1, check_every);
   KrylovScalars h;
   std::memset(&h, 0, sizeof(h));
-  for (int64_t launch = 0;;) {
-    for (int k = 0; k < chunk; ++k, ++launch) {
-      const int par = (int)(launch & 1);
-      hipLaunchKernelGGL(k_spmv64_rec<0>, dim3(gs), dim3(kBS), 0, s, n, rowptr, col, val, recs, p, q, ks, ppq);
-      hipLaunchKernelGGL(k_pcg_update, dim3(gv), dim3(kBS), 0, s, n, dinv, r, q, ks, ppq, (int)gs, pup, par);
-      hipLaunchKernelGGL(k_pcg_dir, dim3(gv), dim3(kBS), 0, s, n, dinv, x, r, p, ks, pup, (int)gv, par);
-    }
-    NGPB_HIP(hipGetLastError());
+  const auto poll = [&]() {
     NGPB_HIP(hipMemcpyAsync(&h, ks, sizeof(KrylovScalars), hipMemcpyDeviceToHost, s));
     NGPB_HIP(hipStreamSynchronize(s));
-    if (h.done) break;
+    return h.done != 0;
+  };
+  if (n <= kBlockRows && !(hb & 8)) {
+    run_pcg_block(s, n, rowptr, val, recs, dinv, b, x, r, p, ks, tol, maxiter, poll);
+  } else {
+    // the launch shapes of ngpb_solve under SpMV schedule 0
+    const unsigned gs = (unsigned)std::min<int64_t>(std::max<int64_t>(1, (n + kBS - 1) / kBS), 2048);
+    const unsigned gv = vec_grid(n);
+    double* ppq = part;
+    double* pup = part + 2048;
+    hipLaunchKernelGGL(k_pcg_init, dim3(gv), dim3(kBS), 0, s, n, b, dinv, x, r, p, pup);
+    hipLaunchKernelGGL(k_fin_init, dim3(1), dim3(kFin), 0, s, ks, pup, (int)gv, tol * tol, maxiter);
+    NGPB_HIP(hipGetLastError());
+    const int chunk = std::max(1, check_every);
+    for (int64_t launch = 0;;) {
+      for (int k = 0; k < chunk; ++k, ++launch) {
+        const int par = (int)(launch & 1);
+        hipLaunchKernelGGL(k_spmv64_rec<0>, dim3(gs), dim3(kBS), 0, s, n, rowptr, col, val, recs, p, q, ks, ppq);
+        hipLaunchKernelGGL(k_pcg_update, dim3(gv), dim3(kBS), 0, s, n, dinv, r, q, ks, ppq, (int)gs, pup, par);
+        hipLaunchKernelGGL(k_pcg_dir, dim3(gv), dim3(kBS), 0, s, n, dinv, x, r, p, ks, pup, (int)gv, par);
+      }
+      NGPB_HIP(hipGetLastError());
+      if (poll()) break;
+    }
   }
   st.status = h.status;
   st.iterations = h.iter;

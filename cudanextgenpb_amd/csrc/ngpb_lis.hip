@@ -696,7 +696,6 @@ const double* psolve(ngpb_ctx* c, int precon, double w, const double* in, double
 }
 
 void prepare_precon(ngpb_ctx* c, int precon, double w) {
-  check_operator(c);  // inverse diagonal, NaN/Inf and diagonal checks
   if (precon != NGPB_PRECON_SSOR) return;
   if (!c->have_levels) build_ssor_levels(c);
   pack_triangle<true>(c, c->ssor_f, w);
@@ -717,6 +716,7 @@ void check_lis_options(const ngpb_solve_opts& o) {
 }
 
 void precond_apply(ngpb_ctx* c, int precon, double omega, const double* r, double* z) {
+  check_operator(c);  // inverse diagonal, NaN/Inf and diagonal checks
   prepare_precon(c, precon, omega);
   ensure_reduce(c, 2048);
   KrylovScalars zero;
@@ -732,6 +732,7 @@ void solve_lis(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
   check_lis_options(o);
   const int64_t n = c->n;
   const double w = ssor_omega(o);
+  const void* rec = slice_records(c, nullptr);
   prepare_precon(c, o.precon, w);
   c->x.resize((size_t)n);
   c->r.resize((size_t)n);
@@ -756,7 +757,6 @@ void solve_lis(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
   NGPB_HIP(hipEventCreate(&e0));
   NGPB_HIP(hipEventCreate(&e1));
   NGPB_HIP(hipEventRecord(e0, c->stream));
-  const void* rec = slice_records(c);
   hipLaunchKernelGGL(k_lis_init, G, B, 0, c->stream, n, c->rhs.p, x, r, rt, p, q, v, dpart);
   hipLaunchKernelGGL(k_lis_fin_init, F, BF, 0, c->stream, ks, dpart, np, o.tol * o.tol, o.maxiter);
   if (o.solver == NGPB_SOLVER_CG) {

@@ -5,7 +5,8 @@ relative residual of 1e-13 by ngpb_solve_csr_noalloc: the relative error is then
 3e-13 plus rounding. Sizes lie around the slice (64) and block (256) edges; the entries
 lie on few diagonals with one value each, on few diagonals with varying values, on
 exactly as many diagonals as a record holds and one more, or anywhere (more than one
-staged piece per slice).
+staged piece per slice). Up to 4,096 rows, on at most 14 diagonals, one block runs the whole CG
+with 1, 2 or 4 rows per thread, 1,024 iterations per launch.
 """
 import ctypes
 from types import SimpleNamespace
@@ -44,7 +45,7 @@ def system(n, form, rng):
 
 
 @pytest.mark.parametrize("form", ["constant", "vary", "full", "over", "random"])
-@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 257, 1000, 70001])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 257, 1000, 1025, 2049, 4096, 4097, 70001])
 def test_forms(n, form):
     rng = np.random.default_rng(n)
     A = system(n, form, rng)
@@ -56,3 +57,21 @@ def test_forms(n, form):
     if ref is not None:
         assert np.linalg.norm(x - ref) <= 1e-12 * np.linalg.norm(ref)
     assert np.linalg.norm(A @ x - b) <= 1e-12 * np.linalg.norm(b)
+
+
+def test_more_iterations_than_one_launch():
+    """A chain whose CG needs more iterations than one launch of the small-system kernel
+    takes."""
+    n = 4000
+    A = sp.diags([-np.ones(n - 1), 2.0 * np.ones(n), -np.ones(n - 1)], [-1, 0, 1]).tocsr()
+    b = np.zeros(n)
+    b[n // 3] = 1.0
+    S = SimpleNamespace(n=n, rowptr=A.indptr, col=A.indices, val=A.data, rhs=b)
+    rc, x, st = solve_noalloc(hip(), S, 1e-13)
+    # a source at row k: the solution is exact once the residual has run through the chain
+    assert rc == 0 and 1024 < st["iterations"] <= 2 * n
+    i = np.arange(1, n + 1)
+    s = n // 3 + 1
+    ref = np.where(i <= s, i * (n + 1 - s), s * (n + 1 - i)) / (n + 1)
+    # condition number about 4 (n + 1)^2 / pi^2 = 6.5e6
+    assert np.linalg.norm(x - ref) <= 6.5e6 * 1e-13 * np.linalg.norm(ref)
