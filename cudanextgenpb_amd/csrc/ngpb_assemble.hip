@@ -508,8 +508,8 @@ __global__ void k_leaf_coeffs(MeshView m, const double* __restrict__ eps, const 
 }
 
 __device__ __forceinline__ double decode_code(uint8_t code) {
-  const double mag = ldexp(1.0, -(code & 0x7f));
-  return (code & 0x80) ? -mag : mag;
+  // +-2^-(code & 0x7f)
+  return __hiloint2double(((1023 - (code & 0x7f)) << 20) | (int)((uint32_t)(code & 0x80) << 24), 0);
 }
 
 __device__ __forceinline__ double emission_value(uint32_t id, uint8_t code, int64_t row, int64_t L,
@@ -521,27 +521,16 @@ __device__ __forceinline__ double emission_value(uint32_t id, uint8_t code, int6
 }
 
 // Matrix values. A block (one wave) owns kSvRows consecutive rows (the blocks of the
-// repacked slot emissions): their emissions (contiguous, in slot order) are loaded
-// coalesced and evaluated in parallel into LDS, then one thread per CSR slot adds its
-// run of values in order, so every sum equals the sequential sum of the reference's
-// leaf sweep. Blocks whose rows hold more than kSvCap emissions evaluate straight from
-// global memory. Small blocks with 4 KB of LDS keep many waves resident; on the 8M
-// globular mesh (8 rows, 512 entries, 64 threads) the numeric assembly takes 4.6 ms
-// against 6.4 ms with 32-row blocks of 256 threads and 32 KB of LDS, with identical
-// results.
+// repacked slot emissions): their emissions (contiguous, in slot order) are evaluated in
+// parallel into LDS, kSvCap at a time, then one thread per CSR slot adds its run of
+// values in order, so every sum equals the sequential sum of the reference's leaf sweep.
+// Bound by latency: bounds, ids, coefficients, sums. So all ids of a piece are loaded at
+// once, then all coefficients, and the sums read LDS eight values ahead. On the 8M-node
+// globular mesh: 1.25 ms, 3.49 ms with one emission per thread in flight and blocks of
+// more than kSvCap emissions evaluated from global memory by the slot's thread. 4 KB of
+// LDS keeps the CU's wave slots filled.
 constexpr int kSvCap = 512;
 constexpr int kSvBS = 64;
-
-// last r in [0, nr) with a[r] <= v (a[0] <= v)
-__device__ __forceinline__ int last_le(const uint32_t* a, int nr, uint32_t v) {
-  int lo = 0, hi = nr - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (a[mid] <= v) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
-}
 
 __device__ __forceinline__ void k_slot_values_body(int64_t bid, int64_t N, int64_t L, const int32_t* __restrict__ rowptr,
                                                        const int64_t* __restrict__ blk_em,
@@ -551,52 +540,83 @@ __device__ __forceinline__ void k_slot_values_body(int64_t bid, int64_t N, int64
                                                        const double* __restrict__ c_edge,
                                                        const double* __restrict__ reac,
                                                        const double* __restrict__ v8, double* __restrict__ val) {
+  static_assert(kSvBS == 64 && kSvRows == 8, "one wave per block; rows found by seven compares");
+  constexpr int kU = kSvCap / kSvBS;
   __shared__ double s_v[kSvCap];
-  __shared__ uint32_t s_re[kSvRows + 1];  // per row: first emission (block-relative)
-  __shared__ uint32_t s_rs[kSvRows + 1];  // per row: first slot (block-relative)
-  const int64_t blk = bid;
-  const int64_t r0 = blk * kSvRows;
+  __shared__ double s_reac[kSvRows];
+  const int64_t r0 = bid * kSvRows;
   const int64_t r1 = min(r0 + kSvRows, N);
-  const int nr = (int)(r1 - r0);
-  const int64_t base = blk_em[blk];
-  const uint32_t nem = (uint32_t)(blk_em[blk + 1] - base);
+  const int64_t base = blk_em[bid];
+  const uint32_t nem = (uint32_t)(blk_em[bid + 1] - base);
   const int64_t sl0 = rowptr[r0], sl1 = rowptr[r1];
-  for (int i = threadIdx.x; i < nr; i += kSvBS) {
-    const int64_t sl = rowptr[r0 + i];
-    s_re[i] = sl < sl1 ? slot_rel[sl] : nem;
-    s_rs[i] = (uint32_t)(sl - sl0);
+  const uint32_t mass0 = (uint32_t)(12 * L);  // ids below: edges; from here on: lumped mass
+  const int t = threadIdx.x;
+  // first emission of each row (rows past the end: nem) and its kappa^2
+  uint32_t row_em = nem;
+  if (r0 + t < r1) {
+    const int64_t sl = rowptr[r0 + t];
+    if (sl < sl1) row_em = slot_rel[sl];
+    s_reac[t & (kSvRows - 1)] = reac[r0 + t];
   }
-  if (threadIdx.x == 0) {
-    s_re[nr] = nem;
-    s_rs[nr] = (uint32_t)(sl1 - sl0);
-  }
-  __syncthreads();
-  const bool staged = nem <= (uint32_t)kSvCap;
-  if (staged) {
-    for (uint32_t i = threadIdx.x; i < nem; i += kSvBS) {
-      const uint32_t id = em_id[base + i];
-      const double w = decode_code(em_code[base + i]);
-      double v;
-      if ((int64_t)id < 12 * L) {
-        v = c_edge[id] * w;
-      } else {
-        const int r = last_le(s_re, nr, i);  // lumped mass: the row's own kappa^2
-        v = reac[r0 + r] * v8[((int64_t)id - 12 * L) >> 3] * w;
+  uint32_t first[kSvRows];
+#pragma unroll
+  for (int r = 1; r < kSvRows; ++r) first[r] = (uint32_t)__builtin_amdgcn_readlane((int)row_em, r);
+  auto bounds = [&](int64_t sl, uint32_t& b, uint32_t& e) {
+    b = slot_rel[sl];
+    e = sl + 1 < sl1 ? slot_rel[sl + 1] : nem;
+  };
+  uint32_t tb = 0, te = 0;  // the thread's first slot
+  if (sl0 + t < sl1) bounds(sl0 + t, tb, te);
+  for (uint32_t p0 = 0; p0 < nem; p0 += kSvCap) {
+    const uint32_t np = min(nem - p0, (uint32_t)kSvCap);
+    uint32_t id[kU];
+    uint8_t code[kU];
+    double v[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const uint32_t i = p0 + min((uint32_t)(u * kSvBS + t), np - 1);
+      id[u] = em_id[base + i];
+      code[u] = em_code[base + i];
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) v[u] = *(id[u] < mass0 ? c_edge + id[u] : v8 + ((id[u] - mass0) >> 3));
+    __syncthreads();  // s_reac is set, the previous piece has been added
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const uint32_t i = p0 + u * kSvBS + t;
+      if (id[u] >= mass0) {  // lumped mass: times the row's own kappa^2
+        int r = 0;
+#pragma unroll
+        for (int k = 1; k < kSvRows; ++k) r += first[k] <= i ? 1 : 0;
+        v[u] *= s_reac[min(r, (int)(r1 - r0) - 1)];
       }
-      s_v[i] = v;
+      s_v[u * kSvBS + t] = v[u] * decode_code(code[u]);
     }
-  }
-  __syncthreads();
-  for (int64_t sl = sl0 + threadIdx.x; sl < sl1; sl += kSvBS) {
-    const uint32_t b = slot_rel[sl], e = sl + 1 < sl1 ? slot_rel[sl + 1] : nem;
-    double v = 0.0;
-    if (staged) {
-      for (uint32_t i = b; i < e; ++i) v += s_v[i];
-    } else {
-      const int64_t row = r0 + last_le(s_rs, nr, (uint32_t)(sl - sl0));
-      for (uint32_t i = b; i < e; ++i) v += emission_value(em_id[base + i], em_code[base + i], row, L, c_edge, reac, v8);
+    __syncthreads();
+    for (int64_t sl = sl0 + t; sl < sl1; sl += kSvBS) {
+      uint32_t b = tb, e = te;
+      if (sl != sl0 + t) bounds(sl, b, e);
+      if (e <= p0 || b >= p0 + np) continue;
+      double sum = b < p0 ? val[sl] : 0.0;  // a run over the end of a piece goes on
+      uint32_t i = max(b, p0) - p0;
+      const uint32_t end = min(e - p0, np);
+      for (; i + 8 <= end; i += 8) {
+        double w[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) w[u] = s_v[i + u];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) sum += w[u];
+      }
+      for (; i + 4 <= end; i += 4) {
+        double w[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) w[u] = s_v[i + u];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) sum += w[u];
+      }
+      for (; i < end; ++i) sum += s_v[i];
+      val[sl] = sum;
     }
-    val[sl] = v;
   }
 }
 
