@@ -299,7 +299,7 @@ int ngpb_precond_apply(ngpb_ctx* ctx, int precon, double omega, const double* r,
    `device`: rowptr (n+1), col (nnz), val (nnz), rhs (n) in, x (n) out, all device
    pointers; stream is a hipStream_t (NULL: the default stream). opts: precision FP64,
    solver CG, precon Jacobi, tol, maxiter, check_every. All work memory (4 vectors of
-   n doubles, partial sums, scalars) lives in a file-scope device array of 32.1 MiB per
+   n doubles, partial sums, scalars) lives in a file-scope device array of 36.6 MiB per
    GPU, held until the process ends; n is limited to 1,048,576 rows (NGPB_E_ARG
    beyond). The call makes no hipMalloc/hipFree or pinned-host allocation. Every call
    on one GPU shares that array: calls that overlap on one GPU race. Returns NGPB_OK,
