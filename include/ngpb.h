@@ -98,7 +98,7 @@ typedef struct {
   int replacements;    /* mixed: FP64 residual replacements */
   double relres;       /* ||b - A x|| / ||b|| : recursive (FP64) or true FP64 (mixed) */
   double ms_solve;     /* wall time of the solve on the device stream */
-  double bytes_per_iter;  /* algorithmic HBM bytes of one iteration */
+  double bytes_per_iter;  /* algorithmic HBM bytes of one iteration (FP64: the operator counted as CSR) */
 } ngpb_solve_stats;
 
 typedef struct {
