@@ -186,6 +186,7 @@ struct KrylovScalars {
   double rho2[2];   // (r, z) entering the iteration of parity par
   double alpha2[2]; // alpha of the iteration of parity par
   int iter2[2];     // iterations completed before the iteration of parity par
+  int halt2[2];     // FP64 CG: 1 = stopped before the direction kernel of parity par
   int stop_par;     // parity of the iteration that raised the stop flag
   int iter;         // iterations done in this solve
   int done;         // 1 = stop flag raised

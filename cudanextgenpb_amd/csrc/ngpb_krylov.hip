@@ -511,7 +511,7 @@ __global__ void __launch_bounds__(kFin) k_fin_init(KrylovScalars* ks, const doub
     ks->iter = 0;
     ks->maxiter = maxiter;
     ks->status = 0;
-    ks->done = (BB == 0.0) ? 1 : 0;
+    ks->done = ks->halt2[0] = ks->halt2[1] = (BB == 0.0) ? 1 : 0;
   }
 }
 
@@ -547,12 +547,17 @@ __global__ void __launch_bounds__(kBS) k_pcg_update(int64_t n, const double* __r
 
 // x += alpha p (here, where p is read for its own update too), the stop test on ||r||^2
 // (every block decides alike), then beta = (r', z') / (r, z) and p = D^-1 r + beta p.
-// Block 0 records the scalars for the next iteration and the host.
+// Block 0 records the scalars for the next iteration and the host. The last step is added
+// by the launch that raises the stop flag, so a block must not return on a flag that this
+// same launch writes: it tests halt2[par], which the launch before has written.
 __global__ void __launch_bounds__(kBS) k_pcg_dir(int64_t n, const double* __restrict__ dinv, double* __restrict__ x,
                                                  const double* __restrict__ r, double* __restrict__ p, KrylovScalars* ks,
                                                  const double* __restrict__ part, int np, int par) {
   __shared__ double s_red[kBS / 64];
-  if (ks->done) return;
+  if (ks->halt2[par]) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) ks->halt2[par ^ 1] = 1;
+    return;
+  }
   const double RZ = dev::sum_partials<kBS>(part, np, 2, s_red);
   const double RR = dev::sum_partials<kBS>(part + 1, np, 2, s_red);
   const int it = ks->iter2[par] + 1;
@@ -565,6 +570,7 @@ __global__ void __launch_bounds__(kBS) k_pcg_dir(int64_t n, const double* __rest
     ks->iter2[par ^ 1] = it;
     if (stop) {
       ks->done = 1;
+      ks->halt2[par ^ 1] = 1;
       ks->status = conv ? 0 : NGPB_E_NOCONV;
       ks->stop_par = par;
     } else {

@@ -36,7 +36,10 @@ def test_reused_blocks_across_threads():
             print(f"[block pool] round {r}", flush=True)
             order = np.random.default_rng(r).permutation(len(jobs))
             for k, got in zip(order, ex.map(lambda k: _solve(*jobs[k]), order)):
-                assert all(np.array_equal(a, b) for a, b in zip(got, ref[k])), jobs[k][0].name
+                for name, a, b in zip(("potential", "energy", "at atoms"), got, ref[k]):
+                    d = np.abs(np.asarray(a) - np.asarray(b))
+                    assert np.array_equal(a, b), (jobs[k][0].name, "mixed" if jobs[k][1] else "fp64", jobs[k][2], name,
+                                                  int((d > 0).sum()), float(d.max()))
 
 
 def test_pool_does_not_grow():
