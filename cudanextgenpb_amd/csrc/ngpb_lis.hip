@@ -370,8 +370,8 @@ static_assert(sizeof(RunLds) <= 160 * 1024, "one block's LDS");
 // It is in memory by then: at least 16 - 3 pieces old, and every solving wave completes
 // all its stores every 8 pieces.
 //
-// Every load is unconditional (addresses clamped): the compiler can then count the
-// loads in flight and wait for just those it needs. A sweep over the 255,000-row mesh
+// Every load is unconditional (addresses clamped, into at least one entry): the compiler
+// can then count the loads in flight and wait for just those it needs. A sweep over the 255,000-row mesh
 // took 2.3 ms with one launch per level; in one block 1.46 ms with guarded loads (each
 // piece waited for all of them), 0.92 ms with clamped loads and every thread doing both
 // jobs, 0.87 ms with loads one piece ahead of their use and 0.69 ms now, about 1 us a
@@ -576,7 +576,9 @@ void order_triangle(ngpb_ctx* c, ngpb_ctx::SsorTriangle& t, const std::vector<in
   std::vector<int32_t> pieces;
   for (int32_t l = 0; l < nlev; ++l) {
     const int32_t a = first[(size_t)l], b = first[(size_t)l + 1];
-    if (b - a > kNarrow || longest > kPieceEntries) {
+    // without any entry (a diagonal operator) there is nothing to stage: k_ssor_run reads
+    // columns at clamped indices and needs one
+    if (b - a > kNarrow || longest > kPieceEntries || longest == 0) {
       t.runs.push_back({a, b, false});
       continue;
     }

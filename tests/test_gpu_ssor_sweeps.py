@@ -1,13 +1,16 @@
 """SSOR sweeps on sparsity patterns that reach every path of the level-ordered sweeps
 (csrc/ngpb_lis.hip), bit-identical to the oracle's sequential sweeps:
 
-* one level of all rows (wider than a one-block run: launched on its own);
+* triangles without entries, from one row up, and one level of all rows (wider than a
+  one-block run): launched on their own;
 * one row per level (a chain; neighbours in the LDS window only);
-* chains with links far behind (neighbours older than the 16384-position window, read
-  from memory) and to the first rows;
-* rows with more neighbours than the register slots (8), and random patterns whose
+* chains with links far behind (neighbours older than the 8192-position window, read
+  from memory) and to the first rows, links at the window's edge, and levels of one full
+  piece (512 rows) linked 15, 16 and 17 levels back;
+* rows with more neighbours than are read together (4, 8, 16), and random patterns whose
   levels are narrow at the ends and wide in the middle (runs between launches);
-* levels of 256 .. 2048 rows around the group sizes (512 and 1024 rows prefetched).
+* levels of 255 .. 2049 rows around the piece size (512 rows) and the widest level of a
+  one-block run (2048).
 """
 import numpy as np
 import pytest
@@ -47,11 +50,18 @@ def layered(width, layers, links, seed, far=0):
 
 
 def cases():
-    yield "diagonal", system(5000, np.zeros((0, 2)), 1)
+    for n in (1, 2, 64, 513, 2048, 2049, 5000):
+        yield f"diagonal_{n}", system(n, np.zeros((0, 2)), 1)
     yield "chain", system(3000, [(i, i - 1) for i in range(1, 3000)], 2)
     n = 30000
     far = [(i, i - 1) for i in range(1, n)] + [(i, i - 20000) for i in range(20000, n, 7)] + [(i, 0) for i in range(2, n, 11)]
     yield "far_chain", system(n, far, 3)
+    n = 9000
+    edge = [(i, i - 1) for i in range(1, n)] + [(i, i - d) for d in (8190, 8191, 8192, 8193) for i in range(d, n, 3)]
+    yield "window_edge", system(n, edge, 6)
+    i = np.arange(512, 512 * 40)
+    back = [np.stack([i, i - 512], 1)] + [np.stack([i, i - 512 * k], 1)[i >= 512 * k] for k in (15, 16, 17)]
+    yield "full_pieces", system(512 * 40, np.concatenate(back), 7)
     yield "long_rows", layered(100, 30, 13, 4)
     for width in (255, 256, 257, 512, 513, 1024, 1025, 2048, 2049):
         yield f"layers_{width}", layered(width, 12, 3, width, far=40)
