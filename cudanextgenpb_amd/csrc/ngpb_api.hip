@@ -68,6 +68,10 @@ void install_device_mesh(ngpb_ctx* c, int64_t N, int64_t H, int64_t L, int64_t N
 
 }  // namespace ngpb
 
+int64_t ngpb_ctx::mg_bytes() const {
+  return mg_pool.bytes() + mg_dense.bytes() + mg_sd.bytes() + mg_r.bytes() + mg_z.bytes() + mg_pos.bytes();
+}
+
 int64_t ngpb_ctx::device_bytes() const {
   int64_t b = 0;
   b += node_xyz.bytes() + hang_xyz.bytes() + hang_np.bytes() + hang_par.bytes() + leaf_corner.bytes();
@@ -89,7 +93,7 @@ int64_t ngpb_ctx::device_bytes() const {
   b += lis_rt.bytes() + lis_u.bytes() + lis_v.bytes() + lis_ph.bytes() + lis_uh.bytes() + lis_t.bytes() +
        diag_pos.bytes() + ssor_f.bytes() + ssor_b.bytes();
   b += xs.bytes() + rs.bytes() + ps.bytes() + qs.bytes() + ks.bytes();
-  b += mg_pool.bytes() + mg_dense.bytes() + mg_sd.bytes() + mg_r.bytes() + mg_z.bytes() + mg_pos.bytes() + slice_rec.bytes();
+  b += mg_bytes() + slice_rec.bytes();
   b += red.partials.bytes() + scan_tmp.bytes();
   for (const auto& t : tmp) b += t.bytes();
   return b;
@@ -1256,6 +1260,24 @@ int ngpb_set_row_order(ngpb_ctx* c, int band) {
       c->row_band = band;
       c->have_compact = false;  // rebuilt in the new order on next use
     }
+  });
+}
+
+int ngpb_set_multigrid(ngpb_ctx* c, int cycle_iters, int64_t max_bytes) {
+  return guarded(c, [&] {
+    not_in_batch(c);
+    NGPB_REQUIRE(cycle_iters >= 0 && max_bytes >= 0, NGPB_E_ARG, "multigrid limits must not be negative");
+    c->mg_cycle_iters = cycle_iters;
+    c->mg_max_bytes = max_bytes;
+    c->mg_state = 0;  // decided anew on next use
+  });
+}
+
+int ngpb_multigrid_info(ngpb_ctx* c, int* in_use, int64_t* bytes) {
+  return guarded(c, [&] {
+    NGPB_REQUIRE(in_use && bytes, NGPB_E_ARG, "NULL output");
+    *in_use = c->have_system && c->have_compact && c->mg_state > 0 ? 1 : 0;
+    *bytes = c->mg_bytes();
   });
 }
 

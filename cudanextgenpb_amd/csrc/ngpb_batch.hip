@@ -866,8 +866,10 @@ int ngpb_batch_add(ngpb_batch* b, ngpb_ctx* c, int* slot) {
     c->x.resize((size_t)n);
     c->q.reserve((size_t)n);
     c->xs.reserve((size_t)n);
-    const bool mg = ngpb::mg_setup(c);
+    c->qs.reserve((size_t)n);
+    c->red.partials.reserve((size_t)std::max<int64_t>(3 * c->n_slices, 1));
     float* const pin = ngpb::spmv_input(c);  // zero guard entries either side
+    const bool mg = ngpb::mg_setup(c);       // takes memory after what every system needs
     float *rs, *zs = nullptr;
     if (mg) {
       rs = ngpb::guarded_vector(c, c->mg_r);
@@ -876,8 +878,6 @@ int ngpb_batch_add(ngpb_batch* b, ngpb_ctx* c, int* slot) {
       c->rs.reserve((size_t)n);
       rs = c->rs.p;
     }
-    c->qs.reserve((size_t)n);
-    c->red.partials.reserve((size_t)std::max<int64_t>(3 * c->n_slices, 1));
     NGPB_HIP(hipStreamSynchronize(c->stream));
     ngpb::BatchDesc d;
     std::memset(&d, 0, sizeof(d));

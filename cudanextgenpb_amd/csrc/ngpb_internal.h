@@ -332,6 +332,8 @@ struct ngpb_ctx {
   ngpb::DBuf<double> dscale;         // 1/sqrt(diag)
   // multigrid preconditioner of the mixed solve, built with the compact operator
   int mg_state = 0;  // 0 not built, 1 in use, -1 does not apply to this operator
+  int mg_cycle_iters = 100;  // iterations of an inner cycle before Jacobi scaling takes over (0: from the start)
+  int64_t mg_max_bytes = 0;  // most device bytes of the hierarchy (0: what the device has)
   ngpb::MgHierarchy mg;
   ngpb::DBuf<float> mg_pool, mg_dense, mg_sd, mg_r, mg_z;  // mg_r, mg_z: with SpMV guard entries
   ngpb::DBuf<uint32_t> mg_pos;
@@ -392,6 +394,7 @@ struct ngpb_ctx {
   int64_t prof_tag = 0;
   bool prof_first = false;
 
+  int64_t mg_bytes() const;
   int64_t device_bytes() const;
 };
 
@@ -482,6 +485,7 @@ double time_spmv_fp64(ngpb_ctx* c, int reps);
 // mixed
 void build_compact(ngpb_ctx* c, bool allow_band = true);  // allow_band: banded row order may apply
 float* spmv_input(ngpb_ctx* c);  // FP32 SpMV input vector (zero guard entries either side)
+constexpr int kGuard = 64;       // those guard entries
 float* guarded_vector(ngpb_ctx* c, DBuf<float>& v);  // n entries between such guards
 void spmv_compact(ngpb_ctx* c, const double* x, double* y);
 void solve_mixed(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st);
@@ -492,6 +496,7 @@ double time_spmv_compact(ngpb_ctx* c, int reps);
 // mg_precondition, an SpMV on z, mg_direction, an SpMV on p and mg_update. par is the
 // parity of the iteration; every kernel returns at once after the stop flag.
 bool mg_setup(ngpb_ctx* c);
+void mg_release(ngpb_ctx* c);
 // z0 from r and ar = Ahat r, and (r, z) up to omega (r, r) in rz_part; stops first if
 // (r, r) from the partials met the target
 void mg_precondition(ngpb_ctx* c, const float* r, const float* ar, float* z, const double* rr_part, int npr,

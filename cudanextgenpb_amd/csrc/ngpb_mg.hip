@@ -440,16 +440,12 @@ dim3 grid_of(const MgGrid& g) {
   return dim3((unsigned)((g.pitch + 63) / 64), (unsigned)((g.cy + 4) / 4), (unsigned)(g.cz + 1));
 }
 
-}  // namespace
-
-// Builds the hierarchy for the context's current operator; false (and c->mg_state = -1)
-// where it does not apply: a system loaded as CSR, a mesh that is not an octree of cubes
-// on one lattice of at most 1022 cells an axis, Dirichlet nodes other than the box
-// faces, or a mesh so sparse on its finest lattice that the dense transfer array would
-// cost more than the iterations it saves.
-bool mg_setup(ngpb_ctx* c) {
-  if (c->mg_state) return c->mg_state > 0;
-  c->mg_state = -1;
+// Builds the hierarchy for the context's current operator; false where it does not apply:
+// a system loaded as CSR, a mesh that is not an octree of cubes on one lattice of at most
+// 1022 cells an axis, Dirichlet nodes other than the box faces, or a mesh so sparse on
+// its finest lattice that the dense transfer array would cost more than the iterations it
+// saves.
+bool build_hierarchy(ngpb_ctx* c) {
   if (c->external_csr || !c->have_mesh || c->n != c->N || c->L <= 0 || c->n < 64) return false;
   const MeshView m = mesh_view_of(c);
   const int64_t n = c->n, L = c->L;
@@ -511,10 +507,17 @@ bool mg_setup(ngpb_ctx* c) {
     floats += l.nodes() * 8;  // ex ey ez dinv b x t f
     if (std::min({cells[0], cells[1], cells[2]}) <= 2) break;
   }
-  c->mg_pool.reserve((size_t)floats);
-  c->mg_dense.reserve((size_t)dense);
-  c->mg_pos.reserve((size_t)n);
-  c->mg_sd.reserve((size_t)n);
+  auto take = [&](auto& buf, int64_t count) {
+    buf.reserve((size_t)count);
+    if (c->mg_max_bytes > 0 && c->mg_bytes() > c->mg_max_bytes)
+      throw Error(NGPB_E_NOMEM, "the multigrid hierarchy exceeds its memory bound");
+  };
+  take(c->mg_pool, floats);
+  take(c->mg_dense, dense);
+  take(c->mg_pos, n);
+  take(c->mg_sd, n);
+  take(c->mg_r, n + 2 * kGuard);
+  take(c->mg_z, n + 2 * kGuard);
   H.dense = c->mg_dense.p;
   {
     float* p = c->mg_pool.p;
@@ -577,8 +580,40 @@ bool mg_setup(ngpb_ctx* c) {
   NGPB_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mg_bottom), hipFuncAttributeMaxDynamicSharedMemorySize,
                                kMgBottomLds));
   NGPB_HIP(hipStreamSynchronize(st));
-  c->mg_state = 1;
   return true;
+}
+
+}  // namespace
+
+void mg_release(ngpb_ctx* c) {
+  c->mg_pool.release();
+  c->mg_dense.release();
+  c->mg_sd.release();
+  c->mg_r.release();
+  c->mg_z.release();
+  c->mg_pos.release();
+  c->mg = MgHierarchy();
+}
+
+// True once the hierarchy of the current operator is built, false (c->mg_state = -1) where
+// it does not apply or there is no memory for it: the solve then uses Jacobi scaling, and
+// nothing is held.
+bool mg_setup(ngpb_ctx* c) {
+  if (c->mg_state) return c->mg_state > 0;
+  c->mg_state = -1;
+  bool ok = false;
+  try {
+    ok = c->mg_cycle_iters > 0 && build_hierarchy(c);
+  } catch (const Error& e) {
+    mg_release(c);
+    if (e.code != NGPB_E_NOMEM) throw;
+  } catch (...) {
+    mg_release(c);
+    throw;
+  }
+  if (ok) c->mg_state = 1;
+  else mg_release(c);
+  return ok;
 }
 
 // ------------------------------------------------------------------ launches

@@ -643,7 +643,6 @@ __global__ void k_pk_hdr_list(int64_t cnt, const int32_t* __restrict__ list, con
 //   * a pair's slice ids, slot pointers and widths come from one 32-byte record, a
 //     packed slice's id and header from two independent loads.
 // Results equal those of k_sell_both except possibly for the sign of an exact zero.
-constexpr int kGuard = 64;
 
 __device__ __forceinline__ void lean_dpair(const Sell& A, const DPair& m, const float* __restrict__ x,
                                            float* __restrict__ y, double* part) {
@@ -1422,18 +1421,18 @@ double time_spmv_compact(ngpb_ctx* c, int reps) {
 
 // Solves with the multigrid preconditioner where it applies (mg_setup): an inner cycle
 // is then CG preconditioned by one V-cycle, 20-30 iterations in all against 300-900 with
-// Jacobi scaling alone. Should the cycle not converge (kMgCycleIters iterations, or a
+// Jacobi scaling alone. Should the cycle not converge (mg_cycle_iters iterations, or a
 // non-finite residual), the solve goes on with the Jacobi-scaled CG.
 void solve_mixed(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
-  constexpr int kMgCycleIters = 100;
   const int64_t n = c->n;
   check_operator(c);
   if (!c->have_compact) build_compact(c);
-  bool mg = mg_setup(c);
   c->x.resize((size_t)n);
   c->q.reserve((size_t)n);
   c->xs.reserve((size_t)n);
+  c->qs.reserve((size_t)n);
   float* const pv = spmv_input(c);
+  bool mg = mg_setup(c);  // takes memory after what every solve needs
   float* rv;  // residual of the inner iteration
   float* zv = nullptr;
   if (mg) {
@@ -1444,7 +1443,6 @@ void solve_mixed(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
     rv = c->rs.p;
   }
   const int32_t* const perm = c->sell_banded ? c->row_perm.p : nullptr;  // FP32 row -> node
-  c->qs.reserve((size_t)n);
   const unsigned gv = vec_grid(n);
   const unsigned gs = (unsigned)sell_partials(c);
   const int64_t region = std::max<int64_t>(gs, 2048);
@@ -1497,7 +1495,7 @@ void solve_mixed(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
       const double ss = h->aux[1], tt = h->aux[0];
       const double ratio = tt > 0.0 ? ss / tt : 1.0;
       h->stop_rr = std::max(drop * drop * ss, 0.25 * target * ratio);
-      h->maxiter = mg ? std::min(o.maxiter, iters + kMgCycleIters) : o.maxiter;
+      h->maxiter = mg ? (int)std::min<int64_t>(o.maxiter, (int64_t)iters + c->mg_cycle_iters) : o.maxiter;
       h->iter = iters;
       h->done = 0;
       h->rho2[launch & 1] = mg ? mg_rho : h->rho;

@@ -124,6 +124,8 @@ SIGNATURES = {
     "ngpb_row_order": (_I, [_P, _P]),
     "ngpb_operator_info": (_I, [_P, _P]),
     "ngpb_set_compact_options": (_I, [_P, _I]),
+    "ngpb_set_multigrid": (_I, [_P, _I, _I64]),
+    "ngpb_multigrid_info": (_I, [_P, _P, _P]),
     "ngpb_set_spmv_schedule": (_I, [_P, _I]),
     "ngpb_batch_create": (_I, [_P, _I, _I]),
     "ngpb_batch_destroy": (_I, [_P]),
@@ -466,6 +468,17 @@ class Context:
 
     def set_compact_options(self, constant_slices: bool = True):
         self._check(lib().ngpb_set_compact_options(self._h, 1 if constant_slices else 0), "set_compact_options")
+
+    def set_multigrid(self, cycle_iters: int = 100, max_bytes: int = 0):
+        """Limits of the multigrid preconditioner of mixed solves: iterations of an inner
+        cycle before Jacobi scaling takes over (0: from the start), and the device bytes
+        it may take (0: no bound; Jacobi scaling where it does not fit)."""
+        self._check(lib().ngpb_set_multigrid(self._h, int(cycle_iters), int(max_bytes)), "set_multigrid")
+
+    def multigrid_info(self) -> dict:
+        u, b = ctypes.c_int(0), ctypes.c_int64(0)
+        self._check(lib().ngpb_multigrid_info(self._h, ctypes.byref(u), ctypes.byref(b)), "multigrid_info")
+        return dict(in_use=bool(u.value), bytes=b.value)
 
     def set_row_order(self, band: int):
         """Row order of the compact FP32 operator: 0 node order, > 0 y-bands of that

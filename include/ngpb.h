@@ -369,6 +369,17 @@ int ngpb_operator_info(ngpb_ctx* ctx, int64_t* info12);
    operator is rebuilt on next use when the setting changes. No counterpart in the
    reference. */
 int ngpb_set_compact_options(ngpb_ctx* ctx, int constant_slices);
+/* Limits of the multigrid preconditioner of mixed solves (alone or in a batch).
+   cycle_iters (default 100): iterations of an inner cycle after which the solve goes on
+   with Jacobi scaling alone; 0: Jacobi scaling from the start. max_bytes (default 0: no
+   bound): device memory its hierarchy and vectors may take; where they do not fit, or the
+   device has no memory left for them, Jacobi scaling is used and nothing is held. Not
+   while the context is in a batch. No counterpart in the reference. */
+int ngpb_set_multigrid(ngpb_ctx* ctx, int cycle_iters, int64_t max_bytes);
+/* Whether the last mixed solve (or batch) of the current system started with the
+   multigrid preconditioner, and the device bytes held for it. No counterpart in the
+   reference. */
+int ngpb_multigrid_info(ngpb_ctx* ctx, int* in_use, int64_t* bytes);
 /* Work schedule of the SpMV kernels. Compact FP32: 0 one kernel per slice form
    (delta / packed / offset, each walking a list of its slices) on up to 2048 blocks,
    1 a single kernel for all forms, 2 as 0 on the resident block count, 3 the delta

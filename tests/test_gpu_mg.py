@@ -1,14 +1,14 @@
 """The multigrid preconditioner of the mixed solve (csrc/ngpb_mg.hip).
 
-Each system's mixed potential against its FP64 solve to 1e-12: both stop on the true
-residual (1e-10 of ||b||), so the difference is bounded by the condition of the scaled
-operator times 1e-10; 1e-8 leaves a factor of 100 over the largest measured (3e-11 on
-meshes of this size). Sizes where a level can go wrong: 3 cells an axis (one coarse
+Each system's mixed potential (true residual 1e-10 of ||b||) against its FP64 solve to
+1e-12: the difference is bounded by the condition of the scaled operator times 1e-10;
+1e-8 leaves a factor of 300 over the largest measured (3e-11 on meshes of this size).
+Sizes where a level can go wrong: 3 cells an axis (one coarse
 interior node), odd counts (the last coarse cell reaches past the box), boxes of uneven
 sides (a last level of several nodes), four refinement levels (nodes that live on levels
 2 to 4), rows in bands. Where the preconditioner does not apply (a lattice too sparse, a
-Dirichlet set other than the box faces, an operator loaded as CSR) the Jacobi-scaled
-iteration gives the same potential.
+Dirichlet set other than the box faces, an operator loaded as CSR, no memory for it) it is
+not in use, nothing is held for it, and the Jacobi-scaled iteration gives the potential.
 """
 import dataclasses
 
@@ -30,12 +30,14 @@ def box_spec(n, h=0.5, levels=0, bands=(), atoms=3):
     return W.Spec("box", W.Physics(), a, -half, h, n, levels, tuple(bands), 2, W.P4EST_TOL * n[0] * h)
 
 
-def solve_both(ctx):
+def solve_both(ctx, multigrid=True):
     phi64, st64 = ctx.solve(native.PREC_FP64, tol=1e-12)
     phi, st = ctx.solve(native.PREC_MIXED, tol=1e-10)
     rel = np.linalg.norm(phi - phi64) / np.linalg.norm(phi64)
     print(f"   n={ctx.n}: FP64 {st64['iterations']} it, mixed {st['iterations']} it, phi rel {rel:.1e}", flush=True)
     assert st["status"] == 0 and st["relres"] <= 1e-10 and rel <= 1e-8
+    info = ctx.multigrid_info()
+    assert info["in_use"] == multigrid and (info["bytes"] > 0) == multigrid
     return phi, st
 
 
@@ -68,7 +70,7 @@ def test_sparse_lattice_uses_jacobi():
     """More than 32 finest-lattice vertices per node: the dense transfer array is not built."""
     p = prepare(box_spec((192, 192, 192), h=0.25, levels=4, bands=(0.1, 0.1, 0.1, 0.1), atoms=1))
     assert 193 ** 3 > 32 * p.n
-    _, st = solve_both(p.ctx)
+    solve_both(p.ctx, multigrid=False)
     p.ctx.close()
 
 
@@ -84,13 +86,40 @@ def test_other_dirichlet_sets_and_csr_use_jacobi():
     nodes = np.append(P.mesh.bnd_nodes, inner).astype(np.int32)  # one fixed node inside
     ctx.set_dirichlet(nodes, np.linspace(0.0, 0.1, len(nodes)))
     ctx.assemble()
-    solve_both(ctx)
+    solve_both(ctx, multigrid=False)
     csr = ctx.export_csr()
     ctx.close()
     other = native.Context(0)
     other.set_csr(*csr)
-    solve_both(other)
+    solve_both(other, multigrid=False)
     other.close()
+
+
+def test_no_memory_uses_jacobi():
+    """A bound on its memory that any of its allocations can run into: the solve goes on
+    as with Jacobi scaling from the start, alone and in a batch."""
+    p = prepare(box_spec((48, 48, 48), levels=2, bands=(1.0, 2.5)))
+    _, st = solve_both(p.ctx)
+    full = p.ctx.multigrid_info()["bytes"]
+    p.ctx.set_multigrid(cycle_iters=0)
+    phi, stj = solve_both(p.ctx, multigrid=False)
+    assert stj["iterations"] > 2 * st["iterations"]
+    n = p.n
+    for bound in (1, full // 2, full - 12 * n - 1, full - 8 * n, full - 1):
+        print(f"[mg] {bound} of {full} bytes", flush=True)
+        p.ctx.set_multigrid(max_bytes=bound)
+        got, s = solve_both(p.ctx, multigrid=False)
+        assert np.array_equal(got, phi) and s["iterations"] == stj["iterations"]
+        with native.Batch(0, max_systems=1, tol=1e-10) as b:
+            slot = b.add(p.ctx)
+            b.run(1000)
+            done, sb = b.status(slot)
+            b.remove(slot)
+        assert done and sb["status"] == 0 and not p.ctx.multigrid_info()["in_use"]
+        assert np.linalg.norm(p.ctx.get_phi() - phi) <= 1e-8 * np.linalg.norm(phi)
+    p.ctx.set_multigrid(max_bytes=full)
+    solve_both(p.ctx)
+    p.ctx.close()
 
 
 def test_host_mesh_equals_device_mesh():
