@@ -6,6 +6,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <list>
 #include <map>
 #include <mutex>
 #include <sstream>
@@ -155,8 +156,39 @@ thread_local int IdleRelease::depth = 0;
 namespace {
 constexpr size_t kPoolMax = size_t(16) << 30;  // per device
 struct Pool {
-  std::multimap<size_t, void*> free;  // by size class
+  struct Block {
+    size_t size;
+    void* p;
+  };
+  std::list<Block> blocks;                                   // oldest first
+  std::multimap<size_t, std::list<Block>::iterator> by_size;  // by size class
   size_t bytes = 0;
+
+  void put(void* p, size_t size) {
+    by_size.emplace(size, blocks.insert(blocks.end(), Block{size, p}));
+    bytes += size;
+  }
+  void* take(size_t size) {
+    auto f = by_size.find(size);
+    if (f == by_size.end()) return nullptr;
+    void* p = f->second->p;
+    blocks.erase(f->second);
+    by_size.erase(f);
+    bytes -= size;
+    return p;
+  }
+  // moves the oldest blocks to `out` until at most `keep` bytes stay
+  void trim(size_t keep, std::vector<void*>& out) {
+    while (bytes > keep) {
+      auto b = blocks.begin();
+      auto f = by_size.lower_bound(b->size);
+      while (f->second != b) ++f;
+      by_size.erase(f);
+      bytes -= b->size;
+      out.push_back(b->p);
+      blocks.erase(b);
+    }
+  }
 };
 std::mutex g_pool_mu;
 std::unordered_map<int, Pool> g_pool;  // by device
@@ -174,32 +206,31 @@ int current_device() {
 }
 }  // namespace
 
+size_t pool_trim(int device, size_t keep) {
+  std::vector<void*> out;
+  size_t held = 0;
+  {
+    std::lock_guard<std::mutex> g(g_pool_mu);
+    Pool& q = g_pool[device];
+    q.trim(keep, out);
+    held = q.bytes;
+  }
+  for (void* p : out) (void)hipFree(p);
+  return held;
+}
+
 void* pool_alloc(size_t bytes, size_t* cap) {
   const size_t size = pool_class(bytes);
   const int dev = current_device();
   *cap = size;
   {
     std::lock_guard<std::mutex> g(g_pool_mu);
-    Pool& q = g_pool[dev];
-    auto f = q.free.find(size);
-    if (f != q.free.end()) {
-      void* p = f->second;
-      q.free.erase(f);
-      q.bytes -= size;
-      return p;
-    }
+    if (void* p = g_pool[dev].take(size)) return p;
   }
   void* p = nullptr;
   if (hipMalloc(&p, size) == hipSuccess) return p;
   (void)hipGetLastError();
-  std::multimap<size_t, void*> all;  // give the pooled memory back and try once more
-  {
-    std::lock_guard<std::mutex> g(g_pool_mu);
-    Pool& q = g_pool[dev];
-    all.swap(q.free);
-    q.bytes = 0;
-  }
-  for (auto& f : all) (void)hipFree(f.second);
+  pool_trim(dev, 0);  // give the pooled memory back and try once more
   if (hipMalloc(&p, size) == hipSuccess) return p;
   (void)hipGetLastError();
   return nullptr;
@@ -210,8 +241,7 @@ void pool_free(void* p, size_t cap) {
     std::lock_guard<std::mutex> g(g_pool_mu);
     Pool& q = g_pool[current_device()];
     if (q.bytes + cap <= kPoolMax) {
-      q.free.emplace(cap, p);
-      q.bytes += cap;
+      q.put(p, cap);
       return;
     }
   }
@@ -363,6 +393,17 @@ int ngpb_destroy(ngpb_ctx* c) {
     delete c;
   } else {
     delete c;
+  }
+  return NGPB_OK;
+}
+
+int ngpb_trim_pool(int device, int64_t keep_bytes, int64_t* held_bytes) {
+  if (device < 0 || keep_bytes < 0) return NGPB_E_ARG;
+  try {
+    const size_t held = ngpb::pool_trim(device, (size_t)keep_bytes);
+    if (held_bytes) *held_bytes = (int64_t)held;
+  } catch (const std::bad_alloc&) {
+    return NGPB_E_NOMEM;
   }
   return NGPB_OK;
 }

@@ -43,9 +43,11 @@ struct Error : std::runtime_error {
 // allocates gigabytes per request soon waits for the driver to clear the memory (160 ->
 // 395 ms per 8M-unknown request). A pooled block is idle: no stream has work pending on
 // it, whichever thread or stream takes it next. The pool holds at most 16 GiB per device
-// (more is freed) and gives everything back when an allocation fails.
+// (more is freed) and gives everything back when an allocation fails, or down to a given
+// size when ngpb_trim_pool asks for it.
 void* pool_alloc(size_t bytes, size_t* cap);  // nullptr: out of memory
 void pool_free(void* p, size_t cap);          // p must be idle
+size_t pool_trim(int device, size_t keep);    // frees the oldest blocks beyond `keep` bytes; bytes held then
 // While an object of this type lives, this thread's plain buffers are released to the
 // pool: their users have been waited for.
 struct IdleRelease {

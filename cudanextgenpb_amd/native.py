@@ -81,6 +81,7 @@ SIGNATURES = {
     "ngpb_device_count": (_I, [_P]),
     "ngpb_create": (_I, [_P, _I]),
     "ngpb_destroy": (_I, [_P]),
+    "ngpb_trim_pool": (_I, [_I, _I64, _P]),
     "ngpb_last_error": (ctypes.c_char_p, [_P]),
     "ngpb_constants": (_I, [_P, _P]),
     "ngpb_device_bytes": (_I, [_P, _P]),
@@ -170,6 +171,16 @@ def device_count() -> int:
     n = ctypes.c_int(0)
     lib().ngpb_device_count(ctypes.byref(n))
     return n.value
+
+
+def trim_pool(device: int = 0, keep_bytes: int = 0) -> int:
+    """Gives idle device blocks of closed contexts back to the driver, the oldest first,
+    until at most `keep_bytes` are held; returns the bytes held afterwards."""
+    held = ctypes.c_int64(0)
+    rc = lib().ngpb_trim_pool(int(device), int(keep_bytes), ctypes.byref(held))
+    if rc != NGPB_OK:
+        raise NGPBError(rc, f"trim_pool(device={device}, keep_bytes={keep_bytes})")
+    return held.value
 
 
 def constants(physics) -> dict:

@@ -127,6 +127,12 @@ const char* ngpb_version(void);
 int ngpb_device_count(int* count);
 int ngpb_create(ngpb_ctx** ctx, int device);
 int ngpb_destroy(ngpb_ctx* ctx);
+/* Destroyed contexts leave their device blocks, at most 16 GiB per device, to later
+   contexts of the process. This gives them back to the driver, the oldest first, until at
+   most keep_bytes are held, for other allocators of the process. *held_bytes (may be
+   NULL) receives the bytes held afterwards. Waits for the device; safe beside calls of
+   other threads. No counterpart in the reference. */
+int ngpb_trim_pool(int device, int64_t keep_bytes, int64_t* held_bytes);
 const char* ngpb_last_error(const ngpb_ctx* ctx);
 /* out[0..5] = eps_in_hat, eps_out_hat, k2 [A^-2], k [A^-1], constant_pol, constant_react
    (include/pb_class.h:47-54, src/pb_class.cpp:1800-1806, 2803-2814). Host only. */

@@ -39,6 +39,13 @@ def test_version_and_constants_host_only():
     assert c["k2"] == pytest.approx(1.537456096972e-2, rel=1e-12)
 
 
+def test_trim_pool_arguments():
+    assert native.trim_pool(0) == 0
+    for args in ((-1, 0), (0, -1)):
+        with pytest.raises(native.NGPBError):
+            native.trim_pool(*args)
+
+
 def test_constants_match_oracle():
     import oracle as O
 

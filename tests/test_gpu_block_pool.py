@@ -4,7 +4,8 @@ device buffers):
 * contexts made, used and destroyed from several threads at once, with sizes that
   alternate, give the potentials and energies of contexts that took fresh memory, bit for
   bit (reused blocks hold old data, so a buffer read before it is written would show);
-* the memory a process holds after many contexts is bounded by what its first ones needed.
+* the memory a process holds after many contexts is bounded by what its first ones needed;
+* trim_pool gives the idle blocks back to the driver, in part and in whole.
 """
 from concurrent.futures import ThreadPoolExecutor
 
@@ -51,3 +52,22 @@ def test_pool_does_not_grow():
         for S in (_spec(0), _spec(2)):
             _solve(S, native.PREC_MIXED, 1.4)
     assert free0 - _free_bytes(hip) < 64 * 2**20
+
+
+def test_pool_is_given_back():
+    hip = _hip()
+    big = _spec(2)
+    ref = _solve(big, native.PREC_MIXED, 1.4)
+    held = native.trim_pool(0, 1 << 60)
+    free0 = _free_bytes(hip)
+    assert held > 32 * 2**20
+    half = native.trim_pool(0, held // 2)
+    assert 0 < half <= held // 2
+    assert native.trim_pool(0, 1 << 60) == half
+    got = _solve(big, native.PREC_MIXED, 1.4)  # part of its blocks from the pool, part new
+    assert all(np.array_equal(a, b) for a, b in zip(got, ref))
+    assert native.trim_pool(0) == 0
+    # the driver rounds blocks; most of what was held must be free again
+    assert _free_bytes(hip) - free0 > held // 2
+    got = _solve(big, native.PREC_MIXED, 1.4)
+    assert all(np.array_equal(a, b) for a, b in zip(got, ref))
