@@ -6,7 +6,6 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <list>
 #include <map>
 #include <mutex>
 #include <sstream>
@@ -16,6 +15,7 @@
 #include <vector>
 
 #include "ngpb_internal.h"
+#include "ngpb_pool.h"
 
 namespace ngpb {
 
@@ -155,43 +155,8 @@ namespace ngpb {
 thread_local int IdleRelease::depth = 0;
 namespace {
 constexpr size_t kPoolMax = size_t(16) << 30;  // per device
-struct Pool {
-  struct Block {
-    size_t size;
-    void* p;
-  };
-  std::list<Block> blocks;                                   // oldest first
-  std::multimap<size_t, std::list<Block>::iterator> by_size;  // by size class
-  size_t bytes = 0;
-
-  void put(void* p, size_t size) {
-    by_size.emplace(size, blocks.insert(blocks.end(), Block{size, p}));
-    bytes += size;
-  }
-  void* take(size_t size) {
-    auto f = by_size.find(size);
-    if (f == by_size.end()) return nullptr;
-    void* p = f->second->p;
-    blocks.erase(f->second);
-    by_size.erase(f);
-    bytes -= size;
-    return p;
-  }
-  // moves the oldest blocks to `out` until at most `keep` bytes stay
-  void trim(size_t keep, std::vector<void*>& out) {
-    while (bytes > keep) {
-      auto b = blocks.begin();
-      auto f = by_size.lower_bound(b->size);
-      while (f->second != b) ++f;
-      by_size.erase(f);
-      bytes -= b->size;
-      out.push_back(b->p);
-      blocks.erase(b);
-    }
-  }
-};
 std::mutex g_pool_mu;
-std::unordered_map<int, Pool> g_pool;  // by device
+std::unordered_map<int, IdleBlocks> g_pool;  // by device
 
 size_t pool_class(size_t bytes) {
   size_t step = 512;
@@ -211,9 +176,9 @@ size_t pool_trim(int device, size_t keep) {
   size_t held = 0;
   {
     std::lock_guard<std::mutex> g(g_pool_mu);
-    Pool& q = g_pool[device];
+    IdleBlocks& q = g_pool[device];
     q.trim(keep, out);
-    held = q.bytes;
+    held = q.bytes();
   }
   for (void* p : out) (void)hipFree(p);
   return held;
@@ -237,15 +202,18 @@ void* pool_alloc(size_t bytes, size_t* cap) {
 }
 
 void pool_free(void* p, size_t cap) {
+  std::vector<void*> out;  // the oldest blocks, where this one needs their room
   {
     std::lock_guard<std::mutex> g(g_pool_mu);
-    Pool& q = g_pool[current_device()];
-    if (q.bytes + cap <= kPoolMax) {
+    if (cap > kPoolMax) {
+      out.push_back(p);
+    } else {
+      IdleBlocks& q = g_pool[current_device()];
+      q.trim(kPoolMax - cap, out);
       q.put(p, cap);
-      return;
     }
   }
-  (void)hipFree(p);
+  for (void* o : out) (void)hipFree(o);
 }
 
 // ---- per-stream cache of released stream-ordered blocks

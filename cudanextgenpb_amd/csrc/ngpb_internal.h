@@ -43,7 +43,7 @@ struct Error : std::runtime_error {
 // allocates gigabytes per request soon waits for the driver to clear the memory (160 ->
 // 395 ms per 8M-unknown request). A pooled block is idle: no stream has work pending on
 // it, whichever thread or stream takes it next. The pool holds at most 16 GiB per device
-// (more is freed) and gives everything back when an allocation fails, or down to a given
+// (the oldest blocks are freed for newer ones) and gives everything back when an allocation fails, or down to a given
 // size when ngpb_trim_pool asks for it.
 void* pool_alloc(size_t bytes, size_t* cap);  // nullptr: out of memory
 void pool_free(void* p, size_t cap);          // p must be idle
