@@ -80,6 +80,8 @@ struct BatchScal {
   int phase, stepped, cycle_start, iters, maxiter, repl, stagnant, status;
   int mg;           // 1: multigrid-preconditioned iterations
   int cycle_iters;  // iterations of the current inner cycle
+  int cycle_limit;  // iterations after which a multigrid cycle gives way to Jacobi scaling
+  int pending;      // 1: the last multigrid step is still to be added to xhat
 };
 
 struct Tile {
@@ -178,8 +180,8 @@ __global__ void __launch_bounds__(WPB * 64) kb_dir(const BatchDesc* __restrict__
   }
 }
 
-// x += S xhat, xhat = 0 (systems whose inner cycle ended; with mg the last step is still
-// to be added to xhat)
+// x += S xhat, xhat = 0 (systems whose inner cycle ended; after a multigrid cycle the last
+// step is still to be added to xhat)
 template <int WPB>
 __global__ void __launch_bounds__(WPB * 64) kb_accum(const BatchDesc* __restrict__ D, const BatchScal* __restrict__ S,
                                                      const Tile* __restrict__ tiles, int tile_slices) {
@@ -192,7 +194,7 @@ __global__ void __launch_bounds__(WPB * 64) kb_accum(const BatchDesc* __restrict
   for (int64_t s = (int64_t)tl.slice + wave; s < s1; s += WPB) {
     const int64_t i = s * kW + lane_id();
     if (i >= d.n) continue;
-    const float xi = S[slot].mg ? fmaf((float)S[slot].alpha, d.ps[i], d.xs[i]) : d.xs[i];
+    const float xi = S[slot].pending ? fmaf((float)S[slot].alpha, d.ps[i], d.xs[i]) : d.xs[i];
     d.x[i] += d.dscale[i] * (double)xi;
     d.xs[i] = 0.f;
   }
@@ -396,10 +398,9 @@ __global__ void __launch_bounds__(kFinBS) kbm_fin_rz(const BatchDesc* __restrict
   }
 }
 
-// Stop test of a multigrid iteration. A cycle that does not converge within
-// kMgCycleIters iterations, or a residual that is not finite, starts the system again
-// with Jacobi scaling.
-constexpr int kMgCycleIters = 100;
+// Stop test of a multigrid iteration. After a cycle that does not converge within its
+// limit the system goes on from its x with Jacobi scaling; after a residual that is not
+// finite it starts again from x = 0 with it. Host code moves it to the other tile list.
 __global__ void __launch_bounds__(kFinBS) kbm_fin_rr(const BatchDesc* __restrict__ D, BatchScal* __restrict__ S) {
   __shared__ double lds[kFinBS / 64];
   BatchScal& sc = S[blockIdx.x];
@@ -410,13 +411,18 @@ __global__ void __launch_bounds__(kFinBS) kbm_fin_rr(const BatchDesc* __restrict
   sc.iters = it;
   sc.rr = RR;
   sc.cycle_iters += 1;
-  if (!(RR > sc.stop_rr) && RR == RR) {
-    sc.phase = kReplace;
-  } else if (!(RR < INFINITY) || (sc.cycle_iters >= kMgCycleIters && it < sc.maxiter)) {
+  if (!(RR < INFINITY)) {
     sc.mg = 0;
     sc.phase = kJoin;
-  } else if (it >= sc.maxiter) {
-    sc.phase = kReplace;
+    return;
+  }
+  const bool stop = !(RR > sc.stop_rr) || it >= sc.maxiter;
+  if (!stop && sc.cycle_iters < sc.cycle_limit) return;
+  sc.phase = kReplace;
+  sc.pending = 1;
+  if (!stop) {
+    sc.mg = 0;
+    sc.rho = 0.0;  // no direction to go on with
   }
 }
 
@@ -458,12 +464,12 @@ __global__ void __launch_bounds__(kFinBS) kb_fin_resid(const BatchDesc* __restri
     BB = dev::block_sum<kFinBS>(s, lds);
   }
   if (threadIdx.x != 0) return;
+  const bool handover = sc.pending && !sc.mg;  // the end of its last multigrid cycle
+  sc.pending = 0;
   sc.stepped = 0;
   if (ph == kJoin) {
     sc.bb = BB;
     sc.target = sc.tol * sc.tol * BB;
-    sc.iters = 0;
-    sc.repl = 0;
     sc.stagnant = 0;
     sc.prev_true = BB;
     sc.beta = 0.0;
@@ -488,12 +494,25 @@ __global__ void __launch_bounds__(kFinBS) kb_fin_resid(const BatchDesc* __restri
     sc.phase = kDone;
     return;
   }
-  if (ph == kReplace) {
+  if (handover) {
+    if (!(RR < sc.bb)) {  // x = 0 is the better start
+      sc.phase = kJoin;
+      return;
+    }
+    sc.stagnant = 0;
+    sc.prev_true = RR;
+  } else if (ph == kReplace) {
     // the FP32 inner solve no longer reduces the FP64 residual
     if (!(RR <= 0.81 * sc.prev_true)) {
       if (++sc.stagnant >= 3 && sc.mg) {
+        // Jacobi scaling from here, once the system is in its tile list: the replacement
+        // step is repeated there (and counted once), or x = 0 is the better start
         sc.mg = 0;
-        sc.phase = kJoin;
+        sc.rho = 0.0;
+        sc.stagnant = 0;
+        sc.prev_true = INFINITY;
+        sc.repl -= 1;
+        sc.phase = RR < sc.bb ? kReplace : kJoin;
         return;
       }
       if (sc.stagnant >= 3) {
@@ -925,6 +944,7 @@ int ngpb_batch_add(ngpb_batch* b, ngpb_ctx* c, int* slot) {
     ngpb::BatchScal sc;
     std::memset(&sc, 0, sizeof(sc));
     sc.mg = mg ? 1 : 0;
+    sc.cycle_limit = c->mg_cycle_iters;
     sc.phase = ngpb::kJoin;
     sc.tol = b->tol;
     sc.drop = b->drop;

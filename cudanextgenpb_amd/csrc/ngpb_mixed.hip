@@ -1422,7 +1422,8 @@ double time_spmv_compact(ngpb_ctx* c, int reps) {
 // Solves with the multigrid preconditioner where it applies (mg_setup): an inner cycle
 // is then CG preconditioned by one V-cycle, 20-30 iterations in all against 300-900 with
 // Jacobi scaling alone. Should the cycle not converge (mg_cycle_iters iterations, or a
-// non-finite residual), the solve goes on with the Jacobi-scaled CG.
+// non-finite residual), or the cycles stagnate, the solve goes on with the Jacobi-scaled
+// CG: from its x where that has a smaller residual than x = 0, otherwise from x = 0.
 void solve_mixed(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
   const int64_t n = c->n;
   check_operator(c);
@@ -1537,14 +1538,19 @@ void solve_mixed(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
       bool mg_failed = false;
       if (mg) {
         mg_rho = h->rho2[(cycle_start + cycle_iters) & 1];
-        mg_failed = !std::isfinite(h->rr) || (h->rr > h->stop_rr && iters < o.maxiter);
+        mg_failed = h->rr > h->stop_rr && iters < o.maxiter;
         ahead = std::max(2, cycle_iters + 1);
       }
-      if (mg && !std::isfinite(h->rr)) {  // start over without the preconditioner
+      auto start_over = [&] {
         mg = false;
         start_jacobi();
         read_scalars();
         true_rr = h->aux[0];
+        prev_true = bb;
+        stagnant = 0;
+      };
+      if (mg && !std::isfinite(h->rr)) {
+        start_over();
         continue;
       }
       // FP64 residual replacement
@@ -1572,7 +1578,12 @@ void solve_mixed(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
       }
       prev_true = std::min(prev_true, true_rr);
       if (mg && (mg_failed || stalled)) {
+        if (!(true_rr < bb)) {
+          start_over();
+          continue;
+        }
         mg = false;
+        prev_true = true_rr;
         stagnant = 0;
         h->beta = 0.0;
       } else if (stalled) {

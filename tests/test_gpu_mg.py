@@ -133,3 +133,57 @@ def test_host_mesh_equals_device_mesh():
         p.ctx.close()
     assert out[0][1]["iterations"] == out[1][1]["iterations"] <= 60
     assert np.array_equal(out[0][0], out[1][0])
+
+
+def solve_batch(ctxs, maxiter=100000, inner=8):
+    """Potentials and statistics of the contexts solved in one batch, and its replays."""
+    with native.Batch(0, max_systems=len(ctxs), tol=1e-10, maxiter=maxiter, inner_per_replay=inner) as b:
+        slots = [b.add(c) for c in ctxs]
+        replays = b.solve_all(5000)
+        out = []
+        for s, c in zip(slots, ctxs):
+            done, st = b.status(s)
+            assert done
+            b.remove(s)
+            out.append((c.get_phi(), st))
+    return out, replays
+
+
+def test_cycle_that_does_not_converge():
+    """A limit on the iterations of a cycle ends it early: the solve goes on from its x
+    with Jacobi scaling, within the iteration limit of the whole solve, and other systems
+    of a batch are not touched by it."""
+    p = prepare(box_spec((48, 48, 48), levels=2, bands=(1.0, 2.5)))
+    other = prepare(box_spec((17, 33, 16)))
+    phi64, _ = p.ctx.solve(native.PREC_FP64, tol=1e-12)
+
+    def close(phi):
+        return np.linalg.norm(phi - phi64) <= 1e-8 * np.linalg.norm(phi64)
+
+    p.ctx.set_multigrid(cycle_iters=0)
+    _, jac = p.ctx.solve(native.PREC_MIXED, tol=1e-10)
+    [(_, jac_b)], _ = solve_batch([p.ctx])
+    [(ref_other, _)], _ = solve_batch([other.ctx])
+    for limit in (1, 3, 5):
+        p.ctx.set_multigrid(cycle_iters=limit)
+        phi, st = p.ctx.solve(native.PREC_MIXED, tol=1e-10)
+        [(alone, sa)], _ = solve_batch([p.ctx])
+        [(mix, sm), (phi_other, _)], _ = solve_batch([p.ctx, other.ctx])
+        print(f"[mg] cycles of {limit}: {st['iterations']} it, batch {sa['iterations']} it "
+              f"(Jacobi {jac['iterations']} and {jac_b['iterations']})", flush=True)
+        assert p.ctx.multigrid_info()["in_use"]
+        for f, s in ((phi, st), (alone, sa), (mix, sm)):
+            assert s["status"] == 0 and s["relres"] <= 1e-10 and close(f)
+        assert np.array_equal(alone, mix) and sa["iterations"] == sm["iterations"]
+        assert np.array_equal(phi_other, ref_other)
+        if limit > 1:  # what the first cycle gained is kept
+            assert limit < st["iterations"] < jac["iterations"] + limit
+            assert limit < sa["iterations"] < jac_b["iterations"] + limit
+        # the iterations of the ended cycle count towards the limit
+        _, s20 = p.ctx.solve(native.PREC_MIXED, tol=1e-10, maxiter=20, raise_on_noconv=False)
+        [(_, b20)], replays = solve_batch([p.ctx], maxiter=20, inner=1)
+        for s in (s20, b20):
+            assert s["status"] == 4 and s["iterations"] == 20
+        assert replays <= 20 + b20["replacements"] + 2
+    p.ctx.close()
+    other.ctx.close()
