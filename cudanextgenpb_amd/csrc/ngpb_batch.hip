@@ -1113,7 +1113,7 @@ int ngpb_batch_status(ngpb_batch* b, int slot, int* done, ngpb_solve_stats* st) 
       st->replacements = sc.repl;
       st->relres = sc.bb > 0.0 ? std::sqrt(sc.true_rr / sc.bb) : 0.0;
       st->ms_solve = 0.0;
-      st->bytes_per_iter = ngpb::spmv_compact_bytes(c) + (double)c->n * 4.0 * 8.0;
+      st->bytes_per_iter = ngpb::mixed_bytes_per_iter(c, sc.mg != 0);
     }
   });
 }

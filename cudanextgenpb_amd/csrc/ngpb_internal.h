@@ -492,6 +492,7 @@ float* guarded_vector(ngpb_ctx* c, DBuf<float>& v);  // n entries between such g
 void spmv_compact(ngpb_ctx* c, const double* x, double* y);
 void solve_mixed(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st);
 double spmv_compact_bytes(const ngpb_ctx* c);
+double mixed_bytes_per_iter(const ngpb_ctx* c, bool mg);  // algorithmic bytes of one iteration
 double time_spmv_compact(ngpb_ctx* c, int reps);
 
 // multigrid preconditioner (ngpb_mg.hip): one CG iteration runs an SpMV on r,

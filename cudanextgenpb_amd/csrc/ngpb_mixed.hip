@@ -1398,6 +1398,16 @@ void spmv_compact(ngpb_ctx* c, const double* x, double* y) {
   NGPB_HIP(hipGetLastError());
 }
 
+// SpMV + update (rhat, q read; rhat written) + direction (rhat, p, xhat read; p, xhat
+// written); with the preconditioner three SpMVs, the vector streams of its four row
+// kernels (20 x 4 bytes) and the uniform levels (the dense array read once, then some 100
+// bytes per node of the first level and an eighth of that for each further one)
+double mixed_bytes_per_iter(const ngpb_ctx* c, bool mg) {
+  const double spmv = spmv_compact_bytes(c), n = (double)c->n;
+  if (!mg) return spmv + n * 4.0 * (3.0 + 5.0);
+  return 3.0 * spmv + n * 4.0 * 20.0 + 4.0 * (double)c->mg_dense.n + 115.0 * (double)c->mg.lev[0].nodes();
+}
+
 double time_spmv_compact(ngpb_ctx* c, int reps) {
   if (!c->have_compact) build_compact(c);
   float* pin = spmv_input(c);
@@ -1602,13 +1612,7 @@ void solve_mixed(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
   st.replacements = repl;
   st.relres = bb > 0 ? std::sqrt(true_rr / bb) : 0.0;
   st.ms_solve = ms;
-  // SpMV + update (rhat, q read; rhat written) + direction (rhat, p, xhat read; p, xhat
-  // written); with the preconditioner three SpMVs, the vector streams of its four row
-  // kernels (20 x 4 bytes) and the uniform levels (the dense array twice, then some 100
-  // bytes per node of the first level and an eighth of that for each further one)
-  st.bytes_per_iter = mg ? 3.0 * spmv_compact_bytes(c) + (double)n * 80.0 + 4.0 * (double)c->mg_dense.n +
-                               115.0 * (double)c->mg.lev[0].nodes()
-                         : spmv_compact_bytes(c) + (double)n * 4.0 * (3.0 + 5.0);
+  st.bytes_per_iter = mixed_bytes_per_iter(c, mg);
   c->have_phi = true;
   c->phi_len = c->n;
 }

@@ -187,3 +187,16 @@ def test_cycle_that_does_not_converge():
         assert replays <= 20 + b20["replacements"] + 2
     p.ctx.close()
     other.ctx.close()
+
+
+def test_batch_reports_the_iteration_it_runs():
+    p = prepare(box_spec((17, 33, 16)))
+    seen = []
+    for cycles in (100, 0):
+        p.ctx.set_multigrid(cycle_iters=cycles)
+        _, st = p.ctx.solve(native.PREC_MIXED, tol=1e-10)
+        [(_, sb)], _ = solve_batch([p.ctx])
+        assert sb["bytes_per_iter"] == st["bytes_per_iter"]
+        seen.append(st["bytes_per_iter"])
+    assert seen[0] > 2 * seen[1]  # three products and the levels against one product
+    p.ctx.close()
