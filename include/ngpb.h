@@ -353,7 +353,9 @@ int ngpb_time_spmv(ngpb_ctx* ctx, int precision, int reps, double* ms_per_launch
 
 /* With profiling on, every SpMV launched by ngpb_solve is bracketed by HIP events on
    the context's stream; ngpb_kernel_stats returns the launch count, their summed time
-   and the algorithmic bytes of one launch for FP64 (CSR) or MIXED (compact) SpMV.
+   and the algorithmic bytes of one launch for FP64 (CSR) or MIXED (compact) SpMV. FP64
+   solves of up to 4,096 rows may run in one launch without separate SpMVs: as many are
+   timed after the solve instead. Results are the same with profiling on or off.
    Enabling or disabling resets the counters. No counterpart in the reference. */
 int ngpb_set_profiling(ngpb_ctx* ctx, int enable);
 int ngpb_kernel_stats(ngpb_ctx* ctx, int precision, int64_t* launches, double* total_ms,

@@ -16,6 +16,8 @@ import pytest
 import scipy.sparse as sp
 import scipy.sparse.linalg as spl
 
+from cudanextgenpb_amd import native
+
 from test_zz_no_alloc import hip, solve_noalloc
 
 pytestmark = pytest.mark.gpu
@@ -75,3 +77,22 @@ def test_more_iterations_than_one_launch():
     ref = np.where(i <= s, i * (n + 1 - s), s * (n + 1 - i)) / (n + 1)
     # condition number about 4 (n + 1)^2 / pi^2 = 6.5e6
     assert np.linalg.norm(x - ref) <= 6.5e6 * 1e-13 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("n,form", [(1000, "vary"), (4096, "full"), (4096, "over"), (4097, "vary")])
+def test_profiling_changes_no_result(n, form):
+    """Solves in one block and solves of three launches per iteration, with products timed
+    and without."""
+    rng = np.random.default_rng(n)
+    A = system(n, form, rng)
+    with native.Context(0) as c:
+        c.set_csr(A.indptr, A.indices, A.data, rng.standard_normal(n))
+        ref, st = c.solve(native.PREC_FP64, tol=1e-13)
+        c.set_profiling(True)
+        got, sp_ = c.solve(native.PREC_FP64, tol=1e-13)
+        k = c.kernel_stats(native.PREC_FP64)
+        c.set_profiling(False)
+        again, _ = c.solve(native.PREC_FP64, tol=1e-13)
+    assert np.array_equal(got, ref) and np.array_equal(again, ref)
+    assert {**sp_, "ms_solve": 0} == {**st, "ms_solve": 0}
+    assert k["launches"] == (st["iterations"] + 3) // 8 and k["total_ms"] > 0.0
