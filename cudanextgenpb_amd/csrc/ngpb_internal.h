@@ -341,7 +341,7 @@ struct ngpb_ctx {
   ngpb::DBuf<uint32_t> mg_pos;
   int spmv_sched = 6;                // SpMV work schedule (0 .. 6)
   int sell_resident = 0;             // resident blocks of the compact SpMV (0: not yet queried)
-  int csr_resident = 0;              // resident blocks of the FP64 CSR SpMV (0: not yet queried)
+  int csr_resident[2] = {0, 0};      // resident blocks of the FP64 SpMV from CSR / records (0: not yet queried)
 
   // solver state
   ngpb::DBuf<double> x, r, z, p, q, dinv;
@@ -460,16 +460,17 @@ OctreeSizes run_build_octree_surface(ngpb_ctx* c, const double* origin, double h
 
 // Krylov
 unsigned vec_grid(int64_t n);
+// 1 / diagonal into c->dinv; throws on NaN or Inf entries and non-positive diagonals
 void check_operator(ngpb_ctx* c);
 void ensure_reduce(ngpb_ctx* c, int64_t blocks);
-// FP64 CSR SpMV y = A x that also writes per-block (x, y) partials and returns at once
-// once the stop flag of c->ks is raised; grid size of its launches
-// FP64 CSR products by per-slice diagonals: check_operator, and the system's records,
-// built anew on each call; *block: the system suits the one-block CG
+// check_operator, and the diagonals of each 64-row slice, built anew on each call, for
+// the FP64 products of a solve; null where products from the CSR alone are faster.
+// *block: the system suits the one-block CG
 const void* slice_records(ngpb_ctx* c, bool* block);
+// FP64 SpMV y = A x that also writes per-block (x, y) partials and returns at once once
+// the stop flag of c->ks is raised; grid size of its launches. rec: slice_records
 void spmv_fp64_dot(ngpb_ctx* c, const double* x, double* y, double* partials, const void* rec);
-unsigned spmv_fp64_grid(ngpb_ctx* c);
-void check_operator(ngpb_ctx* c);
+unsigned spmv_fp64_grid(ngpb_ctx* c, const void* rec);
 // other LIS solvers (ngpb_lis.hip)
 void check_lis_options(const ngpb_solve_opts& o);
 void solve_lis(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st);

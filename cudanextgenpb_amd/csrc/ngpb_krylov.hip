@@ -37,12 +37,16 @@ constexpr int kFin = 1024;  // finalize block size
 // range of chunks, with blocks renumbered so that the blocks on one XCD (block id
 // mod 8) cover one contiguous eighth of the rows (L2 reuse of the x gathers); the
 // grid is then the number of blocks resident at once.
-template <int SCHED>
+template <bool DOT, int SCHED>
 __global__ void __launch_bounds__(kBS) k_spmv64(int64_t n, const int32_t* __restrict__ rowptr,
                                                  const int32_t* __restrict__ col, const double* __restrict__ val,
-                                                 const double* __restrict__ x, double* __restrict__ y) {
+                                                 const double* __restrict__ x, double* __restrict__ y,
+                                                 const KrylovScalars* ks, double* __restrict__ partials) {
   __shared__ double s_val[kCap];
   __shared__ double s_x[kCap];
+  __shared__ double s_red[kBS / 64];
+  if (DOT && ks->done) return;
+  double part = 0.0;
   const int64_t nchunks = (n + kBS - 1) / kBS;
   int64_t c_begin = blockIdx.x, c_end = nchunks, c_step = gridDim.x;
   if (SCHED == 1) {
@@ -89,6 +93,11 @@ __global__ void __launch_bounds__(kBS) k_spmv64(int64_t n, const int32_t* __rest
       for (int64_t k = kb; k < ke; ++k) sum = fma(s_val[k - p0], s_x[k - p0], sum);
     }
     if (row < n) y[row] = sum;
+    if (DOT && row < n) part += x[row] * sum;
+  }
+  if (DOT) {
+    part = dev::block_sum<kBS>(part, s_red);
+    if (threadIdx.x == 0) partials[blockIdx.x] = part;
   }
 }
 
@@ -114,13 +123,23 @@ struct SliceRec {
 };
 static_assert(sizeof(SliceRec) == 288, "SliceRec is 288 bytes");
 
-// one wave per slice; at up to kBlockRows rows bit 8 of *flags is set when a slice has
-// more than kDiags diagonals
+// Whether the products of a system use its records: `staged` of its slices have none. Up
+// to 2^18 rows a wave has one slice, and the slowest slice is the product: only without
+// staged ones. From 2^19 rows on, where waves have several, up to two thirds of them, and
+// in between the line runs straight. Per iteration with records and from the CSR alone:
+// 27,000 rows, 18% staged: 13.9 and 12.3 us; 216,000, none: 17.0 and 18.2, 24%: 19.4 and
+// 18.4; 421,875, 23%: 25.9 and 27.3, 69%: 28.5 and 27.4; 1 million, 58%: 44.5 and 47.4,
+// 85%: 48.9 and 47.5. Rows without any pattern of 183 entries: 443 us a product and 285.
+bool use_records(int64_t n, int64_t staged) {
+  const int64_t lo = int64_t(1) << 18, slices = (n + 63) / 64;
+  return 3 * lo * staged <= 2 * slices * std::clamp<int64_t>(n - lo, 0, lo);
+}
+
+// one wave per slice; flags[1] counts the slices with more than kDiags diagonals
 __global__ void __launch_bounds__(kBS) k_slice_rec(int64_t n, const int32_t* __restrict__ rowptr,
                                                    const int32_t* __restrict__ col, const double* __restrict__ val,
                                                    SliceRec* __restrict__ recs, int* __restrict__ flags) {
   const int64_t s = (int64_t)blockIdx.x * (kBS / 64) + (threadIdx.x >> 6);
-  if (s * 64 >= n) return;
   const int lane = threadIdx.x & 63;
   const int64_t row = s * 64 + lane;
   int64_t e = 0, end = 0;
@@ -155,11 +174,12 @@ __global__ void __launch_bounds__(kBS) k_slice_rec(int64_t n, const int32_t* __r
     if (has) ++e;
     ++k;
   }
-  if (lane == 0) {
+  if (lane == 0 && s * 64 < n) {
     R.count = k;
     R.vary = vary;
-    if (k < 0 && n <= kBlockRows) atomicOr(flags, 8);
   }
+  const int staged = __syncthreads_count(lane == 0 && k < 0);
+  if (staged && threadIdx.x == 0) atomicAdd(flags + 1, staged);
 }
 
 // k_spmv64 from slice records: the same rows per thread and the same partial sums. A
@@ -452,23 +472,29 @@ void run_pcg_block(hipStream_t s, int64_t n, const int32_t* rowptr, const double
   }
 }
 
-unsigned spmv64_grid(ngpb_ctx* c) {
+unsigned spmv64_grid(ngpb_ctx* c, bool records) {
   const int64_t need = std::max<int64_t>(1, (c->n + kBS - 1) / kBS);
   if (c->spmv_sched == 0) return (unsigned)std::min<int64_t>(need, 2048);
-  if (c->csr_resident <= 0) {
+  int& resident = c->csr_resident[records];
+  if (resident <= 0) {
     int cus = 0, per_cu = 0;
     NGPB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
-    NGPB_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_spmv64_rec<1>, kBS, 0));
-    c->csr_resident = std::max(8, (std::max(cus, 1) * std::max(per_cu, 1)) / 8 * 8);
+    if (records) NGPB_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_spmv64_rec<1>, kBS, 0));
+    else NGPB_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (k_spmv64<true, 1>), kBS, 0));
+    resident = std::max(8, (std::max(cus, 1) * std::max(per_cu, 1)) / 8 * 8);
   }
-  if (need >= c->csr_resident) return (unsigned)c->csr_resident;
+  if (need >= resident) return (unsigned)resident;
   return (unsigned)(c->spmv_sched == 1 ? (need + 7) / 8 * 8 : need);
 }
 
-// y = A x from the slice records, with the (x, y) partials
-void launch_spmv64_rec(ngpb_ctx* c, unsigned grid, const double* x, double* y, double* part, const void* rec) {
+// y = A x with the (x, y) partials, from the slice records or (rec null) the CSR
+void launch_product(ngpb_ctx* c, unsigned grid, const double* x, double* y, double* part, const void* rec) {
   const SliceRec* R = static_cast<const SliceRec*>(rec);
-  if (c->spmv_sched == 1)
+  if (!R && c->spmv_sched == 1)
+    spmv_launch(c, k_spmv64<true, 1>, dim3(grid), dim3(kBS), c->n, c->rowptr.p, c->col.p, c->val.p, x, y, c->ks.p, part);
+  else if (!R)
+    spmv_launch(c, k_spmv64<true, 0>, dim3(grid), dim3(kBS), c->n, c->rowptr.p, c->col.p, c->val.p, x, y, c->ks.p, part);
+  else if (c->spmv_sched == 1)
     spmv_launch(c, k_spmv64_rec<1>, dim3(grid), dim3(kBS), c->n, c->rowptr.p, c->col.p, c->val.p, R, x, y, c->ks.p, part);
   else
     spmv_launch(c, k_spmv64_rec<0>, dim3(grid), dim3(kBS), c->n, c->rowptr.p, c->col.p, c->val.p, R, x, y, c->ks.p, part);
@@ -698,12 +724,13 @@ void ensure_reduce(ngpb_ctx* c, int64_t blocks) {
 }
 
 namespace {
-// 1 / diagonal, its checks and, if asked for, the slice records; returns the flags
+// 1 / diagonal, its checks and, if asked for, the slice records; returns how many slices
+// have none
 int check_operator_records(ngpb_ctx* c, bool records) {
   c->dinv.resize((size_t)c->n);
   DBuf<int> bad;
-  bad.resize(1);
-  NGPB_HIP(hipMemsetAsync(bad.p, 0, sizeof(int), c->stream));
+  bad.resize(2);
+  NGPB_HIP(hipMemsetAsync(bad.p, 0, 2 * sizeof(int), c->stream));
   hipLaunchKernelGGL(k_diag_inv, dim3(blocks_for(c->n, 256)), dim3(256), 0, c->stream, c->n, c->rowptr.p, c->col.p,
                      c->val.p, c->dinv.p, bad.p);
   if (records) {
@@ -713,20 +740,20 @@ int check_operator_records(ngpb_ctx* c, bool records) {
                        c->col.p, c->val.p, reinterpret_cast<SliceRec*>(c->slice_rec.p), bad.p);
   }
   NGPB_HIP(hipGetLastError());
-  int hb = 0;
-  NGPB_HIP(hipMemcpyAsync(&hb, bad.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  int hb[2] = {0, 0};
+  NGPB_HIP(hipMemcpyAsync(hb, bad.p, sizeof(hb), hipMemcpyDeviceToHost, c->stream));
   NGPB_HIP(hipStreamSynchronize(c->stream));
-  NGPB_REQUIRE(!(hb & 2), NGPB_E_NUMERIC, "operator holds NaN or Inf entries");
-  NGPB_REQUIRE(!(hb & 1), NGPB_E_NUMERIC, "operator has a zero or negative diagonal entry");
-  return hb;
+  NGPB_REQUIRE(!(hb[0] & 2), NGPB_E_NUMERIC, "operator holds NaN or Inf entries");
+  NGPB_REQUIRE(!(hb[0] & 1), NGPB_E_NUMERIC, "operator has a zero or negative diagonal entry");
+  return hb[1];
 }
 }  // namespace
 
 void spmv_fp64_dot(ngpb_ctx* c, const double* x, double* y, double* partials, const void* rec) {
-  launch_spmv64_rec(c, spmv64_grid(c), x, y, partials, rec);
+  launch_product(c, spmv64_grid(c, rec != nullptr), x, y, partials, rec);
 }
 
-unsigned spmv_fp64_grid(ngpb_ctx* c) { return spmv64_grid(c); }
+unsigned spmv_fp64_grid(ngpb_ctx* c, const void* rec) { return spmv64_grid(c, rec != nullptr); }
 
 double spmv_fp64_bytes(const ngpb_ctx* c) {
   // nnz (value + column) + row pointers + x read + y written
@@ -734,11 +761,13 @@ double spmv_fp64_bytes(const ngpb_ctx* c) {
 }
 
 void spmv_fp64(ngpb_ctx* c, const double* x, double* y) {
-  const unsigned grid = spmv64_grid(c);
+  const unsigned grid = spmv64_grid(c, false);
+  const KrylovScalars* ks = nullptr;
+  double* part = nullptr;
   if (c->spmv_sched == 1)
-    spmv_launch(c, k_spmv64<1>, dim3(grid), dim3(kBS), c->n, c->rowptr.p, c->col.p, c->val.p, x, y);
+    spmv_launch(c, k_spmv64<false, 1>, dim3(grid), dim3(kBS), c->n, c->rowptr.p, c->col.p, c->val.p, x, y, ks, part);
   else
-    spmv_launch(c, k_spmv64<0>, dim3(grid), dim3(kBS), c->n, c->rowptr.p, c->col.p, c->val.p, x, y);
+    spmv_launch(c, k_spmv64<false, 0>, dim3(grid), dim3(kBS), c->n, c->rowptr.p, c->col.p, c->val.p, x, y, ks, part);
   NGPB_HIP(hipGetLastError());
 }
 
@@ -764,9 +793,9 @@ double time_spmv_fp64(ngpb_ctx* c, int reps) {
 void check_operator(ngpb_ctx* c) { (void)check_operator_records(c, false); }
 
 const void* slice_records(ngpb_ctx* c, bool* block) {
-  const int flags = check_operator_records(c, true);
-  if (block) *block = c->n <= kBlockRows && !(flags & 8);
-  return c->slice_rec.p;
+  const int staged = check_operator_records(c, true);
+  if (block) *block = c->n <= kBlockRows && !staged;
+  return use_records(c->n, staged) ? c->slice_rec.p : nullptr;
 }
 
 namespace {
@@ -779,7 +808,7 @@ void time_products(ngpb_ctx* c, unsigned grid, double* part, const void* rec) {
   NGPB_HIP(hipMemcpyAsync(c->ks.p, &h, sizeof(h), hipMemcpyHostToDevice, c->stream));
   for (int64_t k = kProfEvery / 2; k < h.iter; k += kProfEvery) {
     prof_begin(c, 0, k);
-    launch_spmv64_rec(c, grid, c->p.p, c->q.p, part, rec);
+    launch_product(c, grid, c->p.p, c->q.p, part, rec);
     prof_end(c, 0);
   }
   NGPB_HIP(hipGetLastError());
@@ -797,7 +826,7 @@ void solve_fp64(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
   c->r.resize((size_t)n);
   c->p.reserve((size_t)n);
   c->q.reserve((size_t)n);
-  const unsigned gs = spmv64_grid(c), gv = vec_grid(n);
+  const unsigned gs = spmv64_grid(c, rec != nullptr), gv = vec_grid(n);
   ensure_reduce(c, std::max<int64_t>(gs, 2048) + 2 * (int64_t)gv);
   double* part = c->red.partials.p;
   KrylovScalars* ks = c->ks.p;
@@ -825,7 +854,7 @@ void solve_fp64(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
       for (int k = 0; k < chunk; ++k, ++launch) {
         const int par = (int)(launch & 1);
         prof_begin(c, 0, launch);
-        launch_spmv64_rec(c, gs, c->p.p, c->q.p, ppq, rec);
+        launch_product(c, gs, c->p.p, c->q.p, ppq, rec);
         prof_end(c, 0);
         hipLaunchKernelGGL(k_pcg_update, dim3(gv), dim3(kBS), 0, c->stream, n, c->dinv.p, c->r.p, c->q.p, ks, ppq, (int)gs, pup, par);
         hipLaunchKernelGGL(k_pcg_dir, dim3(gv), dim3(kBS), 0, c->stream, n, c->dinv.p, c->x.p, c->r.p, c->p.p, ks, pup,
@@ -877,7 +906,7 @@ constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 double* g_scratch_ptr[kMaxDevices] = {};
 
-__global__ void k_clear_int(int* p) { *p = 0; }
+__global__ void k_clear_flags(int* p) { p[threadIdx.x] = 0; }
 
 // Structure of a CSR the library did not build: row pointers from 0 to nnz, non-
 // decreasing, columns in [0, n). Sets bit 4 of *bad otherwise; reads col only below nnz.
@@ -927,23 +956,23 @@ void solve_csr_noalloc(int device, hipStream_t s, int64_t n, int64_t nnz, const 
   KrylovScalars* ks = reinterpret_cast<KrylovScalars*>(part + kNoAllocPartials);
   int* bad = reinterpret_cast<int*>(ks + 1);
   SliceRec* recs = reinterpret_cast<SliceRec*>(part + kNoAllocPartials + 64);
-  static_assert(sizeof(KrylovScalars) + sizeof(int) <= 64 * sizeof(double), "scalar area too small");
+  static_assert(sizeof(KrylovScalars) + 2 * sizeof(int) <= 64 * sizeof(double), "scalar area too small");
   const auto t0 = std::chrono::steady_clock::now();
-  hipLaunchKernelGGL(k_clear_int, dim3(1), dim3(1), 0, s, bad);
+  hipLaunchKernelGGL(k_clear_flags, dim3(1), dim3(2), 0, s, bad);
   hipLaunchKernelGGL(k_csr_check, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, nnz, rowptr, col, bad);
   NGPB_HIP(hipGetLastError());
-  int hb = 0;
-  NGPB_HIP(hipMemcpyAsync(&hb, bad, sizeof(int), hipMemcpyDeviceToHost, s));
+  int hb[2] = {0, 0};
+  NGPB_HIP(hipMemcpyAsync(hb, bad, sizeof(hb), hipMemcpyDeviceToHost, s));
   NGPB_HIP(hipStreamSynchronize(s));
-  NGPB_REQUIRE(!(hb & 4), NGPB_E_ARG, "row pointers must run from 0 to nnz without decreasing, columns in [0, n)");
+  NGPB_REQUIRE(!(hb[0] & 4), NGPB_E_ARG, "row pointers must run from 0 to nnz without decreasing, columns in [0, n)");
   hipLaunchKernelGGL(k_diag_inv, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, rowptr, col, val, dinv, bad);
   hipLaunchKernelGGL(k_slice_rec, dim3(blocks_for((n + 63) / 64, kBS / 64)), dim3(kBS), 0, s, n, rowptr, col, val, recs,
                      bad);
   NGPB_HIP(hipGetLastError());
-  NGPB_HIP(hipMemcpyAsync(&hb, bad, sizeof(int), hipMemcpyDeviceToHost, s));
+  NGPB_HIP(hipMemcpyAsync(hb, bad, sizeof(hb), hipMemcpyDeviceToHost, s));
   NGPB_HIP(hipStreamSynchronize(s));
-  NGPB_REQUIRE(!(hb & 2), NGPB_E_NUMERIC, "operator holds NaN or Inf entries");
-  NGPB_REQUIRE(!(hb & 1), NGPB_E_NUMERIC, "operator has a zero or negative diagonal entry");
+  NGPB_REQUIRE(!(hb[0] & 2), NGPB_E_NUMERIC, "operator holds NaN or Inf entries");
+  NGPB_REQUIRE(!(hb[0] & 1), NGPB_E_NUMERIC, "operator has a zero or negative diagonal entry");
   KrylovScalars h;
   std::memset(&h, 0, sizeof(h));
   const auto poll = [&]() {
@@ -951,7 +980,7 @@ void solve_csr_noalloc(int device, hipStream_t s, int64_t n, int64_t nnz, const 
     NGPB_HIP(hipStreamSynchronize(s));
     return h.done != 0;
   };
-  if (n <= kBlockRows && !(hb & 8)) {
+  if (n <= kBlockRows && !hb[1]) {
     run_pcg_block(s, n, rowptr, val, recs, dinv, b, x, r, p, ks, tol, maxiter, poll);
   } else {
     // the launch shapes of ngpb_solve under SpMV schedule 0
@@ -962,11 +991,15 @@ void solve_csr_noalloc(int device, hipStream_t s, int64_t n, int64_t nnz, const 
     hipLaunchKernelGGL(k_pcg_init, dim3(gv), dim3(kBS), 0, s, n, b, dinv, x, r, p, pup);
     hipLaunchKernelGGL(k_fin_init, dim3(1), dim3(kFin), 0, s, ks, pup, (int)gv, tol * tol, maxiter);
     NGPB_HIP(hipGetLastError());
+    const bool records = use_records(n, hb[1]);
     const int chunk = std::max(1, check_every);
     for (int64_t launch = 0;;) {
       for (int k = 0; k < chunk; ++k, ++launch) {
         const int par = (int)(launch & 1);
-        hipLaunchKernelGGL(k_spmv64_rec<0>, dim3(gs), dim3(kBS), 0, s, n, rowptr, col, val, recs, p, q, ks, ppq);
+        if (records)
+          hipLaunchKernelGGL(k_spmv64_rec<0>, dim3(gs), dim3(kBS), 0, s, n, rowptr, col, val, recs, p, q, ks, ppq);
+        else
+          hipLaunchKernelGGL((k_spmv64<true, 0>), dim3(gs), dim3(kBS), 0, s, n, rowptr, col, val, p, q, ks, ppq);
         hipLaunchKernelGGL(k_pcg_update, dim3(gv), dim3(kBS), 0, s, n, dinv, r, q, ks, ppq, (int)gs, pup, par);
         hipLaunchKernelGGL(k_pcg_dir, dim3(gv), dim3(kBS), 0, s, n, dinv, x, r, p, ks, pup, (int)gv, par);
       }

@@ -743,7 +743,7 @@ void solve_lis(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
   c->q.reserve((size_t)n);
   for (auto* b : {&c->lis_rt, &c->lis_u, &c->lis_v, &c->lis_ph, &c->lis_uh, &c->lis_t}) b->reserve((size_t)n);
   const unsigned gv = vec_grid(n);
-  const int64_t gs_region = std::max<int64_t>(spmv_fp64_grid(c), 2048);
+  const int64_t gs_region = std::max<int64_t>(spmv_fp64_grid(c, rec), 2048);
   ensure_reduce(c, gs_region + 2 * (int64_t)gv);
   double* spart = c->red.partials.p;             // SpMV (x, y) partials, stride 1
   double* dpart = c->red.partials.p + gs_region;  // vector partials, stride 2
@@ -751,7 +751,7 @@ void solve_lis(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
   double *x = c->x.p, *r = c->r.p, *p = c->p.p, *q = c->q.p, *z = c->z.p;
   double *rt = c->lis_rt.p, *u = c->lis_u.p, *v = c->lis_v.p, *ph = c->lis_ph.p, *uh = c->lis_uh.p, *t = c->lis_t.p;
   const dim3 G(gv), B(kBS), F(1), BF(kFin);
-  const int np = (int)gv, nsp = (int)spmv_fp64_grid(c);
+  const int np = (int)gv, nsp = (int)spmv_fp64_grid(c, rec);
   auto fin = [&](const double* part, int cnt, int stride, int what) {
     hipLaunchKernelGGL(k_lis_fin, F, BF, 0, c->stream, ks, part, cnt, stride, what, o.solver);
   };

@@ -4,9 +4,11 @@ Strictly diagonally dominant symmetric systems (condition number below 3) solved
 relative residual of 1e-13 by ngpb_solve_csr_noalloc: the relative error is then below
 3e-13 plus rounding. Sizes lie around the slice (64) and block (256) edges; the entries
 lie on few diagonals with one value each, on few diagonals with varying values, on
-exactly as many diagonals as a record holds and one more, or anywhere (more than one
-staged piece per slice). Up to 4,096 rows, on at most 14 diagonals, one block runs the whole CG
-with 1, 2 or 4 rows per thread, 1,024 iterations per launch.
+exactly as many diagonals as a record holds and one more, or anywhere. Up to 4,096 rows, on
+at most 14 diagonals, one block runs the whole CG with 1, 2 or 4 rows per thread, 1,024
+iterations per launch. Systems with slices that have no record are multiplied from the
+CSR up to 2^18 rows and where most slices are such; the largest sizes here have a third
+of them, around the rows from which records are used, and several staged pieces per slice.
 """
 import ctypes
 from types import SimpleNamespace
@@ -24,7 +26,12 @@ pytestmark = pytest.mark.gpu
 
 
 def system(n, form, rng):
-    if form == "random":  # about 17 entries a row, in no pattern
+    if form == "part":  # a grid, with rows in no pattern at its start
+        m = n // 8
+        i = np.concatenate([np.arange(n - d) for d in (1, 70, 4900)] + [rng.integers(0, m, 8 * m)])
+        j = np.concatenate([np.arange(d, n) for d in (1, 70, 4900)] + [rng.integers(0, m, 8 * m)])
+        v = -rng.uniform(0.5, 1.0, len(i))
+    elif form == "random":  # about 17 entries a row, in no pattern
         i, j = rng.integers(0, n, 8 * n), rng.integers(0, n, 8 * n)
         v = -rng.uniform(0.5, 1.0, 8 * n)
     else:
@@ -46,8 +53,9 @@ def system(n, form, rng):
     return A
 
 
-@pytest.mark.parametrize("form", ["constant", "vary", "full", "over", "random"])
-@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 257, 1000, 1025, 2049, 4096, 4097, 70001])
+@pytest.mark.parametrize("n,form", [(n, f) for n in (1, 63, 64, 65, 255, 257, 1000, 1025, 2049, 4096, 4097, 70001)
+                                    for f in ("constant", "vary", "full", "over", "random")] +
+                         [(n, "part") for n in (262145, 300000, 340000, 524288, 700001)])
 def test_forms(n, form):
     rng = np.random.default_rng(n)
     A = system(n, form, rng)
@@ -55,7 +63,7 @@ def test_forms(n, form):
     S = SimpleNamespace(n=n, rowptr=A.indptr, col=A.indices, val=A.data, rhs=b)
     rc, x, st = solve_noalloc(hip(), S, 1e-13)
     assert rc == 0 and st["status"] == 0
-    ref = spl.spsolve(A.tocsc(), b) if form != "random" else None
+    ref = spl.spsolve(A.tocsc(), b) if form not in ("random", "part") else None
     if ref is not None:
         assert np.linalg.norm(x - ref) <= 1e-12 * np.linalg.norm(ref)
     assert np.linalg.norm(A @ x - b) <= 1e-12 * np.linalg.norm(b)
