@@ -543,8 +543,10 @@ __global__ void __launch_bounds__(kFin) k_fin_init(KrylovScalars* ks, const doub
 
 // Iteration of parity par. Every block forms (p, q) from the SpMV partials in the
 // same fixed order, so all blocks use the same alpha = rho / (p, q).
-// r -= alpha q; per block (r, D^-1 r), (r, r)
-__global__ void __launch_bounds__(kBS) k_pcg_update(int64_t n, const double* __restrict__ dinv, double* __restrict__ r,
+// r -= alpha q; per block (r, D^-1 r), (r, r); with X x += alpha p
+template <bool X>
+__global__ void __launch_bounds__(kBS) k_pcg_update(int64_t n, const double* __restrict__ dinv, double* __restrict__ x,
+                                                    double* __restrict__ r, const double* __restrict__ p,
                                                     const double* __restrict__ q, KrylovScalars* ks,
                                                     const double* __restrict__ pq_part, int npq,
                                                     double* __restrict__ partials, int par) {
@@ -558,6 +560,7 @@ __global__ void __launch_bounds__(kBS) k_pcg_update(int64_t n, const double* __r
   }
   double rz = 0.0, rr = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * kBS + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBS) {
+    if (X) x[i] += alpha * p[i];
     const double ri = r[i] - alpha * q[i];
     r[i] = ri;
     rz += ri * (dinv[i] * ri);
@@ -571,16 +574,18 @@ __global__ void __launch_bounds__(kBS) k_pcg_update(int64_t n, const double* __r
   }
 }
 
-// x += alpha p (here, where p is read for its own update too), the stop test on ||r||^2
-// (every block decides alike), then beta = (r', z') / (r, z) and p = D^-1 r + beta p.
-// Block 0 records the scalars for the next iteration and the host. The last step is added
-// by the launch that raises the stop flag, so a block must not return on a flag that this
-// same launch writes: it tests halt2[par], which the launch before has written.
+// With X x += alpha p; the stop test on ||r||^2 (every block decides alike), then
+// beta = (r', z') / (r, z) and p = D^-1 r + beta p. Block 0 records the scalars for the
+// next iteration and the host. The last step may be added by the launch that raises the
+// stop flag, so a block must not return on a flag that this same launch writes: it tests
+// halt2[par], which the launch before has written.
+template <bool X>
 __global__ void __launch_bounds__(kBS) k_pcg_dir(int64_t n, const double* __restrict__ dinv, double* __restrict__ x,
                                                  const double* __restrict__ r, double* __restrict__ p, KrylovScalars* ks,
                                                  const double* __restrict__ part, int np, int par) {
   __shared__ double s_red[kBS / 64];
-  if (ks->halt2[par]) {
+  if (!X && ks->done) return;  // nothing is left to do on a stop
+  if (X && ks->halt2[par]) {
     if (blockIdx.x == 0 && threadIdx.x == 0) ks->halt2[par ^ 1] = 1;
     return;
   }
@@ -605,13 +610,34 @@ __global__ void __launch_bounds__(kBS) k_pcg_dir(int64_t n, const double* __rest
       ks->rho2[par ^ 1] = RZ;
     }
   }
+  if (!X && stop) return;
   const double alpha = ks->alpha2[par], beta = RZ / rho;
   for (int64_t i = (int64_t)blockIdx.x * kBS + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBS) {
     const double pi = p[i];
-    x[i] += alpha * pi;
+    if (X) x[i] += alpha * pi;
     if (!stop) p[i] = dinv[i] * r[i] + beta * pi;
   }
 }
+
+// The vector kernels of an iteration. Above kFuseRows bytes count, and x is added to
+// where p is read for its own update (k_pcg_dir: 80 bytes per row for both against 88).
+// Up to there, latency does, and the store of x hides behind the sums of k_pcg_update. Per
+// iteration, x in k_pcg_update and in k_pcg_dir: 8,000 rows 12.0 and 12.3 us, 27,000 12.7
+// and 13.0, 91,125 14.1 and 14.3, 421,875 28.0 and 28.1, 1 million 36.7 and 35.4; the two
+// kernels alone at 4 million 70.4 and 64.8.
+constexpr int64_t kFuseRows = int64_t(1) << 19;
+void launch_pcg_vectors(hipStream_t s, unsigned gv, int64_t n, const double* dinv, double* x, double* r, double* p,
+                        const double* q, KrylovScalars* ks, const double* pq_part, int npq, double* part, int par) {
+  const bool fuse = n > kFuseRows;
+  hipLaunchKernelGGL(fuse ? k_pcg_update<false> : k_pcg_update<true>, dim3(gv), dim3(kBS), 0, s, n, dinv, x, r, p, q, ks,
+                     pq_part, npq, part, par);
+  hipLaunchKernelGGL(fuse ? k_pcg_dir<true> : k_pcg_dir<false>, dim3(gv), dim3(kBS), 0, s, n, dinv, x, r, p, ks, part,
+                     (int)gv, par);
+}
+
+// update (r, q, dinv read; r written) and direction (dinv, r, p read; p written), and x and
+// once or twice p for x += alpha p
+double pcg_vector_bytes(int64_t n) { return (double)n * 8.0 * (n > kFuseRows ? 10.0 : 11.0); }
 
 __global__ void k_diag_inv(int64_t n, const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
                            const double* __restrict__ val, double* __restrict__ dinv, int* __restrict__ bad) {
@@ -856,9 +882,7 @@ void solve_fp64(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
         prof_begin(c, 0, launch);
         launch_product(c, gs, c->p.p, c->q.p, ppq, rec);
         prof_end(c, 0);
-        hipLaunchKernelGGL(k_pcg_update, dim3(gv), dim3(kBS), 0, c->stream, n, c->dinv.p, c->r.p, c->q.p, ks, ppq, (int)gs, pup, par);
-        hipLaunchKernelGGL(k_pcg_dir, dim3(gv), dim3(kBS), 0, c->stream, n, c->dinv.p, c->x.p, c->r.p, c->p.p, ks, pup,
-                           (int)gv, par);
+        launch_pcg_vectors(c->stream, gv, n, c->dinv.p, c->x.p, c->r.p, c->p.p, c->q.p, ks, ppq, (int)gs, pup, par);
       }
       NGPB_HIP(hipGetLastError());
       const bool done = poll();
@@ -879,8 +903,7 @@ void solve_fp64(ngpb_ctx* c, const ngpb_solve_opts& o, ngpb_solve_stats& st) {
   st.replacements = 0;
   st.relres = h.bb > 0 ? std::sqrt(h.rr / h.bb) : 0.0;
   st.ms_solve = ms;
-  // SpMV in CSR form + update (r, q, dinv read; r written) + direction (x, dinv, r, p read; x, p written)
-  st.bytes_per_iter = spmv_fp64_bytes(c) + (double)n * 8.0 * (4.0 + 6.0);
+  st.bytes_per_iter = spmv_fp64_bytes(c) + pcg_vector_bytes(n);
   c->have_phi = true;
   c->phi_len = c->n;
 }
@@ -1000,8 +1023,7 @@ void solve_csr_noalloc(int device, hipStream_t s, int64_t n, int64_t nnz, const 
           hipLaunchKernelGGL(k_spmv64_rec<0>, dim3(gs), dim3(kBS), 0, s, n, rowptr, col, val, recs, p, q, ks, ppq);
         else
           hipLaunchKernelGGL((k_spmv64<true, 0>), dim3(gs), dim3(kBS), 0, s, n, rowptr, col, val, p, q, ks, ppq);
-        hipLaunchKernelGGL(k_pcg_update, dim3(gv), dim3(kBS), 0, s, n, dinv, r, q, ks, ppq, (int)gs, pup, par);
-        hipLaunchKernelGGL(k_pcg_dir, dim3(gv), dim3(kBS), 0, s, n, dinv, x, r, p, ks, pup, (int)gv, par);
+        launch_pcg_vectors(s, gv, n, dinv, x, r, p, q, ks, ppq, (int)gs, pup, par);
       }
       NGPB_HIP(hipGetLastError());
       if (poll()) break;
@@ -1013,7 +1035,7 @@ void solve_csr_noalloc(int device, hipStream_t s, int64_t n, int64_t nnz, const 
   st.relres = h.bb > 0 ? std::sqrt(h.rr / h.bb) : 0.0;
   st.ms_solve = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   // SpMV (12 nnz + 4 (n + 1) + 16 n) + update and direction vector streams, as ngpb_solve
-  st.bytes_per_iter = 12.0 * (double)nnz + 4.0 * (double)(n + 1) + 16.0 * (double)n + (double)n * 8.0 * (4.0 + 6.0);
+  st.bytes_per_iter = 12.0 * (double)nnz + 4.0 * (double)(n + 1) + 16.0 * (double)n + pcg_vector_bytes(n);
 }
 
 }  // namespace ngpb
