@@ -21,7 +21,7 @@
 // sweep's vectors and entries are packed in that order and name neighbours by position.
 //
 // A sweep is a serial chain of levels (427 on a 255,000-row protein mesh, 600 rows each
-// on average), so its time is the chain's latency. Runs of levels of up to kNarrow rows
+// on average), so its time is the chain's latency. Runs of narrow levels (order_triangle)
 // go to one block (k_ssor_run), piece by piece (a piece: rows of one level that fit the
 // staging buffers): the next pieces' entries stream into LDS while one is solved, the
 // solution of the last kWindow positions stays in LDS, and pieces are separated by a
@@ -33,6 +33,7 @@
 // kernel launched after the stop flag returns at once, and the host polls the flag
 // every check_every iterations.
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -316,9 +317,20 @@ constexpr int kRunBS = 1024;
 constexpr int kPieceRows = 512;
 constexpr int kPieceEntries = 4 * (kRunBS - kPieceRows);
 constexpr int kWindow = 8192;  // positions kept in LDS (64 KB)
-// Widest level of a one-block run: four pieces, about 4 us, the time of a launch (5-6 us
-// per dependent level measured).
-constexpr int kNarrow = 2048;
+
+// Time of a level in 1/30 us: in a one-block run, a piece takes 1 us and 1/30 us for every
+// entry of its longest row; a launch takes its latency, more with long rows, most when all
+// rows are long; and a run that starts anew fills its pipeline. Measured with all levels
+// alike, in a run and launched: 256 rows of 4 entries 1.0 and 3.7 us; 1,024 of 4, 8, 16,
+// 32, 64: 2.7 and 4.0, 4.9 and 6.1, 12.7 and 12.4, 37 and 31, 105 and 65; 2,048 of 4, 8,
+// 16: 5.4 and 4.6, 9.5 and 6.8, 25 and 11. On octrees (rows of 3.5, the longest 9 to 13)
+// the plans found so are within 1% of a bound of 2,048 rows: 1.22 million rows 973 ms a
+// solve and 979, 2.2 million 1,557 and 1,564.
+constexpr int64_t piece_cost(int64_t longest) { return 30 + longest; }
+constexpr int64_t launch_cost(int64_t rows, int64_t entries, int64_t longest) {
+  return std::max(100 + 6 * longest, 28 * entries / rows - 45);
+}
+constexpr int64_t kRunStart = 150;
 
 // One triangle in level order: position k has the entries ptr[k] .. ptr[k + 1).
 struct Sweep {
@@ -550,8 +562,8 @@ __global__ void __launch_bounds__(kBS) k_ssor_gather(int64_t n, const int32_t* _
 }
 
 // A triangle in level order: rows (by falling entry count within a level, so that a
-// wave's rows are alike, then ascending), their positions, entry
-// offsets, and the launches of a sweep: pieces of narrow levels and single wide levels.
+// wave's rows are alike, then ascending), their positions, entry offsets, and the launches
+// of a sweep, runs of pieces and single levels, by the least total of the costs above.
 // cnt(i): entries of row i.
 template <class Cnt>
 void order_triangle(ngpb_ctx* c, ngpb_ctx::SsorTriangle& t, const std::vector<int32_t>& lev, int32_t nlev, Cnt&& cnt) {
@@ -572,13 +584,38 @@ void order_triangle(ngpb_ctx* c, ngpb_ctx::SsorTriangle& t, const std::vector<in
     pos[(size_t)i] = k;
   }
   for (size_t k = 0; k < n; ++k) ptr[k + 1] = ptr[k] + cnt((size_t)rows[k]);
+  auto piece_end = [&](int32_t k, int32_t b) {
+    int32_t e = k;
+    while (e < b && e - k < kPieceRows && ptr[(size_t)e + 1] - ptr[(size_t)k] <= kPieceEntries) ++e;
+    return e;
+  };
+  // least cost up to each level with it in a run (0) or launched (1), and the choice before
+  constexpr int64_t kNever = INT64_MAX / 4;
+  std::vector<std::array<int8_t, 2>> from((size_t)nlev);
+  int64_t cost[2] = {kRunStart, 0};  // before the first level: a run would start
+  for (int32_t l = 0; l < nlev; ++l) {
+    const int32_t a = first[(size_t)l], b = first[(size_t)l + 1];
+    const int64_t row = cnt((size_t)rows[(size_t)a]);  // the longest: rows come by falling count
+    int64_t in_run = kNever;
+    // a row has to fit a piece; and without any entry in the whole triangle (a diagonal
+    // operator) there is nothing to stage: k_ssor_run reads columns at clamped indices
+    if (row <= kPieceEntries && longest > 0) {
+      in_run = 0;
+      for (int32_t k = a; k < b; k = piece_end(k, b)) in_run += piece_cost(cnt((size_t)rows[(size_t)k]));
+    }
+    const int64_t go_on = cost[0], start = cost[1] + kRunStart, either = std::min(cost[0], cost[1]);
+    from[(size_t)l] = {(int8_t)(go_on <= start ? 0 : 1), (int8_t)(cost[0] < cost[1] ? 0 : 1)};
+    cost[0] = std::min({go_on, start, kNever}) + in_run;
+    cost[1] = either + launch_cost(b - a, ptr[(size_t)b] - ptr[(size_t)a], row);
+  }
+  std::vector<int8_t> launched((size_t)nlev);
+  for (int32_t l = nlev - 1, s = cost[0] < cost[1] ? 0 : 1; l >= 0; s = from[(size_t)l][(size_t)s], --l)
+    launched[(size_t)l] = (int8_t)s;
   t.runs.clear();
   std::vector<int32_t> pieces;
   for (int32_t l = 0; l < nlev; ++l) {
     const int32_t a = first[(size_t)l], b = first[(size_t)l + 1];
-    // without any entry (a diagonal operator) there is nothing to stage: k_ssor_run reads
-    // columns at clamped indices and needs one
-    if (b - a > kNarrow || longest > kPieceEntries || longest == 0) {
+    if (launched[(size_t)l]) {
       t.runs.push_back({a, b, false});
       continue;
     }
@@ -586,12 +623,7 @@ void order_triangle(ngpb_ctx* c, ngpb_ctx::SsorTriangle& t, const std::vector<in
       t.runs.push_back({(int32_t)pieces.size(), (int32_t)pieces.size(), true});
       pieces.push_back(a);
     }
-    for (int32_t k = a; k < b;) {
-      int32_t e = k;
-      while (e < b && e - k < kPieceRows && ptr[(size_t)e + 1] - ptr[(size_t)k] <= kPieceEntries) ++e;
-      pieces.push_back(e);  // the end of this piece, the start of the next
-      k = e;
-    }
+    for (int32_t k = a; k < b;) pieces.push_back(k = piece_end(k, b));  // an end, the start of the next
     t.runs.back().last = (int32_t)pieces.size() - 1;
   }
   t.rows.upload(rows.data(), n, c->stream);

@@ -9,8 +9,10 @@
   piece (512 rows) linked 15, 16 and 17 levels back;
 * rows with more neighbours than are read together (4, 8, 16), and random patterns whose
   levels are narrow at the ends and wide in the middle (runs between launches);
-* levels of 255 .. 2049 rows around the piece size (512 rows) and the widest level of a
-  one-block run (2048).
+* levels of 255 .. 2049 rows around the piece size (512 rows) and the widths from which
+  levels are launched one by one;
+* levels that are launched between runs for their length or for a row too long for a
+  piece (2048 entries).
 """
 import numpy as np
 import pytest
@@ -66,6 +68,18 @@ def cases():
     for width in (255, 256, 257, 512, 513, 1024, 1025, 2048, 2049):
         yield f"layers_{width}", layered(width, 12, 3, width, far=40)
     rng = np.random.default_rng(9)
+    # narrow levels of short rows, then wide levels of long ones, twice over
+    S, base = [], 0
+    for width, layers, links in ((40, 30, 2), (1500, 6, 12), (40, 30, 2), (1500, 6, 12), (40, 5, 2)):
+        for l in range(layers):
+            i = np.arange(base, base + width)
+            if base:
+                S += [np.stack([i, rng.integers(max(0, base - 40), base, width)], 1) for _ in range(links)]
+            base += width
+    yield "mixed_levels", system(base, np.concatenate(S), 8)
+    n = 6000  # one row coupled to 3,000 before it
+    long_row = [(i, i - 1) for i in range(1, n)] + [(5000, i) for i in range(0, 4999, 1) if i % 5 < 3]
+    yield "row_over_a_piece", system(n, long_row, 10)
     i = rng.integers(1, 60000, 200000)
     yield "random", system(60000, np.stack([i, (i * rng.random(len(i))).astype(np.int64)], 1), 5)
 
