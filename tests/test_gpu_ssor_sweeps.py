@@ -7,6 +7,7 @@
 * chains with links far behind (neighbours older than the 8192-position window, read
   from memory) and to the first rows, links at the window's edge, and levels of one full
   piece (512 rows) linked 15, 16 and 17 levels back;
+* few and many levels that are all launched;
 * rows with more neighbours than are read together (4, 8, 16), and random patterns whose
   levels are narrow at the ends and wide in the middle (runs between launches);
 * levels of 255 .. 2049 rows around the piece size (512 rows) and the widths from which
@@ -67,6 +68,8 @@ def cases():
     yield "long_rows", layered(100, 30, 13, 4)
     for width in (255, 256, 257, 512, 513, 1024, 1025, 2048, 2049):
         yield f"layers_{width}", layered(width, 12, 3, width, far=40)
+    for levels in (2, 3, 8, 9):
+        yield f"wide_levels_{levels}", layered(6000, levels, 4, levels, far=100)
     rng = np.random.default_rng(9)
     # narrow levels of short rows, then wide levels of long ones, twice over
     S, base = [], 0
