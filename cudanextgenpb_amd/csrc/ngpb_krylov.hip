@@ -114,6 +114,10 @@ constexpr int kDiags = 14;
 // launches per iteration, 822 in one block; 512 rows 863 and 239; 8,000 rows 1,774 and
 // 1,708 (8 rows per thread, which spill), so the line lies at 4 rows per thread.
 constexpr int kBlockRows = 4096;
+// and most diagonals over all its slices (nine each at 4,096 rows): an iteration takes 2 us
+// and 1/60 us for each of varying values (448: 9.2 us, 520: 10.7, 611: 12.8, 832: 15.9)
+// against 11 to 14 us, by the host's pace, of three launches.
+constexpr int kBlockDiags = 576;
 struct SliceRec {
   int32_t count;  // diagonals, -1: more than kDiags
   uint32_t vary;  // bit k: diagonal k's values differ
@@ -135,7 +139,11 @@ bool use_records(int64_t n, int64_t staged) {
   return 3 * lo * staged <= 2 * slices * std::clamp<int64_t>(n - lo, 0, lo);
 }
 
-// one wave per slice; flags[1] counts the slices with more than kDiags diagonals
+// whether a system's CG runs in one block
+bool use_block(int64_t n, int staged, int diags) { return n <= kBlockRows && !staged && diags <= kBlockDiags; }
+
+// one wave per slice; flags[1] counts the slices with more than kDiags diagonals, flags[2]
+// the diagonals of the others (at up to kBlockRows rows)
 __global__ void __launch_bounds__(kBS) k_slice_rec(int64_t n, const int32_t* __restrict__ rowptr,
                                                    const int32_t* __restrict__ col, const double* __restrict__ val,
                                                    SliceRec* __restrict__ recs, int* __restrict__ flags) {
@@ -177,6 +185,7 @@ __global__ void __launch_bounds__(kBS) k_slice_rec(int64_t n, const int32_t* __r
   if (lane == 0 && s * 64 < n) {
     R.count = k;
     R.vary = vary;
+    if (n <= kBlockRows && k > 0) atomicAdd(flags + 2, k);
   }
   const int staged = __syncthreads_count(lane == 0 && k < 0);
   if (staged && threadIdx.x == 0) atomicAdd(flags + 1, staged);
@@ -750,13 +759,13 @@ void ensure_reduce(ngpb_ctx* c, int64_t blocks) {
 }
 
 namespace {
-// 1 / diagonal, its checks and, if asked for, the slice records; returns how many slices
-// have none
-int check_operator_records(ngpb_ctx* c, bool records) {
+// 1 / diagonal, its checks and, if asked for, the slice records with the counts of slices
+// without one and of diagonals
+void check_operator_records(ngpb_ctx* c, bool records, int* staged = nullptr, int* diags = nullptr) {
   c->dinv.resize((size_t)c->n);
   DBuf<int> bad;
-  bad.resize(2);
-  NGPB_HIP(hipMemsetAsync(bad.p, 0, 2 * sizeof(int), c->stream));
+  bad.resize(3);
+  NGPB_HIP(hipMemsetAsync(bad.p, 0, 3 * sizeof(int), c->stream));
   hipLaunchKernelGGL(k_diag_inv, dim3(blocks_for(c->n, 256)), dim3(256), 0, c->stream, c->n, c->rowptr.p, c->col.p,
                      c->val.p, c->dinv.p, bad.p);
   if (records) {
@@ -766,12 +775,13 @@ int check_operator_records(ngpb_ctx* c, bool records) {
                        c->col.p, c->val.p, reinterpret_cast<SliceRec*>(c->slice_rec.p), bad.p);
   }
   NGPB_HIP(hipGetLastError());
-  int hb[2] = {0, 0};
+  int hb[3] = {0, 0, 0};
   NGPB_HIP(hipMemcpyAsync(hb, bad.p, sizeof(hb), hipMemcpyDeviceToHost, c->stream));
   NGPB_HIP(hipStreamSynchronize(c->stream));
   NGPB_REQUIRE(!(hb[0] & 2), NGPB_E_NUMERIC, "operator holds NaN or Inf entries");
   NGPB_REQUIRE(!(hb[0] & 1), NGPB_E_NUMERIC, "operator has a zero or negative diagonal entry");
-  return hb[1];
+  if (staged) *staged = hb[1];
+  if (diags) *diags = hb[2];
 }
 }  // namespace
 
@@ -816,11 +826,12 @@ double time_spmv_fp64(ngpb_ctx* c, int reps) {
   return (double)ms / std::max(reps, 1);
 }
 
-void check_operator(ngpb_ctx* c) { (void)check_operator_records(c, false); }
+void check_operator(ngpb_ctx* c) { check_operator_records(c, false); }
 
 const void* slice_records(ngpb_ctx* c, bool* block) {
-  const int staged = check_operator_records(c, true);
-  if (block) *block = c->n <= kBlockRows && !staged;
+  int staged = 0, diags = 0;
+  check_operator_records(c, true, &staged, &diags);
+  if (block) *block = use_block(c->n, staged, diags);
   return use_records(c->n, staged) ? c->slice_rec.p : nullptr;
 }
 
@@ -979,12 +990,12 @@ void solve_csr_noalloc(int device, hipStream_t s, int64_t n, int64_t nnz, const 
   KrylovScalars* ks = reinterpret_cast<KrylovScalars*>(part + kNoAllocPartials);
   int* bad = reinterpret_cast<int*>(ks + 1);
   SliceRec* recs = reinterpret_cast<SliceRec*>(part + kNoAllocPartials + 64);
-  static_assert(sizeof(KrylovScalars) + 2 * sizeof(int) <= 64 * sizeof(double), "scalar area too small");
+  static_assert(sizeof(KrylovScalars) + 3 * sizeof(int) <= 64 * sizeof(double), "scalar area too small");
   const auto t0 = std::chrono::steady_clock::now();
-  hipLaunchKernelGGL(k_clear_flags, dim3(1), dim3(2), 0, s, bad);
+  hipLaunchKernelGGL(k_clear_flags, dim3(1), dim3(3), 0, s, bad);
   hipLaunchKernelGGL(k_csr_check, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, nnz, rowptr, col, bad);
   NGPB_HIP(hipGetLastError());
-  int hb[2] = {0, 0};
+  int hb[3] = {0, 0, 0};
   NGPB_HIP(hipMemcpyAsync(hb, bad, sizeof(hb), hipMemcpyDeviceToHost, s));
   NGPB_HIP(hipStreamSynchronize(s));
   NGPB_REQUIRE(!(hb[0] & 4), NGPB_E_ARG, "row pointers must run from 0 to nnz without decreasing, columns in [0, n)");
@@ -1003,7 +1014,7 @@ void solve_csr_noalloc(int device, hipStream_t s, int64_t n, int64_t nnz, const 
     NGPB_HIP(hipStreamSynchronize(s));
     return h.done != 0;
   };
-  if (n <= kBlockRows && !hb[1]) {
+  if (use_block(n, hb[1], hb[2])) {
     run_pcg_block(s, n, rowptr, val, recs, dinv, b, x, r, p, ks, tol, maxiter, poll);
   } else {
     // the launch shapes of ngpb_solve under SpMV schedule 0

@@ -5,8 +5,8 @@ relative residual of 1e-13 by ngpb_solve_csr_noalloc: the relative error is then
 3e-13 plus rounding. Sizes lie around the slice (64) and block (256) edges; the entries
 lie on few diagonals with one value each, on few diagonals with varying values, on
 exactly as many diagonals as a record holds and one more, or anywhere. Up to 4,096 rows, on
-at most 14 diagonals, one block runs the whole CG with 1, 2 or 4 rows per thread, 1,024
-iterations per launch. Systems with slices that have no record are multiplied from the
+at most 14 diagonals (nine a slice on average at 4,096 rows), one block runs the whole CG
+with 1, 2 or 4 rows per thread, 1,024 iterations per launch. Systems with slices that have no record are multiplied from the
 CSR up to 2^18 rows and where most slices are such; the largest sizes here have a third
 of them, around the rows from which records are used, and several staged pieces per slice.
 """
