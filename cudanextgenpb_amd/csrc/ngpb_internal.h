@@ -188,12 +188,12 @@ struct KrylovScalars {
   double rho2[2];   // (r, z) entering the iteration of parity par
   double alpha2[2]; // alpha of the iteration of parity par
   int iter2[2];     // iterations completed before the iteration of parity par
-  int halt2[2];     // FP64 CG: 1 = stopped before the direction kernel of parity par
   int stop_par;     // parity of the iteration that raised the stop flag
   int iter;         // iterations done in this solve
   int done;         // 1 = stop flag raised
   int maxiter;      // iteration limit for the current cycle
   int status;       // 0 converged, 4 maxiter
+  int halt2[2];     // FP64 CG: 1 = stopped before the direction kernel of parity par
 };
 
 // Grow-only device scratch slots held by the context and reused across calls, so that

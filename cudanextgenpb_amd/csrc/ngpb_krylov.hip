@@ -185,10 +185,18 @@ __global__ void __launch_bounds__(kBS) k_slice_rec(int64_t n, const int32_t* __r
   if (lane == 0 && s * 64 < n) {
     R.count = k;
     R.vary = vary;
-    if (n <= kBlockRows && k > 0) atomicAdd(flags + 2, k);
   }
-  const int staged = __syncthreads_count(lane == 0 && k < 0);
-  if (staged && threadIdx.x == 0) atomicAdd(flags + 1, staged);
+  __shared__ int s_k[kBS / 64];
+  if (lane == 0) s_k[threadIdx.x >> 6] = k;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  int staged = 0, diags = 0;
+  for (int q = 0; q < kBS / 64; ++q) {
+    staged += s_k[q] < 0 ? 1 : 0;
+    diags += max(s_k[q], 0);
+  }
+  if (staged) atomicAdd(flags + 1, staged);
+  if (n <= kBlockRows) atomicAdd(flags + 2, diags);
 }
 
 // k_spmv64 from slice records: the same rows per thread and the same partial sums. A
@@ -335,8 +343,10 @@ __device__ __forceinline__ double2 blk_sum2(double a, double b, double2* slot) {
   return t;
 }
 
+// Aligned: the loop is fetched over and over by one CU, and where its code falls moved an
+// iteration at 4,096 rows between 8.3 and 8.5 us.
 template <int R>
-__global__ void __launch_bounds__(kBlk) k_pcg_block(int n, const int32_t* __restrict__ rowptr, const double* __restrict__ val,
+__global__ void __launch_bounds__(kBlk) __attribute__((aligned(4096))) k_pcg_block(int n, const int32_t* __restrict__ rowptr, const double* __restrict__ val,
                                                      const SliceRec* __restrict__ recs, const double* __restrict__ dinv,
                                                      const double* __restrict__ b, double* __restrict__ x,
                                                      double* __restrict__ r, double* __restrict__ p, KrylovScalars* ks,
