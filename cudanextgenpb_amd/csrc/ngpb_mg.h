@@ -10,8 +10,9 @@ constexpr int kMgLevels = 10;  // 1022 cells an axis halve nine times
 // Finest-lattice vertices per unknown up to which the dense transfer array is used. An
 // iteration then moves some 4 x 32 bytes for it and 2 x 32 for the uniform levels per
 // unknown, ~450 with the three SpMVs, against ~60 for a Jacobi-scaled one of which there
-// are ten or more times as many: at 18 per unknown (the 47,302-unknown mesh above) the
-// solve is still 1.5x faster, at twice that the two meet.
+// are ten or more times as many: at 18 per unknown (a 47,302-unknown mesh) the solve is
+// still 1.5x faster, at 24 (706,224 unknowns) 5.9 ms for 12.5. The bound is on memory: at 32
+// the hierarchy takes some 290 bytes per unknown.
 constexpr int64_t kMgDenseRatio = 32;
 // the finest lattice of the mesh's box
 struct MgBox {

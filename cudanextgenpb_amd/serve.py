@@ -62,7 +62,8 @@ def predict_bytes(problem: W.Problem) -> int:
     sorting; per hanging node 64; per border leaf (fractions, normals and the energy's
     sources and accumulators) 3.6 KB, with the border leaves bounded by the atoms'
     summed sphere areas over the finest leaf face (the surface of their union is
-    smaller)."""
+    smaller). The mixed solve's multigrid hierarchy, at most 290 per node, is built after
+    the symbolic temporaries (498 per node) are gone, and is covered by them."""
     mesh = problem.mesh
     N, L, H = mesh.n_nodes, mesh.n_leaves, mesh.n_hang
     per_node = 24 + 16 + 9 + 12 + 24 + 8 + 64 + 10 + 210 + 12 * (12 + 4 + 6 + 24)
